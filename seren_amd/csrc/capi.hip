@@ -244,6 +244,8 @@ int ensure_capacity(Ctx &c, int n) {
     SX_TRY(dalloc(&c.ovf_idx, nn));
     SX_TRY(dalloc(&c.nbl, particle_waves(n) * NB_CAP));
     SX_TRY(dalloc(&c.nbl_len, particle_waves(n)));
+    SX_TRY(dalloc(&c.hq, nn));
+    SX_TRY(dalloc(&c.hq_len, 1));
     SX_TRY(dalloc(&c.hrec, nn * 16));
     SX_TRY(dalloc(&c.grec, nn * 8));
     SX_TRY(dalloc(&c.gax, nn));
@@ -287,7 +289,7 @@ void free_all(Ctx &c) {
                     c.press, c.sound, c.divv, c.drhodt, c.ax, c.ay, c.az, c.gpot, c.agm,
                     c.u, c.dudt,
                     c.tmpd, c.hrec, c.hlist, c.porig, c.tmpi, c.active, c.pptot, c.pplist, c.ovf_off,
-                    c.ovf_idx, c.nbl, c.nbl_len,
+                    c.ovf_idx, c.nbl, c.nbl_len, c.hq, c.hq_len, c.bn, c.c_first, c.c_last,
                     c.ovf_list, c.ovf_count, c.khi, c.klo, c.khi2, c.klo2, c.idx, c.idx2,
                     c.cpl, c.pact, c.flag, c.incl, c.cellof, c.ncs, c.off, c.firstlev,
                     c.root, c.bbpart, c.cloud_off, c.cid, c.chunks, c.chunk_first,
@@ -356,10 +358,12 @@ size_t ctx_device_bytes(const Ctx &c) {
     b += walk_max_groups(c.cap, c.pp_gather) * (size_t)(4 + 8 + 6 * 8);  // walk groups
     b += near_list_entries(c.cap) * 12;                              // near-field lists
     b += particle_waves(c.cap) * (NB_CAP + 1) * 4;                   // neighbour-walk leaves
+    b += nn * 4;                                                     // wave h-solve queue
     b += nn * (5 * 4 + 1) + nn * (size_t)c.pp_limit * 4;    // ints, active, neighbour rows
     b += (((size_t)c.cap + 255) / 256) * 4 * HL_SLOTS * WAVE * 4;   // h-solve lists
     b += nn * (4 * 8 + 2 * 4 + 2 + 5 * 4 + 1);              // tree build scratch
-    b += cc * (sizeof(GNode) + 10 * 8 + sizeof(GNodeF) + sizeof(HNode) + 8 * 4 + 7 * 8);
+    b += cc * (sizeof(GNode) + 10 * 8 + sizeof(GNodeF) + sizeof(HNode) + sizeof(BNode) +
+               10 * 4 + 7 * 8);
     b += c.sorttmp_bytes + c.ovf_cap * 4 + sizeof(double) * KT_TOTAL;
     if (c.st.on) b += nn * (11 * 8 + 8 + 4);                 // step state
     if (c.sv.on) b += nn * 3 * 8 + (size_t)c.ncloud * 25;    // serving state

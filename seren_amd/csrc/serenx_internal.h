@@ -144,6 +144,20 @@ struct __attribute__((aligned(64))) HNode {
                       // particle of the subtree lies within r +- half
 };
 
+// Hydro node in BFS order, where a branch's children are consecutive: the
+// searches of one particle by a whole wave test 64 nodes at once and put a
+// branch's children in its place, which keeps a list of nodes in DFS order
+// without following a chain of next links.  Same box data as HNode.
+struct __attribute__((aligned(64))) BNode {
+    double r[3];
+    double rmax;
+    double hrangemax; // KERNRANGE max(h) over the subtree (k_hmax_bfs)
+    float half[3];
+    int fc;           // branch: first child (BFS id); leaf: first particle
+    int k;            // > 0: particles of a leaf; < 0: minus the children of a branch
+    int parent;       // BFS id of the parent (roots: -1)
+};
+
 // Mixed-precision gravity node: FP64 COM (the cell offset is subtracted in
 // FP64) and MAC data, FP32 moments; walk data in the first 64 bytes.
 struct __attribute__((aligned(64))) GNodeF {
@@ -162,6 +176,7 @@ struct __attribute__((aligned(64))) GNodeF {
 static_assert(offsetof(GNode, q) == 64 && sizeof(GNode) == 256, "GNode layout");
 static_assert(offsetof(GNodeF, q) <= 64 && sizeof(GNodeF) == 128, "GNodeF layout");
 static_assert(sizeof(HNode) == 64, "HNode layout");
+static_assert(sizeof(BNode) == 64, "BNode layout");
 
 struct DevBuf {
     void *p = nullptr;
@@ -274,6 +289,8 @@ struct Ctx {
     double *gs = nullptr;        // octupole moments s[10] per node (stock, export)
     GNodeF *gnf = nullptr;
     HNode *hn = nullptr;
+    BNode *bn = nullptr;         // hydro nodes by BFS id (h solve and lists by waves)
+    int *c_first = nullptr, *c_last = nullptr;   // children of a branch: [first, last) BFS ids
     int nc = 0, ltot = 0;
     int level_off[LMAX + 2] = {0};
     int level_cnt[LMAX + 2] = {0};
@@ -289,6 +306,8 @@ struct Ctx {
     // leaves each wave of the neighbour walk opened (NB_CAP per wave of 64
     // particles, in DFS order) and their number, for the overflow rows
     int *nbl = nullptr, *nbl_len = nullptr;
+    // particles the lane h solve leaves to the wave solve, and their number
+    int *hq = nullptr, *hq_len = nullptr;
 
     // kernel tables [NTAB][KT] (kernel.F90)
     double *ktab = nullptr;

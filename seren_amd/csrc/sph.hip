@@ -8,6 +8,7 @@
 // reference's potential-neighbour list, and use the reference's operation
 // order (built without FMA contraction), so h, rho, Omega, zeta and the
 // neighbour lists come out identical to the reference.
+#include <algorithm>
 #include <cstring>
 #include <rocprim/rocprim.hpp>
 
@@ -19,9 +20,6 @@ namespace {
 
 constexpr int TB = 256;
 inline int nblk(long n, int tb = TB) { return (int)((n + tb - 1) / tb); }
-
-// lane modes of the h solve
-enum { M_DONE = 0, M_ITER = 1, M_FINAL = 2 };
 
 // Compact 32-byte records for the per-lane candidate loops of the h solve,
 // in the record buffer (which the hydro pass later rewrites): rec[i] =
@@ -114,6 +112,19 @@ __device__ __forceinline__ void list_loop(const int *__restrict__ wl, int nslot,
     }
 }
 
+// appends the particles of the lanes with pred set to the queue, one atomic
+// per wave
+__device__ __forceinline__ void queue_lanes(bool pred, int p, int *__restrict__ q,
+                                            int *__restrict__ len) {
+    const unsigned long long m = ballot(pred);
+    if (m == 0) return;
+    const int lane = (int)(threadIdx.x & (WAVE - 1));
+    int at = 0;
+    if (lane == 0) at = atomicAdd(len, __popcll(m));
+    at = __shfl(at, 0, WAVE);
+    if (pred) q[at + __popcll(m & ((1ull << lane) - 1ull))] = p;
+}
+
 // all_sph_gradh.F90:103-309, the h iteration, for every active particle.
 //
 // Potential-neighbour lists (BHhydrowalk_hgather) are recorded once per
@@ -122,10 +133,12 @@ __device__ __forceinline__ void list_loop(const int *__restrict__ wl, int nslot,
 // slots per lane (slot-major, so the lanes of a wave read one contiguous row
 // per step).  The iterations loop over each lane's own list, which is the
 // reference's pp_potlist in the reference's order, so every sum is formed
-// exactly as the reference forms it.  A wave with a lane whose list does not
-// fit sums over the tree walk itself for that radius (same leaves, same
-// order).  On exit every lane leaves rhotemp in rho, h_high in hhigh and its
-// list length in nlist (-1: list incomplete) for k_hsolve_final; its list
+// exactly as the reference forms it.  A lane whose list does not fit leaves
+// its particle to k_hsolve_wave (hq) and stops: summed here over the tree
+// walk, it held its wave in walks of the whole cloud (one particle on its
+// way through the bisection took 1 s of a 131k-particle step).  On exit
+// every other lane leaves rhotemp in rho, h_high in hhigh and its list
+// length in nlist (-1: left to k_hsolve_wave) for k_hsolve_final; its list
 // stays in hlist (a lane joins no walk after it has converged).
 //
 // WAVES > 0 holds the kernel to WAVES waves per SIMD (64 VGPRs at 8, with a
@@ -142,7 +155,7 @@ __attribute__((amdgpu_waves_per_eu(WAVES > 0 ? WAVES : 1, WAVES > 0 ? WAVES : 8)
     const uint8_t *__restrict__ active, const double *__restrict__ ktab,
     double h_fac, int pp_gather, double *__restrict__ h,
     double *__restrict__ rho, double *__restrict__ hhigh, int *__restrict__ nlist,
-    unsigned long long *__restrict__ wstat) {
+    int *__restrict__ hq, int *__restrict__ hq_len, unsigned long long *__restrict__ wstat) {
     const int p = xcd_block() * blockDim.x + threadIdx.x;
     const bool valid = p < n && active[p];
     int *wl = hlist + (size_t)(p / WAVE) * (HL_SLOTS * WAVE) + (threadIdx.x & (WAVE - 1));
@@ -163,9 +176,9 @@ __attribute__((amdgpu_waves_per_eu(WAVES > 0 ? WAVES : 1, WAVES > 0 ? WAVES : 8)
     double rhotemp = 0.0;
     int iteration = 0;
     bool iterating = valid;
-    unsigned passes = 0, vis = 0, lvis = 0, walks = 0, fallback = 0;
+    unsigned passes = 0, vis = 0, lvis = 0, walks = 0;
     int nslot = 0, cnt = 0, slot_max = 0;
-    bool have_list = false, wave_ovf = false, my_ovf = false;
+    bool have_list = false, my_ovf = false;
 
     while (any_lane(iterating)) {
         passes++;
@@ -180,7 +193,6 @@ __attribute__((amdgpu_waves_per_eu(WAVES > 0 ? WAVES : 1, WAVES > 0 ? WAVES : 8)
         const double hrangesqd = kg.rangesqd * hp * hp;
         double srho = mp * w0[0] * hfactor_p;                  // :209-210
         double som = mp * hfactor_p * invhp * wh[0];
-        auto visit = [&](const HNode &nd, bool) { return hgather_visit(nd, rpx, rpy, rpz, R); };
         // :214-231 for one potential neighbour
         auto pair = [&](double xj, double yj, double zj, double mj) {
             const double ex = xj - rpx, ey = yj - rpy, ez = zj - rpz;
@@ -201,8 +213,11 @@ __attribute__((amdgpu_waves_per_eu(WAVES > 0 ? WAVES : 1, WAVES > 0 ? WAVES : 8)
                 nslot = 0;
                 cnt = 0;
             }
-            bool lovf = false;
-            vis += group_walk(hn, nc, iterating, rr.x, rr.y, lvis, visit,
+            bool lovf = false;   // the list is full: the lane passes over the rest
+            vis += group_walk(hn, nc, iterating, rr.x, rr.y, lvis,
+                              [&](const HNode &nd, bool) {
+                                  return lovf ? WALK_SKIP : hgather_visit(nd, rpx, rpy, rpz, R);
+                              },
                               [&](const HNode &nd, bool mine) {
                 if (mine) {
                     cnt += nd.leaf;                       // the reference's pp_pot
@@ -218,29 +233,16 @@ __attribute__((amdgpu_waves_per_eu(WAVES > 0 ? WAVES : 1, WAVES > 0 ? WAVES : 8)
             if (iterating) {
                 slot_max = max(slot_max, nslot);
                 my_ovf = lovf;
+                if (lovf) iterating = false;
             }
             have_list = true;
-            wave_ovf = any_lane(lovf);
             walks++;
         }
         // too few potential neighbours: grow h and gather again (:185-189)
         const bool grow = iterating && newlist && cnt < pp_gather;
         const bool sum = iterating && !grow;
-        if (!wave_ovf) {
-            list_loop(wl, nslot, sum, p, [&](int j) { return rec[j]; },
-                      [&](int, const double4 &a) { pair(a.x, a.y, a.z, a.w); });
-        } else {
-            vis += group_walk(hn, nc, sum, rr.x, rr.y, lvis, visit,
-                              [&](const HNode &nd, bool mine) {
-                const bool use = mine && leaf_near(nd, rpx, rpy, rpz, R, box);
-                for (int i = 0; i < nd.leaf; i++) {
-                    const int j = nd.first + i;
-                    const double4 a = rec[j];
-                    if (use && j != p) pair(a.x, a.y, a.z, a.w);
-                }
-            });
-            fallback++;
-        }
+        list_loop(wl, nslot, sum, p, [&](int j) { return rec[j]; },
+                  [&](int, const double4 &a) { pair(a.x, a.y, a.z, a.w); });
 
         if (grow) {
             h_high = 0.0;
@@ -281,8 +283,9 @@ __attribute__((amdgpu_waves_per_eu(WAVES > 0 ? WAVES : 1, WAVES > 0 ? WAVES : 8)
         hhigh[p] = h_high;
         nlist[p] = my_ovf ? -1 : nslot;
     }
+    queue_lanes(my_ovf, p, hq, hq_len);
     // walk statistics: cells visited / lane visits, passes, lane iterations,
-    // list walks, fallback passes, longest list
+    // list walks, longest list
     wave_stats(wstat, 2, vis, lvis);
     unsigned long long it = valid ? (unsigned long long)iteration : 0ull;
 #pragma unroll
@@ -295,42 +298,44 @@ __attribute__((amdgpu_waves_per_eu(WAVES > 0 ? WAVES : 1, WAVES > 0 ? WAVES : 8)
         atomicAdd(ws + 6, it);
         atomicAdd(ws + 7, 1ull);
         atomicAdd(ws + 10, (unsigned long long)walks);
-        atomicAdd(ws + 11, (unsigned long long)fallback);
         atomicMax(ws + 12, (unsigned long long)smx);
     }
 }
 
 // all_sph_gradh.F90:310-489: with h from the converged density, the gather
-// sums rho, Omega, div v and zeta over the last potential-neighbour list.
+// sums rho, Omega, div v and zeta over the last potential-neighbour list, for
+// the particles whose list k_hsolve_iter holds; k_hsolve_wave does the others.
 __global__ void __launch_bounds__(256) k_hsolve_final(
-    KGeom kg, bool box, int n, int nc, const HNode *__restrict__ hn, const double4 *__restrict__ rec,
-    const int *__restrict__ cid, const int2 *__restrict__ root_range,
-    const int *__restrict__ hlist, const uint8_t *__restrict__ active,
+    KGeom kg, bool box, int n, const double4 *__restrict__ rec, const int *__restrict__ hlist, const uint8_t *__restrict__ active,
     const double *__restrict__ ktab, double h_fac, const double *__restrict__ hhigh,
     const int *__restrict__ nlist, double *__restrict__ h, double *__restrict__ zeta,
     double *__restrict__ rho, double *__restrict__ omega, double *__restrict__ divv,
-    double *__restrict__ drhodt, int *__restrict__ err, unsigned long long *__restrict__ wstat) {
+    double *__restrict__ drhodt, int *__restrict__ hq, int *__restrict__ hq_len,
+    int *__restrict__ err) {
     const int p = xcd_block() * blockDim.x + threadIdx.x;
-    const bool valid = p < n && active[p];
+    bool valid = p < n && active[p];
     const int *wl = hlist + (size_t)(p / WAVE) * (HL_SLOTS * WAVE) + (threadIdx.x & (WAVE - 1));
     const double *w0 = ktab + T_W0 * KT;
     const double *wh = ktab + T_WH * KT;
     const double *wg = ktab + T_WG * KT;
     const double *h4 = ktab + KT_H4_OFF;   // (w0, wh, w4, wg) per index
     const double4 *vrec = rec + n;
-    double rpx = 0, rpy = 0, rpz = 0, mp = 0, vpx = 0, vpy = 0, vpz = 0, R = 0, hp = 1;
+    double rpx = 0, rpy = 0, rpz = 0, mp = 0, vpx = 0, vpy = 0, vpz = 0, hp = 1;
     int nslot = 0;
+    bool beyond = false;
+    if (valid) nslot = nlist[p];
+    valid = valid && nslot >= 0;
     if (valid) {
         const double4 a = rec[p], b = vrec[p];
         rpx = a.x; rpy = a.y; rpz = a.z; mp = a.w;
         vpx = b.x; vpy = b.y; vpz = b.z;
         hp = h_fac * ref_pow_third(mp / rho[p]);                 // :317
-        R = kg.range * hhigh[p];
-        nslot = nlist[p];
-        // a final h beyond the list's radius can reach particles past R in
-        // leaves the box test left out: gather over the walk instead
-        if (box && kg.range * hp > R) nslot = -1;
+        // a final h beyond the list's radius can reach particles past it in
+        // leaves the box test left out: left to k_hsolve_wave as well
+        beyond = box && kg.range * hp > kg.range * hhigh[p];
+        valid = !beyond;
     }
+    queue_lanes(beyond, p, hq, hq_len);
     const double invhp = 1.0 / hp;
     const double hfactor_p = cr_pow3(invhp);
     const double hrangesqd = kg.rangesqd * hp * hp;
@@ -356,27 +361,8 @@ __global__ void __launch_bounds__(256) k_hsolve_final(
         sdiv = sdiv - mj * dvdr * w.z * hfactor_p * invhp / drmag;
         szeta = szeta + mj * invhp * invhp * w.w;
     };
-    list_loop(wl, nslot, valid && nslot >= 0, p, [&](int j) { return rec[j]; },
+    list_loop(wl, nslot, valid, p, [&](int j) { return rec[j]; },
               [&](int j, const double4 &a) { pair(a.x, a.y, a.z, a.w, j); });
-    unsigned vis = 0, lvis = 0;
-    const bool walk = valid && nslot < 0;
-    if (any_lane(walk)) {
-        // lists that did not fit: gather over the tree walk at the same radius
-        const int2 rr = valid ? root_range[cid[p]] : make_int2(nc, nc);
-        vis = group_walk(
-            hn, nc, walk, rr.x, rr.y, lvis,
-            [&](const HNode &nd, bool) { return hgather_visit(nd, rpx, rpy, rpz, R); },
-            [&](const HNode &nd, bool mine) {
-                const bool use = mine && leaf_near(nd, rpx, rpy, rpz, fmax(R, kg.range * hp), box);
-                for (int i = 0; i < nd.leaf; i++) {
-                    const int j = nd.first + i;
-                    const double4 a = rec[j];
-                    if (use && j != p) pair(a.x, a.y, a.z, a.w, j);
-                }
-            });
-        wave_stats(wstat, 2, vis, lvis);
-        if ((threadIdx.x & 63) == 0) atomicAdd(ctr_row(wstat) + 11, 1ull);
-    }
     if (valid) {
         const double om = 1.0 + ((hp * som) / (3.0 * srho));
         const double dv = sdiv / srho;
@@ -387,6 +373,431 @@ __global__ void __launch_bounds__(256) k_hsolve_final(
         h[p] = hp;
         zeta[p] = -(hp * szeta) / (3.0 * srho * om);
         if (hp < 0.0) atomicOr(err, 1);
+    }
+}
+
+// ---- searches of one particle by a whole wave ------------------------------
+//
+// The lane kernels give a particle to a lane, and a wave's time is its
+// slowest lane's; with few waves in the launch (small clouds) or one particle
+// with a long search (far outskirts, the bisection of the h solve) the
+// serial chain of one lane's loads is what the launch takes.  Here a wave
+// serves one particle: 64 nodes are tested at once, the candidates are
+// evaluated 64 at once, and only the additions of the terms inside the
+// kernel range are serial, because the sums keep the order of the
+// reference's list (DFS order) and with it its rounding.
+
+// nodes of a search front, and leaves of a list, held in LDS.  512 entries
+// hold a front of the largest chain of a resumed search (7 siblings on each
+// of LMAX levels) and the lists of all but a few particles; 8 KB per wave
+// leave 20 waves on a CU.
+constexpr int WS_CAP = 512;
+static_assert(WS_CAP >= 8 * (LMAX + 1), "a resumed search's first front must fit");
+
+struct WaveSearch {
+    int front[2][WS_CAP];
+    int leaf[WS_CAP];      // leaves found: (first particle << 4) | particles
+    double4 term[WAVE];    // terms of one batch of candidates, in list order
+};
+
+// orders the wave's LDS accesses around a point
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// inclusive prefix sum over the lanes of a wave
+__device__ __forceinline__ int wave_prefix(int v, int lane) {
+#pragma unroll
+    for (int d = 1; d < WAVE; d <<= 1) {
+        const int u = __shfl_up(v, d, WAVE);
+        if (lane >= d) v += u;
+    }
+    return v;
+}
+
+// The leaves below root, from the subtree at resume on (DFS order), that
+// test() passes together with all their ancestors at or below the start, in
+// DFS order into L.leaf; returns their number.  The front is expanded level
+// by level, each branch's children in its place.  A front that would pass
+// WS_CAP is cut: resume then names the first node left out (another call
+// continues there), else it is -1.  Every call moves resume on or ends the
+// search: the node it starts at is expanded until it is a leaf or fails.
+template <class Test>
+__device__ __forceinline__ int wave_leaves(WaveSearch &L, const BNode *__restrict__ bn, int root,
+                                           int &resume, unsigned &visits, Test &&test) {
+    const int lane = (int)(threadIdx.x & (WAVE - 1));
+    int len = 0, cur = 0;
+    if (resume == root) {
+        if (lane == 0) L.front[0][0] = root;
+        len = 1;
+    } else {
+        // the rest of the tree in DFS order: resume and its later siblings,
+        // then the later siblings of each ancestor
+        int c = resume, p = bn[c].parent;
+        for (;;) {
+            const int end = bn[p].fc - bn[p].k;
+            if (c + lane < end) L.front[0][len + lane] = c + lane;
+            len += max(end - c, 0);
+            if (p == root) break;
+            c = p + 1;
+            p = bn[p].parent;
+        }
+    }
+    resume = -1;
+    bool branches = true;
+    while (branches) {
+        branches = false;
+        int out = 0;
+        const int *in = L.front[cur];
+        int *dst = L.front[cur ^ 1];
+        wave_lds_fence();
+        for (int base = 0; base < len; base += WAVE) {
+            const int e = base + lane;
+            int v = 0, nout = 0, first = 0;   // a leaf that passed is kept as ~id
+            bool branch = false;
+            if (e < len) {
+                v = in[e];
+                if (v < 0) {
+                    nout = 1;
+                    first = v;
+                } else {
+                    const BNode nd = bn[v];
+                    if (test(nd)) {
+                        branch = nd.k < 0;
+                        nout = branch ? -nd.k : 1;
+                        first = branch ? nd.fc : ~v;
+                    }
+                }
+            }
+            visits += (unsigned)min(WAVE, len - base);
+            const int incl = wave_prefix(nout, lane);
+            const unsigned long long over = ballot(nout > 0 && out + incl > WS_CAP);
+            const int cutlane = over ? __ffsll((long long)over) - 1 : WAVE;
+            if (lane < cutlane) {
+                const int o = out + incl - nout;
+                if (branch)
+                    for (int i = 0; i < nout; i++) dst[o + i] = first + i;
+                else if (nout)
+                    dst[o] = first;
+            }
+            branches = branches || ballot(branch && lane < cutlane) != 0;
+            if (over) {
+                const int r = __shfl(v, cutlane, WAVE);
+                resume = r < 0 ? ~r : r;
+                if (cutlane > 0) out += __shfl(incl, cutlane - 1, WAVE);
+                break;
+            }
+            out += __shfl(incl, WAVE - 1, WAVE);
+        }
+        wave_lds_fence();
+        len = out;
+        cur ^= 1;
+    }
+    // the nodes kept are all leaves now
+    for (int e = lane; e < len; e += WAVE) {
+        const BNode &nd = bn[~L.front[cur][e]];
+        L.leaf[e] = (nd.fc << 4) | nd.k;
+    }
+    wave_lds_fence();
+    return len;
+}
+
+// Calls use(j, record, ok) for the particles of the leaves found, 64 slots
+// at a time in list order: 8 leaves, lane l the particle l & 7 of leaf l >> 3
+// (ok: that particle exists).  The loads of four batches are in flight
+// together.  use returns true to stop.
+template <class Use>
+__device__ __forceinline__ void wave_candidates(const WaveSearch &L, int nleaf,
+                                                const double4 *__restrict__ rec, int p,
+                                                Use &&use) {
+    const int lane = (int)(threadIdx.x & (WAVE - 1)), sub = lane >> 3, k = lane & 7;
+    constexpr int U = 4;
+    for (int e0 = 0; e0 < nleaf; e0 += 8 * U) {
+        double4 a[U];
+        int j[U];
+        bool ok[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int e = e0 + 8 * u + sub;
+            const int d = e < nleaf ? L.leaf[e] : 0;
+            ok[u] = k < (d & 15);
+            j[u] = ok[u] ? (d >> 4) + k : p;
+            a[u] = rec[j[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (e0 + 8 * u < nleaf && use(j[u], a[u], ok[u])) return;
+    }
+}
+
+// all_sph_gradh.F90:103-489 for one particle per wave: the state machine of
+// k_hsolve_iter and the sums of k_hsolve_final, with the same arithmetic in
+// the same order, so both give the same bits.  Runs over the particles
+// hq[0 .. *hq_len) when hq is given, else over all n.
+//
+// While the bisection runs, a pass only decides whether h is too large.  Its
+// density sum grows with every term (masses and kernel are not negative), so
+// the pass ends as soon as the sum shows that h exceeds the h of that density
+// by more than the convergence test's 2 % (2.1 % here, which covers the
+// rounding of the powers): the rest of the sum cannot change the decision.
+// The bisection starts at half the cloud's extent, where the full sum takes
+// in most of the cloud.
+//
+// Bound by the latency of the front's node loads and of the serial sums
+// (about a microsecond each per pass), hidden by the 20 waves on a CU.
+// Measured (steady evaluation, beside the gravity walk): 60 us at 2,048
+// particles, 232 us at 16,384 and 4.4 ms at 131,072, against 680, 980 and
+// 3,560 us of the lane kernels, which keep 64 particles' worth of work per
+// wave: clouds up to HSOLVE_WAVE_MAX particles take this kernel, larger ones
+// the lane kernels (first evaluation of a 2,053-particle Plummer sphere,
+// whose outskirts go through the bisection: 21 -> 3.2 ms).  Held to 4 or 5
+// waves per SIMD instead of the compiler's 153 registers it was slower (242
+// and 289 us at 16,384).
+constexpr int HSOLVE_WAVE_MAX = 1 << 16;
+
+__global__ void __launch_bounds__(256) k_hsolve_wave(
+    KGeom kg, bool box, int n, const BNode *__restrict__ bn, const double4 *__restrict__ rec,
+    const int *__restrict__ cid, const double *__restrict__ roots,
+    const uint8_t *__restrict__ active, const double *__restrict__ ktab, double h_fac,
+    int pp_gather, int list_cap, const int *__restrict__ hq, const int *__restrict__ hq_len,
+    double *__restrict__ h, double *__restrict__ zeta, double *__restrict__ rho,
+    double *__restrict__ omega, double *__restrict__ divv, double *__restrict__ drhodt,
+    int *__restrict__ err, unsigned long long *__restrict__ wstat) {
+    __shared__ WaveSearch lds[256 / WAVE];
+    WaveSearch &L = lds[threadIdx.x / WAVE];
+    const int lane = (int)(threadIdx.x & (WAVE - 1)), wv = (int)(threadIdx.x / WAVE);
+    const double *w0 = ktab + T_W0 * KT;
+    const double *wh = ktab + T_WH * KT;
+    const double *wg = ktab + T_WG * KT;
+    const double *h4 = ktab + KT_H4_OFF;   // (w0, wh, w4, wg) per index
+    const double4 *vrec = rec + n;
+    const int total = hq ? uniform(*hq_len) : n;
+    // each block a contiguous run of the particles, its waves in turn
+    const int nb = (int)gridDim.x, blk = xcd_block();
+    const int lo = (int)((long long)blk * total / nb), hi = (int)((long long)(blk + 1) * total / nb);
+    unsigned passes = 0, passmax = 0, iters = 0, nwave = 0, walks = 0, streamed = 0, longest = 0,
+             vis = 0;
+    for (int t = lo + wv; t < hi; t += 256 / WAVE) {
+        const int p = hq ? uniform(hq[t]) : t;
+        if (!active[p]) continue;
+        const double4 self = rec[p];
+        const double rpx = self.x, rpy = self.y, rpz = self.z, mp = self.w;
+        const int root = uniform(cid[p]);   // a cloud's root has the cloud's BFS id
+        const double rextent = roots[11 * root + 4];
+        double hp = h[p], h_high = 0.0, h_lower = 0.0, h_upper = rextent, rhotemp = 0.0;
+        int iteration = 0, nleaf = 0;
+        unsigned mypasses = 0;
+        bool complete = false;   // L.leaf holds the whole list of radius h_high
+        // BHhydrowalk_hgather.F90:40 at radius R, and with fresh boxes the
+        // nodes that can hold a particle within Rb
+        auto near = [&](const BNode &nd, double R, double Rb) {
+            const double dx = nd.r[0] - rpx, dy = nd.r[1] - rpy, dz = nd.r[2] - rpz;
+            const double drsqd = dx * dx + dy * dy + dz * dz;
+            if (!(drsqd <= (R + nd.rmax) * (R + nd.rmax))) return false;
+            if (!box) return true;
+            const double ex = fmax(fabs(dx) - (double)nd.half[0], 0.0);
+            const double ey = fmax(fabs(dy) - (double)nd.half[1], 0.0);
+            const double ez = fmax(fabs(dz) - (double)nd.half[2], 0.0);
+            return ex * ex + ey * ey + ez * ez <= Rb * Rb * (1.0 + 1.0e-12);
+        };
+        // f(nleaf) over the candidates within Rb (of the list of radius
+        // h_high): from the list when it is complete, else searched anew in
+        // pieces of at most WS_CAP leaves.  f returns true to stop.
+        auto sweep = [&](double Rb, bool from_list, auto &&f) {
+            if (from_list) {
+                f(nleaf);
+                return;
+            }
+            streamed++;
+            complete = false;
+            const double R = kg.range * h_high;
+            int resume = root;
+            do {
+                const int m = wave_leaves(L, bn, root, resume, vis,
+                                          [&](const BNode &nd) { return near(nd, R, Rb); });
+                if (f(m)) break;
+            } while (resume >= 0);
+        };
+        bool iterating = true;
+        while (iterating) {
+            passes++;
+            mypasses++;
+            if (hp > h_high) {
+                h_high = hp * HMULT;
+                const double R = kg.range * h_high;
+                walks++;
+                int resume = root;
+                nleaf = wave_leaves(L, bn, root, resume, vis,
+                                    [&](const BNode &nd) { return near(nd, R, R); });
+                complete = resume < 0 && nleaf <= list_cap;
+                longest = max(longest, (unsigned)nleaf);
+                // the particles of the reference's list (:185-189): those of
+                // the leaves found are a part of it
+                auto count = [&](int m) {
+                    int s = 0;
+                    for (int e = lane; e < m; e += WAVE) s += L.leaf[e] & 15;
+                    return uniform(__shfl(wave_prefix(s, lane), WAVE - 1, WAVE));
+                };
+                int cnt = count(nleaf);
+                if (cnt < pp_gather && (box || resume >= 0)) {
+                    // by the sphere test alone
+                    complete = false;
+                    cnt = 0;
+                    resume = root;
+                    do {
+                        const int m = wave_leaves(L, bn, root, resume, vis, [&](const BNode &nd) {
+                            const double dx = nd.r[0] - rpx, dy = nd.r[1] - rpy,
+                                         dz = nd.r[2] - rpz;
+                            return dx * dx + dy * dy + dz * dz <= (R + nd.rmax) * (R + nd.rmax);
+                        });
+                        cnt += count(m);
+                    } while (resume >= 0 && cnt < pp_gather);
+                }
+                if (cnt < pp_gather) {   // grow h and gather again
+                    h_high = 0.0;
+                    hp = hp * HMULT;
+                    continue;
+                }
+            }
+            const double invhp = 1.0 / hp;
+            const double hfactor_p = cr_pow3(invhp);
+            const double hrangesqd = kg.rangesqd * hp * hp;
+            double srho = mp * w0[0] * hfactor_p;                  // :209-210
+            const bool bisecting = iteration > GRADH_ITERATION_MAX &&
+                                   iteration < 2 * GRADH_ITERATION_MAX;
+            const double hq1 = h_fac / (0.979 * hp);
+            const double enough = mp * hq1 * hq1 * hq1;
+            bool decided = bisecting && srho >= enough;
+            if (!decided) {
+                sweep(kg.range * hp, complete, [&](int m) {
+                    wave_candidates(L, m, rec, p, [&](int j, const double4 &a, bool ok) {
+                        // :214-231
+                        const double ex = a.x - rpx, ey = a.y - rpy, ez = a.z - rpz;
+                        const double dsq = ex * ex + ey * ey + ez * ez;
+                        const double drmag = sqrt(dsq) + SMALL_NUMBER;
+                        const int kern = (int)(kg.half * drmag * invhp);
+                        const bool in = ok && j != p && !(dsq >= hrangesqd) && !(kern >= KERNTOT);
+                        const unsigned long long mask = ballot(in);
+                        if (in)
+                            L.term[__popcll(mask & ((1ull << lane) - 1ull))].x =
+                                a.w * hfactor_p * h4[4 * (size_t)kern];
+                        wave_lds_fence();
+                        const int cnt = __popcll(mask);
+#pragma unroll 8
+                        for (int i = 0; i < cnt; i++) srho = srho + L.term[i].x;
+                        wave_lds_fence();
+                        decided = bisecting && srho >= enough;
+                        return decided;
+                    });
+                    return decided;
+                });
+            }
+            rhotemp = srho;
+            if (decided) {   // fb > 0 (:262) and not converged
+                h_upper = hp;
+                hp = 0.5 * (h_lower + h_upper);
+                iteration++;
+                continue;
+            }
+            const double hnew = h_fac * ref_pow_third(mp / rhotemp);
+            if (fabs(hp - hnew) / hp < H_CON && iteration >= 1) {  // :246
+                iterating = false;
+            } else if (iteration < GRADH_ITERATION_MAX) {           // :252
+                hp = hnew;
+                iteration++;
+            } else if (iteration == GRADH_ITERATION_MAX) {          // :256
+                h_upper = rextent;
+                h_lower = 0.0;
+                hp = 0.5 * (h_lower + h_upper);
+                iteration++;
+            } else if (iteration < 2 * GRADH_ITERATION_MAX) {       // :262
+                double fb;
+                if (rhotemp > SMALL_NUMBER)
+                    fb = cr_pow3(hp) - cr_pow3(h_fac) * mp / rhotemp;
+                else
+                    fb = 1.0;
+                if (fb > 0.0)
+                    h_upper = hp;
+                else
+                    h_lower = hp;
+                hp = 0.5 * (h_lower + h_upper);
+                iteration++;
+            } else {                                                // :276-279
+                iterating = false;
+            }
+        }
+        // :310-489 with h from the converged density
+        hp = h_fac * ref_pow_third(mp / rhotemp);                   // :317
+        const double4 vself = vrec[p];
+        const double invhp = 1.0 / hp;
+        const double hfactor_p = cr_pow3(invhp);
+        const double hrangesqd = kg.rangesqd * hp * hp;
+        double srho = mp * w0[0] * hfactor_p;
+        double som = mp * hfactor_p * invhp * wh[0];
+        double sdiv = 0.0;
+        double szeta = mp * invhp * invhp * wg[0];
+        const bool from_list = complete && !(box && kg.range * hp > kg.range * h_high);
+        sweep(kg.range * hp, from_list, [&](int m) {
+            wave_candidates(L, m, rec, p, [&](int j, const double4 &a, bool ok) {
+                const double ex = a.x - rpx, ey = a.y - rpy, ez = a.z - rpz;
+                const double dsq = ex * ex + ey * ey + ez * ez;
+                const double drmag = sqrt(dsq) + SMALL_NUMBER;
+                const int kern = (int)(kg.half * drmag * invhp);
+                const bool in = ok && j != p && !(dsq > hrangesqd) && !(kern > KERNTOT);
+                const unsigned long long mask = ballot(in);
+                if (in) {
+                    const double4 vj = vrec[j];
+                    const double dvx = vj.x - vself.x, dvy = vj.y - vself.y, dvz = vj.z - vself.z;
+                    const double dvdr = dvx * ex + dvy * ey + dvz * ez;
+                    const double4 w = *reinterpret_cast<const double4 *>(h4 + 4 * (size_t)kern);
+                    L.term[__popcll(mask & ((1ull << lane) - 1ull))] =
+                        make_double4(a.w * hfactor_p * w.x, a.w * hfactor_p * invhp * w.y,
+                                     a.w * dvdr * w.z * hfactor_p * invhp / drmag,
+                                     a.w * invhp * invhp * w.w);
+                }
+                wave_lds_fence();
+                const int cnt = __popcll(mask);
+#pragma unroll 4
+                for (int i = 0; i < cnt; i++) {
+                    const double4 v = L.term[i];
+                    srho = srho + v.x;
+                    som = som + v.y;
+                    sdiv = sdiv - v.z;
+                    szeta = szeta + v.w;
+                }
+                wave_lds_fence();
+                return false;
+            });
+            return false;
+        });
+        if (lane == 0) {
+            const double om = 1.0 + ((hp * som) / (3.0 * srho));
+            const double dv = sdiv / srho;
+            rho[p] = srho;
+            omega[p] = om;
+            divv[p] = dv;
+            drhodt[p] = -srho * dv / om;
+            h[p] = hp;
+            zeta[p] = -(hp * szeta) / (3.0 * srho * om);
+            if (hp < 0.0) atomicOr(err, 1);
+        }
+        iters += (unsigned)iteration;
+        passmax = max(passmax, mypasses);
+        nwave++;
+    }
+    if (nwave > 0 && lane == 0) {
+        unsigned long long *ws = ctr_row(wstat);
+        atomicAdd(ws + 2, (unsigned long long)((vis + WAVE - 1) / WAVE));
+        atomicAdd(ws + 3, (unsigned long long)vis);
+        atomicAdd(ws + 4, (unsigned long long)passes);
+        atomicMax(ws + 5, (unsigned long long)passmax);
+        atomicAdd(ws + 6, (unsigned long long)iters);
+        atomicAdd(ws + 7, (unsigned long long)nwave);
+        atomicAdd(ws + 10, (unsigned long long)walks);
+        atomicAdd(ws + 11, (unsigned long long)streamed);
+        atomicMax(ws + 12, (unsigned long long)longest);
     }
 }
 
@@ -1303,18 +1714,32 @@ int sph_hsolve(Ctx &c) {
     hipLaunchKernelGGL(k_pack_hsolve, dim3(nblk(c.n)), dim3(TB), 0, c.stream, c.n, c.x, c.y, c.z,
                        c.vx, c.vy, c.vz, c.m, rec);
     SX_HIP(hipGetLastError());
-    // h_high per particle in the permutation scratch, list lengths in tmpi
-    // the h solve at 8 waves per SIMD in mixed precision, where it is on the
-    // critical path; beside the FP64 walk (issue-bound) at the compiler's 5
-    const bool w8 = c.hsolve_waves == 8 || (c.hsolve_waves < 0 && c.opt.precision == SERENX_MIXED);
-    hipLaunchKernelGGL(w8 ? k_hsolve_iter<8> : k_hsolve_iter<0>, dim3(nblk(c.n)), dim3(TB), 0, c.stream, c.kg, c.box_ok, c.n, c.nc, c.hn,
-                       rec, c.cid, c.root_range, c.root, c.hlist, c.hl_cap, c.active, c.ktab,
-                       c.opt.h_fac,
-                       c.pp_gather, c.h, c.rho, c.tmpd, c.tmpi, c.wstat);
-    SX_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_hsolve_final, dim3(nblk(c.n)), dim3(TB), 0, c.stream, c.kg, c.box_ok, c.n, c.nc, c.hn,
-                       rec, c.cid, c.root_range, c.hlist, c.active, c.ktab, c.opt.h_fac, c.tmpd, c.tmpi, c.h, c.zeta,
-                       c.rho, c.omega, c.divv, c.drhodt, c.flag, c.wstat);
+    // leaves a particle may list (the tuning knob's slots, when lowered)
+    const int list_cap = c.hl_cap < HL_SLOTS ? c.hl_cap : WS_CAP;
+    const bool by_waves = c.n <= HSOLVE_WAVE_MAX;
+    if (!by_waves) {
+        SX_TRY(zero_words(c.hq_len, 1, c.stream));
+        // h_high per particle in the permutation scratch, list lengths in tmpi
+        // the h solve at 8 waves per SIMD in mixed precision, where it is on the
+        // critical path; beside the FP64 walk (issue-bound) at the compiler's 5
+        const bool w8 =
+            c.hsolve_waves == 8 || (c.hsolve_waves < 0 && c.opt.precision == SERENX_MIXED);
+        hipLaunchKernelGGL(w8 ? k_hsolve_iter<8> : k_hsolve_iter<0>, dim3(nblk(c.n)), dim3(TB), 0,
+                           c.stream, c.kg, c.box_ok, c.n, c.nc, c.hn, rec, c.cid, c.root_range,
+                           c.root, c.hlist, c.hl_cap, c.active, c.ktab, c.opt.h_fac, c.pp_gather,
+                           c.h, c.rho, c.tmpd, c.tmpi, c.hq, c.hq_len, c.wstat);
+        SX_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_hsolve_final, dim3(nblk(c.n)), dim3(TB), 0, c.stream, c.kg, c.box_ok,
+                           c.n, rec, c.hlist, c.active, c.ktab, c.opt.h_fac, c.tmpd, c.tmpi, c.h,
+                           c.zeta, c.rho, c.omega, c.divv, c.drhodt, c.hq, c.hq_len, c.flag);
+        SX_HIP(hipGetLastError());
+    }
+    // all particles of a small cloud, or those the lanes left
+    const int blocks = std::min(nblk(c.n, 256 / WAVE), 5 * c.ncu);
+    hipLaunchKernelGGL(k_hsolve_wave, dim3(blocks), dim3(256), 0, c.stream, c.kg, c.box_ok, c.n,
+                       c.bn, rec, c.cid, c.root, c.active, c.ktab, c.opt.h_fac, c.pp_gather,
+                       list_cap, by_waves ? nullptr : c.hq, c.hq_len, c.h, c.zeta, c.rho, c.omega,
+                       c.divv, c.drhodt, c.flag, c.wstat);
     SX_HIP(hipGetLastError());
     SX_HIP(hipMemcpyAsync(c.hostpin + 8, c.flag, sizeof(int), hipMemcpyDeviceToHost, c.stream));
     return SERENX_OK;

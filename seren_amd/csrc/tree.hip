@@ -322,6 +322,17 @@ __global__ void k_dfs(int n, int nc, const int *__restrict__ c_start, const int 
     hn[d].first = s;
 }
 
+// the children of every branch, consecutive in BFS order
+__global__ void k_children(int nc, const int *__restrict__ c_parent, int *__restrict__ c_first,
+                           int *__restrict__ c_last) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= nc) return;
+    const int p = c_parent[c];
+    if (p < 0) return;
+    if (c_parent[c - 1] != p) c_first[p] = c;
+    if (c + 1 == nc || c_parent[c + 1] != p) c_last[p] = c + 1;
+}
+
 __global__ void k_dfs_parent(int nc, const int *__restrict__ c_parent, const int *__restrict__ bfs2dfs,
                              int *__restrict__ dfs_parent) {
     int c = blockIdx.x * blockDim.x + threadIdx.x;
@@ -408,7 +419,9 @@ __device__ __forceinline__ void octupole_shift_exact(double *sc, const double *c
 __global__ void __launch_bounds__(256) k_stock(
     int nc, int base, int cnt, const int *__restrict__ bfs2dfs, GNode *__restrict__ gn,
     double *__restrict__ gs,
-    HNode *__restrict__ hn, double *__restrict__ bbmin, double *__restrict__ bbmax,
+    HNode *__restrict__ hn, BNode *__restrict__ bn, const int *__restrict__ c_first,
+    const int *__restrict__ c_last, const int *__restrict__ c_parent,
+    double *__restrict__ bbmin, double *__restrict__ bbmax,
     double *__restrict__ hmaxs, const double *__restrict__ x, const double *__restrict__ y,
     const double *__restrict__ z, const double *__restrict__ m, const double *__restrict__ h,
     int octupole, int mac, double thetamaxsqd, double abserror, double daux, double kernrange) {
@@ -603,6 +616,15 @@ __global__ void __launch_bounds__(256) k_stock(
         for (int k = 0; k < 3; k++)
             hh.half[k] = (float)((half[k] + 1.0e-9 * (fabs(hc[k]) + half[k])) * (1.0 + 1.0e-6));
     }
+    BNode &b = bn[base + j];
+    for (int k = 0; k < 3; k++) {
+        b.r[k] = hh.r[k];
+        b.half[k] = hh.half[k];
+    }
+    b.rmax = hh.rmax;
+    b.fc = leaf > 0 ? first : c_first[base + j];
+    b.k = leaf > 0 ? leaf : c_first[base + j] - c_last[base + j];
+    b.parent = c_parent[base + j];
 }
 
 // macscale multiplies the multipole-MAC term for the mixed walk's own
@@ -733,6 +755,9 @@ int ensure_tree_buffers(Ctx &c) {
     SX_TRY(dalloc(&c.gs, cc * 10));
     SX_TRY(dalloc(&c.gnf, cc));
     SX_TRY(dalloc(&c.hn, cc));
+    SX_TRY(dalloc(&c.bn, cc));
+    SX_TRY(dalloc(&c.c_first, cc));
+    SX_TRY(dalloc(&c.c_last, cc));
     // temporary storage for sort and scans
     size_t b1 = 0, b2 = 0, b3 = 0, b4 = 0;
     SX_HIP(rocprim::radix_sort_pairs(nullptr, b1, c.khi, c.khi2, c.idx, c.idx2, (unsigned)n, 0,
@@ -937,6 +962,8 @@ int build_tree(Ctx &c) {
                                    rocprim::plus<int>(), s));
     hipLaunchKernelGGL(k_dfs, dim3(nblk(c.nc)), dim3(TB), 0, s, n, c.nc, c.c_start, c.c_end,
                        c.c_level, c.c_leaf, c.off, c.firstlev, c.bfs2dfs, c.dfs2bfs, c.gn, c.hn);
+    hipLaunchKernelGGL(k_children, dim3(nblk(c.nc)), dim3(TB), 0, s, c.nc, c.c_parent, c.c_first,
+                       c.c_last);
     hipLaunchKernelGGL(k_dfs_parent, dim3(nblk(c.nc)), dim3(TB), 0, s, c.nc, c.c_parent,
                        c.bfs2dfs, c.dfs_parent);
     hipLaunchKernelGGL(k_leafsort, dim3(nblk(c.nc)), dim3(TB), 0, s, c.nc, c.c_start, c.c_leaf,
@@ -973,7 +1000,8 @@ int stock_tree(Ctx &c) {
         const int cnt = c.level_cnt[L];
         if (cnt == 0) continue;
         hipLaunchKernelGGL(k_stock, dim3(nblk(cnt)), dim3(TB), 0, s, c.nc, c.level_off[L], cnt,
-                           c.bfs2dfs, c.gn, c.gs, c.hn, c.bbmin, c.bbmax, c.hmaxs, c.x, c.y, c.z, c.m,
+                           c.bfs2dfs, c.gn, c.gs, c.hn, c.bn, c.c_first, c.c_last,
+                           c.c_parent, c.bbmin, c.bbmax, c.hmaxs, c.x, c.y, c.z, c.m,
                            c.h, oct, c.opt.mac, c.opt.thetamaxsqd, c.opt.abserror, c.daux,
                            c.kg.range);
     }
