@@ -76,16 +76,16 @@ __device__ __forceinline__ double rcp_fp64(double d) {
 // gravity_gradh.F90:42-86 for one pair, (dx, dy, dz) = r_j - r_p; t4 holds
 // (w4, w5, w6, 0) per table index; rangehj = KERNRANGE h_j (the reference's
 // product), invhj = 1/h_j.  The kernel index uses the reference's drmag =
-// sqrt(r^2) + 1e-20; 1/drmag comes from rcp_fp64.
+// sqrt(r^2) + 1e-20; 1/drmag comes from rcp_fp64.  The pair adds
+// f (dx, dy, dz) to the acceleration and m_j / 2 dpot to the potential, each
+// by one fused multiply-add; both tables' entries are loaded before either
+// is used.
 // Returns bit 0: r inside the kernel range of h_p, bit 1: of h_j.
-__device__ __forceinline__ unsigned pair_fp64(const KGeom &kg, const double4 *__restrict__ t4,
-                                               double invhp,
-                                               double zo_p, double dx, double dy, double dz,
-                                               double mj, double rangehj, double invhj,
-                                               double zetaj,
-                                               double &ax, double &ay, double &az,
-                                               double &pot) {
-#pragma clang fp contract(fast)
+__device__ __forceinline__ unsigned pair_terms(const KGeom &kg, const double4 *__restrict__ t4,
+                                               double invhp, double zo_p, double dx, double dy,
+                                               double dz, double mj, double rangehj, double invhj,
+                                               double zetaj, double &f, double &dpot) {
+#pragma clang fp contract(off)
     // r^2 unfused, as the reference forms it: standard SPH's h_gather puts
     // the pp_gather-th neighbour at r = KERNRANGE h_p exactly, and a fused
     // sum can move r across that boundary
@@ -93,34 +93,37 @@ __device__ __forceinline__ unsigned pair_fp64(const KGeom &kg, const double4 *__
     const double drmag = sqrt(drsqd) + SMALL_NUMBER;
     const double invdrmag = rcp_fp64(drmag);
     const double id2 = invdrmag * invdrmag;
-    double grav, dpot;
-    unsigned inside = 0;
-    if (invdrmag > kg.invrange * invhp) {
-        inside = 1;
-        const int kern = min((int)(kg.half * drmag * invhp), KERNTOT);
-        const double4 w = t4[kern];
-        grav = invhp * invhp * (w.y + zo_p * w.x * invhp * invhp);
-        dpot = invhp * w.z;
-    } else {
-        grav = id2;
-        dpot = invdrmag;
+    const bool in_p = invdrmag > kg.invrange * invhp;
+    const bool in_j = drmag < rangehj;
+    double4 wp = make_double4(0.0, 0.0, 0.0, 0.0), wj = wp;
+    if (in_p) wp = t4[min((int)(kg.half * drmag * invhp), KERNTOT)];
+    if (in_j) wj = t4[min((int)(kg.half * drmag * invhj), KERNTOT)];
+    double gp = id2, pp = invdrmag, gj = id2, pj = invdrmag;
+    if (in_p) {
+        gp = invhp * invhp * __fma_rn(zo_p * wp.x * invhp, invhp, wp.y);
+        pp = invhp * wp.z;
     }
-    if (drmag < rangehj) {
-        inside |= 2;
-        const int kern = min((int)(kg.half * drmag * invhj), KERNTOT);
-        const double4 w = t4[kern];
-        grav = grav + invhj * invhj * (w.y + zetaj * w.x * invhj * invhj);
-        dpot = dpot + invhj * w.z;
-    } else {
-        grav = grav + id2;
-        dpot = dpot + invdrmag;
+    if (in_j) {
+        gj = invhj * invhj * __fma_rn(zetaj * wj.x * invhj, invhj, wj.y);
+        pj = invhj * wj.z;
     }
-    const double f = 0.5 * mj * invdrmag * grav;
-    ax = ax + f * dx;
-    ay = ay + f * dy;
-    az = az + f * dz;
-    pot = pot + 0.5 * mj * dpot;
-    return inside;
+    f = 0.5 * mj * invdrmag * (gp + gj);
+    dpot = pp + pj;
+    return (in_p ? 1u : 0u) | (in_j ? 2u : 0u);
+}
+
+// the pair's terms added to a lane's own sums
+__device__ __forceinline__ void pair_fp64(const KGeom &kg, const double4 *__restrict__ t4,
+                                          double invhp, double zo_p, double dx, double dy,
+                                          double dz, double mj, double rangehj, double invhj,
+                                          double zetaj, double &ax, double &ay, double &az,
+                                          double &pot) {
+    double f, dpot;
+    (void)pair_terms(kg, t4, invhp, zo_p, dx, dy, dz, mj, rangehj, invhj, zetaj, f, dpot);
+    ax = __fma_rn(f, dx, ax);
+    ay = __fma_rn(f, dy, ay);
+    az = __fma_rn(f, dz, az);
+    pot = __fma_rn(0.5 * mj, dpot, pot);
 }
 
 // Gravity source record of particle j, 64 bytes in a buffer of its own (the
@@ -376,111 +379,212 @@ __global__ void __launch_bounds__(256) k_grav_cells_fp64(
     wave_stats(wstat, 0, vis, lvis);
 }
 
-// Phase 2: the pair terms of gravity_gradh.F90 over each lane's opened
-// leaves, in list order, added to the cell sums of phase 1.  A group whose
-// list did not fit repeats its walk (the same MAC decisions: they read the
-// stocked tree and the previous |a|, which phase 2 overwrites only after)
-// and takes the pairs from the leaves as it opens them.  One wave per group
-// at a time; the kernels below take the groups from the walk's queue.
+// Phase 2: the pair terms of gravity_gradh.F90 over each particle's opened
+// leaves, in list order, added to the cell sums of phase 1.
+//
+// A wave takes a part of a group, PAIR_TW = 16 targets with four lanes each.
+// The group's list comes 64 leaves at a time, one per lane; 16 ballots turn
+// its lane masks into one word of leaves per target, and each target goes
+// through its own leaves, its four lanes on four of a leaf's particles.  The
+// terms of four sources (f d and m_j / 2 dpot as factor pairs) go through
+// LDS to the target's four lanes, which add them in list order, one lane per
+// component: the same fused additions in the same order as one lane would
+// make, so the sums do not depend on the split.
+//
+// Why: with one lane per target (one wave per group, the union of its leaves
+// by uniform loads) a quarter of the lanes had opened the leaf at hand, and
+// the chain of record load, square root, reciprocal and table load took
+// half a microsecond per source.  Alone: uniform sphere of 2,048 particles
+// 467 -> 130 us, r^-2 sphere of 4,096 918 -> 361 us; the sums are the same
+// bit for bit.
+//
+// A group whose list did not fit repeats its walk for the part's 16 targets
+// (the same MAC decisions: they read the stocked tree and the previous |a|
+// and potential of these targets, which only this wave overwrites, after).
+constexpr int PAIR_LPT = 4;                  // lanes per target
+constexpr int PAIR_TW = WAVE / PAIR_LPT;     // targets of a wave
+
 template <int MACT, bool QUINTIC>
-__device__ __forceinline__ void pairs_group_fp64(
-    int g, int n, int nc, const GNode *__restrict__ gn, const double4 *__restrict__ rec,
-    const int *__restrict__ cid, const int2 *__restrict__ root_range,
-    const uint8_t *__restrict__ active, const double4 *__restrict__ t4,
-    double *__restrict__ ax, double *__restrict__ ay, double *__restrict__ az,
-    const double *__restrict__ cp, double *__restrict__ gpot, double *__restrict__ agm,
-    NearList near, unsigned long long *__restrict__ icount, const int2 *__restrict__ grp,
-    int ngrp,
-    unsigned &npp_out, unsigned &nin_p_out, unsigned &nin_j_out) {
+__device__ __forceinline__ void pairs_part_fp64(
+    int g, int part, int nc, const GNode *__restrict__ gn, const double4 *__restrict__ rec,
+    double2 (*__restrict__ xch)[WAVE + 1], const int *__restrict__ cid,
+    const int2 *__restrict__ root_range, const uint8_t *__restrict__ active,
+    const double4 *__restrict__ t4, double *__restrict__ ax, double *__restrict__ ay,
+    double *__restrict__ az, const double *__restrict__ cp, double *__restrict__ gpot,
+    double *__restrict__ agm, NearList near, const int2 *__restrict__ grp, unsigned &npp,
+    unsigned &nin_p, unsigned &nin_j) {
     constexpr KGeom kg = walk_geom<QUINTIC>();
-    const int lane = (int)(threadIdx.x & (WAVE - 1));
+    const int lane = (int)(threadIdx.x & (WAVE - 1)), sub = lane & (PAIR_LPT - 1);
     const int2 gr = grp[g];
-    const int p = gr.x + lane;
+    const int p = gr.x + part * PAIR_TW + lane / PAIR_LPT;
     const bool valid = p < gr.y && active[p];
     if (ballot(valid) == 0) return;
-    double rpx = 0, rpy = 0, rpz = 0, invhp = 1.0, zo_p = 0.0;
-    double gx = 0, gy = 0, gz = 0, gp = 0, afactor = 0.0;
+    double rpx = 0, rpy = 0, rpz = 0, invhp = 1.0, zo_p = 0.0, acc = 0.0;
     if (valid) {
         const double4 a = rec[2 * (size_t)p], b = rec[2 * (size_t)p + 1];
         rpx = a.x; rpy = a.y; rpz = a.z;
         invhp = b.y;
         zo_p = b.z;
-        gx = ax[p]; gy = ay[p]; gz = az[p]; gp = cp[p];
-        if (MACT != SERENX_MAC_GEOMETRIC) afactor = mac_afactor<MACT>(agm[p], gpot[p]);
+        acc = (sub == 0 ? ax : sub == 1 ? ay : sub == 2 ? az : cp)[p];
     }
-    unsigned npp = 0, nin_p = 0, nin_j = 0;
-    auto leaf_pairs = [&](int first, int count, bool mine) {
-        for (int i = 0; i < count; i++) {
-            const int j = first + i;
-            const double4 a = rec[2 * (size_t)j], b = rec[2 * (size_t)j + 1];
-            const bool act = mine && j != p;
+    // 64 entries of the list, one per lane (d: leaf, word: the entries the
+    // lane's target opened)
+    auto chunk = [&](int d, unsigned long long word) {
+        int k0 = 0;   // first particle of the leaf's part at hand
+        // the target's next four sources: particle j of the lane, if any
+        auto next = [&](int &j) -> bool {
+            const int e = word ? __ffsll((long long)word) - 1 : 0;
+            const int de = __shfl(d, e, WAVE);
+            const int cnt = de & 15, i = k0 + sub;
+            const bool act = word != 0 && i < cnt;
+            j = act ? (de >> 4) + i : gr.x;
+            if (word) {
+                k0 += PAIR_LPT;
+                if (k0 >= cnt) {
+                    k0 = 0;
+                    word &= word - 1;
+                }
+            }
+            return act && j != p;
+        };
+        bool more = ballot(word != 0) != 0;
+        int j;
+        bool act = next(j);
+        double4 a = rec[2 * (size_t)j], b = rec[2 * (size_t)j + 1];
+        while (more) {
+            more = ballot(word != 0) != 0;
+            // the next sources' records are in flight while these are used
+            int jn;
+            const bool actn = next(jn);
+            const double4 an = rec[2 * (size_t)jn], bn = rec[2 * (size_t)jn + 1];
+            double dx = 0.0, dy = 0.0, dz = 0.0, f = 0.0, hm = 0.0, dpot = 0.0;
             unsigned in_ = 0;
-            if (act)
-                in_ = pair_fp64(kg, t4, invhp, zo_p, a.x - rpx, a.y - rpy, a.z - rpz, a.w, b.w,
-                                b.y, b.z, gx, gy, gz, gp);
+            if (act) {
+                dx = a.x - rpx;
+                dy = a.y - rpy;
+                dz = a.z - rpz;
+                hm = 0.5 * a.w;
+                in_ = pair_terms(kg, t4, invhp, zo_p, dx, dy, dz, a.w, b.w, b.y, b.z, f, dpot);
+            }
             npp += lanes(act);
             nin_p += lanes(in_ & 1);
             nin_j += lanes(in_ & 2);
+            // a lane without a source adds 0 * 0, which leaves the sum (never
+            // -0) as it is
+            xch[0][lane] = make_double2(f, dx);
+            xch[1][lane] = make_double2(f, dy);
+            xch[2][lane] = make_double2(f, dz);
+            xch[3][lane] = make_double2(hm, dpot);
+            wave_lds_fence();
+            double2 t[PAIR_LPT];
+#pragma unroll
+            for (int i = 0; i < PAIR_LPT; i++) t[i] = xch[sub][(lane & ~(PAIR_LPT - 1)) + i];
+            wave_lds_fence();
+#pragma unroll
+            for (int i = 0; i < PAIR_LPT; i++) acc = __fma_rn(t[i].x, t[i].y, acc);
+            a = an;
+            b = bn;
+            act = actn;
         }
+    };
+    // the words of the lanes' targets from the entries' lane masks: target t
+    // of the part is bit lo + t of a mask
+    auto words = [&](unsigned long long m, int lo) {
+        const unsigned mm = (unsigned)(m >> lo);
+        unsigned long long word = 0;
+#pragma unroll
+        for (int t = 0; t < PAIR_TW; t++) {
+            const unsigned long long b = ballot((mm >> t) & 1u);
+            if (lane / PAIR_LPT == t) word = b;
+        }
+        return valid ? word : 0ull;
     };
     const int len = uniform(near.len[g]);
     if (len <= near.cap) {
-        for (int e = 0; e < len; e++) {
-            const int d = uniform(near.leaf[(size_t)g * near.stride + e]);
-            const unsigned long long m = near.mask[(size_t)g * near.stride + e];
-            leaf_pairs(d >> 4, d & 15, valid && ((m >> lane) & 1ull));
+        const size_t at = (size_t)g * near.stride;
+        for (int e0 = 0; e0 < len; e0 += WAVE) {
+            const bool have = e0 + lane < len;
+            const int d = have ? near.leaf[at + e0 + lane] : 0;
+            const unsigned long long m = have ? near.mask[at + e0 + lane] : 0ull;
+            chunk(d, words(m, part * PAIR_TW));
         }
     } else {
-        const int2 rr = valid ? root_range[cid[p]] : make_int2(nc, nc);
+        // the part's walk again, target t on lane t
+        const int q = gr.x + part * PAIR_TW + lane;
+        const bool walks = lane < PAIR_TW && q < gr.y && active[q];
+        double qx = 0, qy = 0, qz = 0, afactor = 0.0;
+        int2 rr = make_int2(nc, nc);
+        if (walks) {
+            const double4 a = rec[2 * (size_t)q];
+            qx = a.x; qy = a.y; qz = a.z;
+            if (MACT != SERENX_MAC_GEOMETRIC) afactor = mac_afactor<MACT>(agm[q], gpot[q]);
+            rr = root_range[cid[q]];
+        }
+        int resume = rr.x;
+        int c = uniform(wave_min_int(resume));
         unsigned lv = 0;
-        (void)group_walk(
-            gn, nc, valid, rr.x, rr.y, lv,
-            [&](const GNode &nd, bool) -> int {
-                const double dr[3] = {rpx - nd.r[0], rpy - nd.r[1], rpz - nd.r[2]};
-                const double drsqd = dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2];
-                bool accept;
-                if (MACT == SERENX_MAC_GEOMETRIC)
-                    accept = drsqd > nd.dminsqd;
-                else
-                    accept = drsqd > nd.mac * afactor && drsqd > nd.dminsqd;
-                accept = accept && nd.leaf != 1;
-                if (accept) return WALK_SKIP;
-                return nd.leaf > 0 ? WALK_LEAF : WALK_DESCEND;
-            },
-            [&](const GNode &nd, bool mine) { leaf_pairs(nd.first, nd.leaf, mine); });
+        while (c < nc) {
+            int cnt = 0, d = 0;
+            unsigned long long m = 0;
+            while (c < nc && cnt < WAVE)
+                group_step(
+                    gn, nc, rr.y, c, resume, lv,
+                    [&](const GNode &nd, bool) -> int {
+                        const double dr[3] = {qx - nd.r[0], qy - nd.r[1], qz - nd.r[2]};
+                        const double drsqd = dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2];
+                        bool accept;
+                        if (MACT == SERENX_MAC_GEOMETRIC)
+                            accept = drsqd > nd.dminsqd;
+                        else
+                            accept = drsqd > nd.mac * afactor && drsqd > nd.dminsqd;
+                        accept = accept && nd.leaf != 1;
+                        if (accept) return WALK_SKIP;
+                        return nd.leaf > 0 ? WALK_LEAF : WALK_DESCEND;
+                    },
+                    [&](const GNode &nd, bool mine) {
+                        const unsigned long long mm = ballot(mine);
+                        if (lane == cnt) {
+                            d = (nd.first << 4) | nd.leaf;
+                            m = mm;
+                        }
+                        cnt++;
+                    });
+            chunk(d, words(m, 0));
+        }
     }
+    // the gravity acceleration (k_add_grav adds it to a) and the potential
+    const int t0 = lane & ~(PAIR_LPT - 1);
+    const double gx = __shfl(acc, t0, WAVE), gy = __shfl(acc, t0 + 1, WAVE),
+                 gz = __shfl(acc, t0 + 2, WAVE);
     if (valid) {
-        ax[p] = gx;   // the gravity acceleration; k_add_grav adds it to a
-        ay[p] = gy;
-        az[p] = gz;
-        gpot[p] = gp;
-        if (MACT != SERENX_MAC_GEOMETRIC) agm[p] = sqrt(gx * gx + gy * gy + gz * gz);
+        (sub == 0 ? ax : sub == 1 ? ay : sub == 2 ? az : gpot)[p] = acc;
+        if (MACT != SERENX_MAC_GEOMETRIC && sub == 0) agm[p] = sqrt(gx * gx + gy * gy + gz * gz);
     }
-    npp_out += npp;
-    nin_p_out += nin_p;
-    nin_j_out += nin_j;
 }
 
 template <int MACT, bool QUINTIC>
 __global__ void __launch_bounds__(256) k_grav_pairs_fp64(
-    int n, int nc, const GNode *__restrict__ gn, const double4 *__restrict__ rec,
+    int nc, const GNode *__restrict__ gn, const double4 *__restrict__ rec,
     const int *__restrict__ cid, const int2 *__restrict__ root_range,
     const uint8_t *__restrict__ active, const double4 *__restrict__ t4,
     double *__restrict__ ax, double *__restrict__ ay, double *__restrict__ az,
     const double *__restrict__ cp, double *__restrict__ gpot, double *__restrict__ agm,
     NearList near, unsigned long long *__restrict__ icount, const int2 *__restrict__ grp,
-    int ngrp,
     GroupQueue queue) {
     // persistent over the walk's queue: the groups of each XCD range
     // longest-first (by the previous walk's cost), as phase 1 takes them
     __builtin_amdgcn_s_setprio(2);
+    // per wave and component, the lanes' factor pairs; one slot of padding
+    // spreads the components of a target's four lanes over the banks
+    __shared__ double2 xch[256 / WAVE][PAIR_LPT][WAVE + 1];
     unsigned npp = 0, nin_p = 0, nin_j = 0;   // wave totals
     const int home = blockIdx.x % NXCD;
-    int qdone = 0;
-    for (int g = next_group(queue, home, qdone); g >= 0; g = next_group(queue, home, qdone))
-        pairs_group_fp64<MACT, QUINTIC>(g, n, nc, gn, rec, cid, root_range, active, t4, ax, ay,
-                                        az, cp, gpot, agm, near, icount, grp, ngrp, npp, nin_p,
-                                        nin_j);
+    int qdone = 0, part = 0;
+    for (int g = next_part<PAIR_LPT>(queue, home, qdone, part); g >= 0;
+         g = next_part<PAIR_LPT>(queue, home, qdone, part))
+        pairs_part_fp64<MACT, QUINTIC>(g, part, nc, gn, rec, xch[threadIdx.x / WAVE], cid,
+                                       root_range, active, t4, ax, ay, az, cp, gpot, agm, near,
+                                       grp, npp, nin_p, nin_j);
     if ((threadIdx.x & 63) == 0) {
         unsigned long long *ic = ctr_row(icount);
         atomicAdd(ic + 1, (unsigned long long)npp);
@@ -926,8 +1030,8 @@ __global__ void __launch_bounds__(256) k_direct(KGeom kg, int n, int nt,
         if (valid) {
             for (int k = 0; k < lim; k++) {
                 if (base + k == p || base + k < lo || base + k >= hi) continue;
-                (void)pair_fp64(kg, t4, invhp, zo_p, sx[k] - rpx, sy[k] - rpy, sz[k] - rpz, sm[k],
-                                sh[k], sih[k], szt[k], gx, gy, gz, gp);
+                pair_fp64(kg, t4, invhp, zo_p, sx[k] - rpx, sy[k] - rpy, sz[k] - rpz, sm[k],
+                          sh[k], sih[k], szt[k], gx, gy, gz, gp);
             }
         }
         __syncthreads();
@@ -960,8 +1064,8 @@ int pair_cap(const Ctx &c) {
 // many as the device holds at once (each wave then takes group after
 // group); without it, one wave per group.
 template <class K>
-int walk_blocks(Ctx &c, K kernel, int cap) {
-    const int per_wave = (c.gq.ngroups + 3) / 4;
+int walk_blocks(Ctx &c, K kernel, int cap, int parts = 1) {
+    const int per_wave = (c.gq.ngroups * parts + 3) / 4;
     if (c.walk_queue == 0) return std::max(per_wave, 1);
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, TB, 0) != hipSuccess ||
@@ -1015,10 +1119,10 @@ void launch_pairs(Ctx &c, const double4 *rec, hipStream_t s, int cap) {
                            c.gaz, c.gpc, c.gpot, c.agm, near_list(c), c.icount, c.grp, c.ngrp, q);
     } else {
         auto k = k_grav_pairs_fp64<MACT, QUINTIC>;
-        hipLaunchKernelGGL(k, dim3(walk_blocks(c, k, cap)), dim3(TB), 0, s, c.n, c.nc, c.gn,
+        hipLaunchKernelGGL(k, dim3(walk_blocks(c, k, cap, PAIR_LPT)), dim3(TB), 0, s, c.nc, c.gn,
                            rec, c.cid, c.root_range, c.active,
                            reinterpret_cast<const double4 *>(c.ktab + KT_G4_OFF), c.gax, c.gay,
-                           c.gaz, c.gpc, c.gpot, c.agm, near_list(c), c.icount, c.grp, c.ngrp, q);
+                           c.gaz, c.gpc, c.gpot, c.agm, near_list(c), c.icount, c.grp, q);
     }
 }
 

@@ -400,13 +400,6 @@ struct WaveSearch {
     double4 term[WAVE];    // terms of one batch of candidates, in list order
 };
 
-// orders the wave's LDS accesses around a point
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // inclusive prefix sum over the lanes of a wave
 __device__ __forceinline__ int wave_prefix(int v, int lane) {
 #pragma unroll

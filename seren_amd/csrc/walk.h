@@ -26,6 +26,13 @@ __device__ __forceinline__ unsigned long long ballot(bool pred) {
     return __builtin_amdgcn_ballot_w64(pred);
 }
 
+// orders the wave's LDS accesses around a point
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The dispatcher deals the workgroups of a launch to the 8 XCDs round-robin
 // (workgroup i runs on XCD i % 8), and each XCD has its own L2.  This returns
 // the logical block index under which XCD x receives the x-th contiguous
@@ -147,6 +154,39 @@ static __device__ __noinline__ double ref_pow_third(double x) {
 // walk's SIMD utilisation).
 enum { WALK_SKIP = 0, WALK_DESCEND = 1, WALK_LEAF = 2 };
 
+// One visit: cell c, then c moves to the wave's next cell (nc: the walk is
+// over).  resume is the lane's own position.
+template <class Node, class Visit, class Leaf>
+__device__ __forceinline__ void group_step(const Node *__restrict__ nodes, int nc, int end, int &c,
+                                           int &resume, unsigned &lane_visits, Visit &&visit,
+                                           Leaf &&leaf) {
+    // read the cell in wave-uniform control flow from a uniform address so
+    // that it comes through the scalar cache into SGPRs
+    const Node nd = nodes[c];
+    const bool here = resume == c;
+    int act = visit(nd, here);
+    lane_visits += (unsigned)__popcll(ballot(here));
+    if (here) {
+        resume = (act == WALK_DESCEND) ? c + 1 : nd.next;
+        if (resume >= end) resume = nc;   // past the end of the lane's own tree
+    } else {
+        act = WALK_SKIP;
+    }
+    if (ballot(act == WALK_LEAF)) leaf(nd, act == WALK_LEAF);
+    // the next cell is the lowest resume pointer.  A lane descending makes
+    // it c + 1.  Otherwise no lane's pointer lies inside c's subtree
+    // (c, next): a lane reaches such a cell only through c itself, since
+    // subtrees are contiguous and nest, so a lane that was at c and moved
+    // on to c's next (not past its tree's end) holds the minimum; only
+    // when none did is the wave minimum reduced.
+    if (ballot(act == WALK_DESCEND))
+        c = c + 1;
+    else if (ballot(here) & ballot(resume == nd.next))
+        c = nd.next;
+    else
+        c = uniform(wave_min_int(resume));
+}
+
 template <class Node, class Visit, class Leaf>
 __device__ __forceinline__ unsigned group_walk(const Node *__restrict__ nodes, int nc,
                                                bool walking, int start, int end,
@@ -156,32 +196,8 @@ __device__ __forceinline__ unsigned group_walk(const Node *__restrict__ nodes, i
     int c = uniform(wave_min_int(resume));
     unsigned visits = 0;
     while (c < nc) {
-        // read the cell in wave-uniform control flow from a uniform address so
-        // that it comes through the scalar cache into SGPRs
-        const Node nd = nodes[c];
         visits++;
-        const bool here = resume == c;
-        int act = visit(nd, here);
-        lane_visits += (unsigned)__popcll(ballot(here));
-        if (here) {
-            resume = (act == WALK_DESCEND) ? c + 1 : nd.next;
-            if (resume >= end) resume = nc;   // past the end of the lane's own tree
-        } else {
-            act = WALK_SKIP;
-        }
-        if (ballot(act == WALK_LEAF)) leaf(nd, act == WALK_LEAF);
-        // the next cell is the lowest resume pointer.  A lane descending makes
-        // it c + 1.  Otherwise no lane's pointer lies inside c's subtree
-        // (c, next): a lane reaches such a cell only through c itself, since
-        // subtrees are contiguous and nest, so a lane that was at c and moved
-        // on to c's next (not past its tree's end) holds the minimum; only
-        // when none did is the wave minimum reduced.
-        if (ballot(act == WALK_DESCEND))
-            c = c + 1;
-        else if (ballot(here) & ballot(resume == nd.next))
-            c = nd.next;
-        else
-            c = uniform(wave_min_int(resume));
+        group_step(nodes, nc, end, c, resume, lane_visits, visit, leaf);
     }
     return visits;
 }
@@ -206,19 +222,30 @@ struct GroupQueue {
 
 __device__ __forceinline__ int queue_lo(int q, int ngroups) { return (q * ngroups + NXCD - 1) / NXCD; }
 
-// the next group of the calling wave (wave-uniform), -1 when none is left;
-// q counts the ranges this wave has exhausted
-__device__ __forceinline__ int next_group(const GroupQueue &Q, int home, int &q) {
+// the next part of a group for the calling wave (wave-uniform): the queue
+// hands out PARTS parts of every group in turn.  Returns the group and its
+// part, -1 when none is left; q counts the ranges this wave has exhausted
+template <int PARTS>
+__device__ __forceinline__ int next_part(const GroupQueue &Q, int home, int &q, int &part) {
     while (q < NXCD) {
         const int r = (home + q) % NXCD;
         const int lo = queue_lo(r, Q.ngroups), hi = queue_lo(r + 1, Q.ngroups);
         int t = 0;
         if ((threadIdx.x & 63) == 0) t = atomicAdd(Q.ctr + r, 1);
         t = uniform(__shfl(t, 0, 64));
-        if (lo + t < hi) return Q.order[lo + t];
+        if (lo + t / PARTS < hi) {
+            part = t % PARTS;
+            return Q.order[lo + t / PARTS];
+        }
         q++;
     }
     return -1;
+}
+
+// the next group of the calling wave (wave-uniform), -1 when none is left
+__device__ __forceinline__ int next_group(const GroupQueue &Q, int home, int &q) {
+    int part;
+    return next_part<1>(Q, home, q, part);
 }
 
 // Adds per-wave walk statistics into stats[k0], stats[k0 + 1] from lane 0:
