@@ -255,14 +255,27 @@ int ensure_capacity(Ctx &c, int n) {
     // per group of the gravity walk (at most one partial group per cloud)
     const size_t ng = walk_max_groups(n, c.pp_gather);
     SX_TRY(dalloc(&c.grp, ng));
-    c.pl_entries = near_list_entries(n);
-    SX_TRY(dalloc(&c.pl_leaf, c.pl_entries));
-    SX_TRY(dalloc(&c.pl_mask, c.pl_entries));
+    c.pl_npage = (int)(near_list_entries(n) / PL_PAGE);
+    SX_TRY(dalloc(&c.pl_leaf, near_list_entries(n)));
+    SX_TRY(dalloc(&c.pl_mask, near_list_entries(n)));
     SX_TRY(dalloc(&c.pl_len, ng));
+    SX_TRY(dalloc(&c.pl_page, ng * PL_PAGES));
+    // two list-walk blocks fit a CU; a block never visits more cells than the
+    // context has (2 n + 2 and the roots of a forest)
+    c.lw_blocks = (int)std::min(ng, (size_t)2 * c.ncu);
+    c.lw_cap = (int)std::min((size_t)LW_CAP, 2 * nn + (size_t)forest_max_clouds(n, c.pp_gather));
+    const size_t lw = (size_t)c.lw_blocks * c.lw_cap;
+    SX_TRY(dalloc(&c.lw_ids, lw));
+    SX_TRY(dalloc(&c.lw_list, lw + 8 * (size_t)c.lw_blocks));
+    SX_TRY(dalloc(&c.lw_in, lw));
+    SX_TRY(dalloc(&c.lw_open, lw));
+    SX_TRY(dalloc(&c.lw_mask, lw + 8 * (size_t)c.lw_blocks));
+    SX_TRY(dalloc(&c.lw_group, ng));
+    SX_TRY(dalloc(&c.lw_at, ng));
     SX_TRY(dalloc(&c.hlist, (((size_t)n + 255) / 256) * 4 * HL_SLOTS * WAVE));
     // work queue of the gravity walk: one entry per group
     Ctx::WalkQueue &q = c.gq;
-    SX_TRY(dalloc(&q.ctr, (size_t)(2 * NXCD)));   // phase 1 and phase 2 counters
+    SX_TRY(dalloc(&q.ctr, (size_t)(2 * NXCD + 3)));   // phase 1 and phase 2 counters, ...
     SX_TRY(dalloc(&q.cost, ng));
     SX_TRY(dalloc(&q.order, ng));
     SX_TRY(dalloc(&q.vals, ng));
@@ -296,7 +309,8 @@ void free_all(Ctx &c) {
                     c.root_range, c.sorttmp, c.c_start, c.c_end, c.c_parent, c.c_leaf,
                     c.c_level, c.bfs2dfs, c.dfs2bfs, c.dfs_parent, c.bbmin, c.bbmax,
                     c.hmaxs, c.gn, c.gs, c.gnf, c.hn, c.ktab, c.icount, c.wstat, c.band,
-                    c.grec, c.gax, c.gay, c.gaz, c.gpc, c.grp, c.pl_leaf, c.pl_mask, c.pl_len, c.gq.ctr, c.gq.cost, c.gq.order,
+                    c.grec, c.gax, c.gay, c.gaz, c.gpc, c.grp, c.pl_leaf, c.pl_mask, c.pl_len, c.pl_page,
+                    c.lw_ids, c.lw_list, c.lw_in, c.lw_open, c.lw_mask, c.lw_group, c.lw_at, c.gmac, c.gq.ctr, c.gq.cost, c.gq.order,
                     c.gq.vals, c.gq.keys, c.gq.keys2, c.gq.tmp, c.fs_ck, c.fs_ck2, c.fs_pos,
                     c.fs_perm, c.fs_v, c.fs_k};
     for (void *p : ptrs)
@@ -357,13 +371,15 @@ size_t ctx_device_bytes(const Ctx &c) {
     b += nn * (24 * 8 + 16 * 8 + 12 * 8);                   // SoA, tmpd, hydro/gravity records
     b += walk_max_groups(c.cap, c.pp_gather) * (size_t)(4 + 8 + 6 * 8);  // walk groups
     b += near_list_entries(c.cap) * 12;                              // near-field lists
+    b += walk_max_groups(c.cap, c.pp_gather) * (PL_PAGES + 2) * (size_t)4; // their pages, left walks
+    b += (size_t)c.lw_blocks * (c.lw_cap * (size_t)32 + 96);             // list walk
     b += particle_waves(c.cap) * (NB_CAP + 1) * 4;                   // neighbour-walk leaves
     b += nn * 4;                                                     // wave h-solve queue
     b += nn * (5 * 4 + 1) + nn * (size_t)c.pp_limit * 4;    // ints, active, neighbour rows
     b += (((size_t)c.cap + 255) / 256) * 4 * HL_SLOTS * WAVE * 4;   // h-solve lists
     b += nn * (4 * 8 + 2 * 4 + 2 + 5 * 4 + 1);              // tree build scratch
     b += cc * (sizeof(GNode) + 10 * 8 + sizeof(GNodeF) + sizeof(HNode) + sizeof(BNode) +
-               10 * 4 + 7 * 8);
+               sizeof(GMac) + 10 * 4 + 7 * 8);
     b += c.sorttmp_bytes + c.ovf_cap * 4 + sizeof(double) * KT_TOTAL;
     if (c.st.on) b += nn * (11 * 8 + 8 + 4);                 // step state
     if (c.sv.on) b += nn * 3 * 8 + (size_t)c.ncloud * 25;    // serving state

@@ -112,18 +112,20 @@ __device__ __forceinline__ unsigned pair_terms(const KGeom &kg, const double4 *_
     return (in_p ? 1u : 0u) | (in_j ? 2u : 0u);
 }
 
-// the pair's terms added to a lane's own sums
-__device__ __forceinline__ void pair_fp64(const KGeom &kg, const double4 *__restrict__ t4,
-                                          double invhp, double zo_p, double dx, double dy,
-                                          double dz, double mj, double rangehj, double invhj,
-                                          double zetaj, double &ax, double &ay, double &az,
-                                          double &pot) {
+// the pair's terms added to a lane's own sums; the same bits returned
+__device__ __forceinline__ unsigned pair_fp64(const KGeom &kg, const double4 *__restrict__ t4,
+                                              double invhp, double zo_p, double dx, double dy,
+                                              double dz, double mj, double rangehj, double invhj,
+                                              double zetaj, double &ax, double &ay, double &az,
+                                              double &pot) {
     double f, dpot;
-    (void)pair_terms(kg, t4, invhp, zo_p, dx, dy, dz, mj, rangehj, invhj, zetaj, f, dpot);
+    const unsigned in_ =
+        pair_terms(kg, t4, invhp, zo_p, dx, dy, dz, mj, rangehj, invhj, zetaj, f, dpot);
     ax = __fma_rn(f, dx, ax);
     ay = __fma_rn(f, dy, ay);
     az = __fma_rn(f, dz, az);
     pot = __fma_rn(0.5 * mj, dpot, pot);
+    return in_;
 }
 
 // Gravity source record of particle j, 64 bytes in a buffer of its own (the
@@ -242,40 +244,54 @@ __device__ __forceinline__ void cell_terms(T x, T y, T z, T ir, T m, const T *q,
 // 10 moments instead of 18 coefficients to stay at two cache lines):
 // G = grad S = 2 H, S formed as (r.G) / 3.
 //   s = [x^3 x^2y y^2x y^3 z^2x z^2y z^3 x^2z y^2z xyz]
-template <int OCT, class T>
-__device__ __forceinline__ void cell_terms_s(T x, T y, T z, T ir, T m, const T *q, const T *s,
-                                             T &ax, T &ay, T &az, T &pot) {
-#pragma clang fp contract(fast)
-    const T ir2 = ir * ir;
-    const T ir3 = ir2 * ir;
-    const T ir5 = ir3 * ir2;
-    const T ir7 = ir5 * ir2;
-    const T Qx = q[0] * x + q[1] * y + q[3] * z;
-    const T Qy = q[1] * x + q[2] * y + q[4] * z;
-    const T Qz = q[3] * x + q[4] * y + q[5] * z;
-    const T qs = x * Qx + y * Qy + z * Qz;
-    T crad = -(m * ir3) - T(2.5) * qs * ir7;
-    T phi = m * ir + T(0.5) * qs * ir5;
-    T fx = Qx * ir5, fy = Qy * ir5, fz = Qz * ir5;
+// Every multiply-add is written out: left to the compiler, which of two
+// products is rounded changes from one caller to the next, and with it the
+// FP32 rounding of the results.
+template <int OCT>
+__device__ __forceinline__ void cell_terms_s(float x, float y, float z, float ir, float m,
+                                             const float *q, const float *s, float &ax, float &ay,
+                                             float &az, float &pot) {
+#pragma clang fp contract(off)
+    const float ir2 = ir * ir;
+    const float ir3 = ir * ir2;
+    const float ir5 = ir2 * ir3;
+    const float ir7 = ir2 * ir5;
+    auto dot = [](float a0, float b0, float a1, float b1, float a2, float b2) {
+        return __builtin_fmaf(a2, b2, __builtin_fmaf(a1, b1, a0 * b0));
+    };
+    const float Qx = dot(q[0], x, q[1], y, q[3], z);
+    const float Qy = dot(q[1], x, q[2], y, q[4], z);
+    const float Qz = dot(q[3], x, q[4], y, q[5], z);
+    const float qs = dot(Qx, x, Qy, y, Qz, z);
+    float crad = __builtin_fmaf(ir7, -2.5f * qs, -(m * ir3));
+    float phi = __builtin_fmaf(m, ir, ir5 * (0.5f * qs));
+    float fx, fy, fz;
     if (OCT) {
-        const T xx = x * x, yy = y * y, zz = z * z;
-        const T xy = x * y, xz = x * z, yz = y * z;
-        const T xx3 = T(3) * xx, yy3 = T(3) * yy, zz3 = T(3) * zz;
-        const T xy2 = xy + xy, xz2 = xz + xz, yz2 = yz + yz;
-        const T Gx = s[0] * xx3 + s[1] * xy2 + s[7] * xz2 + s[2] * yy + s[4] * zz + s[9] * yz;
-        const T Gy = s[1] * xx + s[2] * xy2 + s[3] * yy3 + s[5] * zz + s[9] * xz + s[8] * yz2;
-        const T Gz = s[7] * xx + s[8] * yy + s[6] * zz3 + s[4] * xz2 + s[5] * yz2 + s[9] * xy;
-        const T rg = x * Gx + y * Gy + z * Gz;   // 3 S
-        const T h7 = T(0.5) * ir7;
-        crad = crad - T(3.5 / 3.0) * rg * ir7 * ir2;
-        phi = phi + T(0.5 / 3.0) * rg * ir7;
-        fx = fx + h7 * Gx;
-        fy = fy + h7 * Gy;
-        fz = fz + h7 * Gz;
+        const float xx = x * x, yy = y * y, zz = z * z;
+        const float xy = x * y, xz = x * z, yz = y * z;
+        const float xx3 = 3.0f * xx, yy3 = 3.0f * yy, zz3 = 3.0f * zz;
+        const float xy2 = xy + xy, xz2 = xz + xz, yz2 = yz + yz;
+        auto dot3 = [](float v, float a0, float b0, float a1, float b1, float a2, float b2) {
+            return __builtin_fmaf(a2, b2, __builtin_fmaf(a1, b1, __builtin_fmaf(a0, b0, v)));
+        };
+        const float Gx = dot3(dot(s[0], xx3, s[1], xy2, s[7], xz2), s[2], yy, s[4], zz, s[9], yz);
+        const float Gy = dot3(dot(s[1], xx, s[2], xy2, s[3], yy3), s[5], zz, s[9], xz, s[8], yz2);
+        const float Gz = dot3(dot(s[7], xx, s[8], yy, s[6], zz3), s[4], xz2, s[5], yz2, s[9], xy);
+        const float rg = dot(Gx, x, Gy, y, Gz, z);   // 3 S
+        const float h7 = 0.5f * ir7;
+        crad = __builtin_fmaf(ir2, ir7 * ((-3.5f / 3.0f) * rg), crad);
+        phi = __builtin_fmaf(ir7, (0.5f / 3.0f) * rg, phi);
+        fx = __builtin_fmaf(crad, x, __builtin_fmaf(h7, Gx, Qx * ir5));
+        fy = __builtin_fmaf(crad, y, __builtin_fmaf(h7, Gy, Qy * ir5));
+        fz = __builtin_fmaf(crad, z, __builtin_fmaf(h7, Gz, Qz * ir5));
+    } else {
+        fx = __builtin_fmaf(ir5, Qx, crad * x);
+        fy = __builtin_fmaf(ir5, Qy, crad * y);
+        fz = __builtin_fmaf(ir5, Qz, crad * z);
     }
-    ax = ax + (fx + crad * x);
-    ay = ay + (fy + crad * y);
-    az = az + (fz + crad * z);
+    ax = ax + fx;
+    ay = ay + fy;
+    az = az + fz;
     pot = pot + phi;
 }
 
@@ -286,284 +302,63 @@ __device__ __forceinline__ void cell_fp64(const GNode &g, const double dr[3], do
     cell_terms<OCT, double>(dr[0], dr[1], dr[2], ir, g.m, g.q, g.oc, ax, ay, az, pot);
 }
 
-// Near-field list of a group: the leaves its walk opened, in DFS order, as
+// Near-field lists: per group, the leaves its walk opened, in DFS order, as
 // (first particle << 4) | particle count, with the mask of the lanes that
-// opened each.  Phase 1 of the walk writes it, phase 2 reads it.
+// opened each.  Phase 1 of the walk writes them, phase 2 reads them.  Entries
+// lie in pages of a pool (a group knows its number of leaves before it takes
+// its pages, so the pool serves lists of any length without waste).
 struct NearList {
-    int *leaf;                    // ngroups x stride entries
-    unsigned long long *mask;     // ngroups x stride lane masks
-    int *len;                     // per group: entries found (> cap: list incomplete)
-    int cap;                      // entries a group may store (<= stride)
-    int stride;                   // entries per group in leaf[] and mask[]
-};
-
-__device__ __forceinline__ void near_append(const NearList &L, int g, int &len, int first,
-                                            int count, unsigned long long mask) {
-    if ((threadIdx.x & 63) == 0 && len < L.cap) {
-        L.leaf[(size_t)g * L.stride + len] = (first << 4) | count;
-        L.mask[(size_t)g * L.stride + len] = mask;
+    int *leaf;                    // npage x PL_PAGE entries
+    unsigned long long *mask;     // their lane masks
+    int *page;                    // per group: PL_PAGES page numbers
+    int *next;                    // next free page
+    int *len;                     // per group: entries (NEAR_DROPPED: not stored)
+    int cap;                      // entries a group may store (<= PL_PAGES PL_PAGE)
+    int npage;                    // pages of the pool
+    __device__ __forceinline__ size_t slot(int g, int e) const {
+        return (size_t)page[(size_t)g * PL_PAGES + e / PL_PAGE] * PL_PAGE + e % PL_PAGE;
     }
-    len++;
-}
+};
+constexpr int NEAR_DROPPED = 0x7FFFFFFF;
 
-// The FP64 walk in two phases, so that the traversal and the cell terms --
-// which need only the positions, the tree stocked with the previous h (Q2:
+// The walk in two phases, so that the traversal and the cell terms -- which
+// need only the positions, the tree stocked with the previous h (Q2:
 // BHgrav_stock runs before sph_update) and the previous |a| -- run beside
 // the h solve, and only the kernel-softened pair terms wait for the new h
 // and zeta.  The reference sums the cell terms of the walk first and the
 // near-field pairs of its list afterwards (BHgrav_accel.F90:225-226,
 // 272-290); so does this split, in the same orders.
 //
-// Phase 1: at each cell every active lane applies its own MAC
-// (BHgrav_accel.F90:154-158); accepted cells add a multipole term, opened
-// leaves go to the group's near-field list, opened branches descend.
-template <int OCT, int MACT>
-__global__ void __launch_bounds__(256) k_grav_cells_fp64(
-    int n, int nc, const GNode *__restrict__ gn, const double *__restrict__ x,
-    const double *__restrict__ y, const double *__restrict__ z, const int *__restrict__ cid,
-    const int2 *__restrict__ root_range, const uint8_t *__restrict__ active,
-    const double *__restrict__ gpot, const double *__restrict__ agm, double *__restrict__ cx,
-    double *__restrict__ cy, double *__restrict__ cz, double *__restrict__ cp, NearList near,
-    unsigned long long *__restrict__ icount, unsigned long long *__restrict__ wstat,
-    GroupQueue queue, int *__restrict__ cost, const int2 *__restrict__ grp) {
-    // the walk is the critical path while the SPH kernels run beside it: its
-    // waves take issue priority over theirs on shared SIMDs
-    __builtin_amdgcn_s_setprio(2);
-    unsigned ncell = 0, vis = 0, lvis = 0;   // wave totals
-    const int home = blockIdx.x % NXCD;
-    int qdone = 0;
-    for (int g = next_group(queue, home, qdone); g >= 0; g = next_group(queue, home, qdone)) {
-        const int2 gr = grp[g];
-        const int p = gr.x + (int)(threadIdx.x & (WAVE - 1));
-        const bool valid = p < gr.y && active[p];
-        double rpx = 0, rpy = 0, rpz = 0, afactor = 0.0;
-        if (valid) {
-            rpx = x[p]; rpy = y[p]; rpz = z[p];
-            if (MACT != SERENX_MAC_GEOMETRIC) afactor = mac_afactor<MACT>(agm[p], gpot[p]);
-        }
-        double gx = 0, gy = 0, gz = 0, gp = 0;
-        int len = 0;
-        const int2 rr = valid ? root_range[cid[p]] : make_int2(nc, nc);
-        const unsigned gv = group_walk(
-            gn, nc, valid, rr.x, rr.y, lvis,
-            [&](const GNode &nd, bool here) -> int {
-                const double dr[3] = {rpx - nd.r[0], rpy - nd.r[1], rpz - nd.r[2]};
-                const double drsqd = dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2];
-                bool accept;
-                if (MACT == SERENX_MAC_GEOMETRIC)
-                    accept = drsqd > nd.dminsqd;
-                else
-                    accept = drsqd > nd.mac * afactor && drsqd > nd.dminsqd;
-                accept = accept && nd.leaf != 1;                   // :128-136, no MAC test
-                ncell += lanes(here && accept);
-                if (here && accept) cell_fp64<OCT>(nd, dr, drsqd, gx, gy, gz, gp);
-                if (accept) return WALK_SKIP;
-                return nd.leaf > 0 ? WALK_LEAF : WALK_DESCEND;     // :242-258
-            },
-            [&](const GNode &nd, bool mine) {
-                near_append(near, g, len, nd.first, nd.leaf, ballot(mine));
-            });
-        vis += gv;
-        if ((threadIdx.x & 63) == 0) {
-            cost[g] = (int)gv;
-            near.len[g] = len;
-        }
-        if (valid) {
-            cx[p] = gx;
-            cy[p] = gy;
-            cz[p] = gz;
-            cp[p] = gp;
-        }
-    }
-    if ((threadIdx.x & 63) == 0) atomicAdd(ctr_row(icount) + 0, (unsigned long long)ncell);
-    wave_stats(wstat, 0, vis, lvis);
-}
+// Phase 1 is k_grav_list below.  FP64: each target applies its own MAC
+// (BHgrav_accel.F90:154-158); cells it accepts add a multipole term, leaves it
+// opens go to the group's near-field list, branches it opens descend.
 
 // Phase 2: the pair terms of gravity_gradh.F90 over each particle's opened
 // leaves, in list order, added to the cell sums of phase 1.
 //
-// A wave takes a part of a group, PAIR_TW = 16 targets with four lanes each.
-// The group's list comes 64 leaves at a time, one per lane; 16 ballots turn
-// its lane masks into one word of leaves per target, and each target goes
-// through its own leaves, its four lanes on four of a leaf's particles.  The
-// terms of four sources (f d and m_j / 2 dpot as factor pairs) go through
-// LDS to the target's four lanes, which add them in list order, one lane per
-// component: the same fused additions in the same order as one lane would
-// make, so the sums do not depend on the split.
+// A block takes a group: every wave has all its targets, one per lane, and
+// takes the list's batches of PF_STAGE leaves in turn: lane l copies particle
+// l of the batch's leaves into LDS (the loads of a batch are in flight at
+// once), then the wave goes through the leaves and the lanes that opened one
+// add its terms.  The waves' sums are added in wave order at the end.
 //
-// Why: with one lane per target (one wave per group, the union of its leaves
-// by uniform loads) a quarter of the lanes had opened the leaf at hand, and
-// the chain of record load, square root, reciprocal and table load took
-// half a microsecond per source.  Alone: uniform sphere of 2,048 particles
-// 467 -> 130 us, r^-2 sphere of 4,096 918 -> 361 us; the sums are the same
-// bit for bit.
+// Why: the chain of record load, square root, reciprocal and table load takes
+// half a microsecond per source, so a wave that has a group's list alone takes
+// as long as the longest list (the centre of a uniform sphere, where
+// |a| -> 0, opens 10,000 leaves).  Uniform sphere of 131,071 particles: 10.6 ->
+// 0.9 ms, of 2,048: 128 -> 60 us (four lanes per target, a wave per 16
+// targets); r^-2 sphere of 300,007, which fills the device: 1.7 -> 1.3 ms.
 //
-// A group whose list did not fit repeats its walk for the part's 16 targets
-// (the same MAC decisions: they read the stocked tree and the previous |a|
-// and potential of these targets, which only this wave overwrites, after).
-constexpr int PAIR_LPT = 4;                  // lanes per target
-constexpr int PAIR_TW = WAVE / PAIR_LPT;     // targets of a wave
+// A group whose list was not stored walks again, all its targets in every
+// wave (the same MAC decisions: they read the stocked tree and the previous
+// |a| and potential, which the block overwrites only when all its waves are
+// done), so the batches and the sums are the same.
+constexpr int PF_STAGE = WAVE / LEAFMAX;
+constexpr int PF_WAVES = 8;
+constexpr int PF_TB = PF_WAVES * WAVE;
 
 template <int MACT, bool QUINTIC>
-__device__ __forceinline__ void pairs_part_fp64(
-    int g, int part, int nc, const GNode *__restrict__ gn, const double4 *__restrict__ rec,
-    double2 (*__restrict__ xch)[WAVE + 1], const int *__restrict__ cid,
-    const int2 *__restrict__ root_range, const uint8_t *__restrict__ active,
-    const double4 *__restrict__ t4, double *__restrict__ ax, double *__restrict__ ay,
-    double *__restrict__ az, const double *__restrict__ cp, double *__restrict__ gpot,
-    double *__restrict__ agm, NearList near, const int2 *__restrict__ grp, unsigned &npp,
-    unsigned &nin_p, unsigned &nin_j) {
-    constexpr KGeom kg = walk_geom<QUINTIC>();
-    const int lane = (int)(threadIdx.x & (WAVE - 1)), sub = lane & (PAIR_LPT - 1);
-    const int2 gr = grp[g];
-    const int p = gr.x + part * PAIR_TW + lane / PAIR_LPT;
-    const bool valid = p < gr.y && active[p];
-    if (ballot(valid) == 0) return;
-    double rpx = 0, rpy = 0, rpz = 0, invhp = 1.0, zo_p = 0.0, acc = 0.0;
-    if (valid) {
-        const double4 a = rec[2 * (size_t)p], b = rec[2 * (size_t)p + 1];
-        rpx = a.x; rpy = a.y; rpz = a.z;
-        invhp = b.y;
-        zo_p = b.z;
-        acc = (sub == 0 ? ax : sub == 1 ? ay : sub == 2 ? az : cp)[p];
-    }
-    // 64 entries of the list, one per lane (d: leaf, word: the entries the
-    // lane's target opened)
-    auto chunk = [&](int d, unsigned long long word) {
-        int k0 = 0;   // first particle of the leaf's part at hand
-        // the target's next four sources: particle j of the lane, if any
-        auto next = [&](int &j) -> bool {
-            const int e = word ? __ffsll((long long)word) - 1 : 0;
-            const int de = __shfl(d, e, WAVE);
-            const int cnt = de & 15, i = k0 + sub;
-            const bool act = word != 0 && i < cnt;
-            j = act ? (de >> 4) + i : gr.x;
-            if (word) {
-                k0 += PAIR_LPT;
-                if (k0 >= cnt) {
-                    k0 = 0;
-                    word &= word - 1;
-                }
-            }
-            return act && j != p;
-        };
-        bool more = ballot(word != 0) != 0;
-        int j;
-        bool act = next(j);
-        double4 a = rec[2 * (size_t)j], b = rec[2 * (size_t)j + 1];
-        while (more) {
-            more = ballot(word != 0) != 0;
-            // the next sources' records are in flight while these are used
-            int jn;
-            const bool actn = next(jn);
-            const double4 an = rec[2 * (size_t)jn], bn = rec[2 * (size_t)jn + 1];
-            double dx = 0.0, dy = 0.0, dz = 0.0, f = 0.0, hm = 0.0, dpot = 0.0;
-            unsigned in_ = 0;
-            if (act) {
-                dx = a.x - rpx;
-                dy = a.y - rpy;
-                dz = a.z - rpz;
-                hm = 0.5 * a.w;
-                in_ = pair_terms(kg, t4, invhp, zo_p, dx, dy, dz, a.w, b.w, b.y, b.z, f, dpot);
-            }
-            npp += lanes(act);
-            nin_p += lanes(in_ & 1);
-            nin_j += lanes(in_ & 2);
-            // a lane without a source adds 0 * 0, which leaves the sum (never
-            // -0) as it is
-            xch[0][lane] = make_double2(f, dx);
-            xch[1][lane] = make_double2(f, dy);
-            xch[2][lane] = make_double2(f, dz);
-            xch[3][lane] = make_double2(hm, dpot);
-            wave_lds_fence();
-            double2 t[PAIR_LPT];
-#pragma unroll
-            for (int i = 0; i < PAIR_LPT; i++) t[i] = xch[sub][(lane & ~(PAIR_LPT - 1)) + i];
-            wave_lds_fence();
-#pragma unroll
-            for (int i = 0; i < PAIR_LPT; i++) acc = __fma_rn(t[i].x, t[i].y, acc);
-            a = an;
-            b = bn;
-            act = actn;
-        }
-    };
-    // the words of the lanes' targets from the entries' lane masks: target t
-    // of the part is bit lo + t of a mask
-    auto words = [&](unsigned long long m, int lo) {
-        const unsigned mm = (unsigned)(m >> lo);
-        unsigned long long word = 0;
-#pragma unroll
-        for (int t = 0; t < PAIR_TW; t++) {
-            const unsigned long long b = ballot((mm >> t) & 1u);
-            if (lane / PAIR_LPT == t) word = b;
-        }
-        return valid ? word : 0ull;
-    };
-    const int len = uniform(near.len[g]);
-    if (len <= near.cap) {
-        const size_t at = (size_t)g * near.stride;
-        for (int e0 = 0; e0 < len; e0 += WAVE) {
-            const bool have = e0 + lane < len;
-            const int d = have ? near.leaf[at + e0 + lane] : 0;
-            const unsigned long long m = have ? near.mask[at + e0 + lane] : 0ull;
-            chunk(d, words(m, part * PAIR_TW));
-        }
-    } else {
-        // the part's walk again, target t on lane t
-        const int q = gr.x + part * PAIR_TW + lane;
-        const bool walks = lane < PAIR_TW && q < gr.y && active[q];
-        double qx = 0, qy = 0, qz = 0, afactor = 0.0;
-        int2 rr = make_int2(nc, nc);
-        if (walks) {
-            const double4 a = rec[2 * (size_t)q];
-            qx = a.x; qy = a.y; qz = a.z;
-            if (MACT != SERENX_MAC_GEOMETRIC) afactor = mac_afactor<MACT>(agm[q], gpot[q]);
-            rr = root_range[cid[q]];
-        }
-        int resume = rr.x;
-        int c = uniform(wave_min_int(resume));
-        unsigned lv = 0;
-        while (c < nc) {
-            int cnt = 0, d = 0;
-            unsigned long long m = 0;
-            while (c < nc && cnt < WAVE)
-                group_step(
-                    gn, nc, rr.y, c, resume, lv,
-                    [&](const GNode &nd, bool) -> int {
-                        const double dr[3] = {qx - nd.r[0], qy - nd.r[1], qz - nd.r[2]};
-                        const double drsqd = dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2];
-                        bool accept;
-                        if (MACT == SERENX_MAC_GEOMETRIC)
-                            accept = drsqd > nd.dminsqd;
-                        else
-                            accept = drsqd > nd.mac * afactor && drsqd > nd.dminsqd;
-                        accept = accept && nd.leaf != 1;
-                        if (accept) return WALK_SKIP;
-                        return nd.leaf > 0 ? WALK_LEAF : WALK_DESCEND;
-                    },
-                    [&](const GNode &nd, bool mine) {
-                        const unsigned long long mm = ballot(mine);
-                        if (lane == cnt) {
-                            d = (nd.first << 4) | nd.leaf;
-                            m = mm;
-                        }
-                        cnt++;
-                    });
-            chunk(d, words(m, 0));
-        }
-    }
-    // the gravity acceleration (k_add_grav adds it to a) and the potential
-    const int t0 = lane & ~(PAIR_LPT - 1);
-    const double gx = __shfl(acc, t0, WAVE), gy = __shfl(acc, t0 + 1, WAVE),
-                 gz = __shfl(acc, t0 + 2, WAVE);
-    if (valid) {
-        (sub == 0 ? ax : sub == 1 ? ay : sub == 2 ? az : gpot)[p] = acc;
-        if (MACT != SERENX_MAC_GEOMETRIC && sub == 0) agm[p] = sqrt(gx * gx + gy * gy + gz * gz);
-    }
-}
-
-template <int MACT, bool QUINTIC>
-__global__ void __launch_bounds__(256) k_grav_pairs_fp64(
+__global__ void __launch_bounds__(PF_TB) k_grav_pairs_fp64(
     int nc, const GNode *__restrict__ gn, const double4 *__restrict__ rec,
     const int *__restrict__ cid, const int2 *__restrict__ root_range,
     const uint8_t *__restrict__ active, const double4 *__restrict__ t4,
@@ -574,18 +369,128 @@ __global__ void __launch_bounds__(256) k_grav_pairs_fp64(
     // persistent over the walk's queue: the groups of each XCD range
     // longest-first (by the previous walk's cost), as phase 1 takes them
     __builtin_amdgcn_s_setprio(2);
-    // per wave and component, the lanes' factor pairs; one slot of padding
-    // spreads the components of a target's four lanes over the banks
-    __shared__ double2 xch[256 / WAVE][PAIR_LPT][WAVE + 1];
+    // per wave: the records of a batch; in their place at the end, the sums
+    __shared__ double4 stage_all[PF_WAVES][2 * WAVE];
+    __shared__ int job;
+    constexpr KGeom kg = walk_geom<QUINTIC>();
+    const int lane = (int)(threadIdx.x & (WAVE - 1));
+    const int wave = uniform((int)(threadIdx.x / WAVE));
+    double4 *stage = stage_all[wave];
     unsigned npp = 0, nin_p = 0, nin_j = 0;   // wave totals
     const int home = blockIdx.x % NXCD;
-    int qdone = 0, part = 0;
-    for (int g = next_part<PAIR_LPT>(queue, home, qdone, part); g >= 0;
-         g = next_part<PAIR_LPT>(queue, home, qdone, part))
-        pairs_part_fp64<MACT, QUINTIC>(g, part, nc, gn, rec, xch[threadIdx.x / WAVE], cid,
-                                       root_range, active, t4, ax, ay, az, cp, gpot, agm, near,
-                                       grp, npp, nin_p, nin_j);
-    if ((threadIdx.x & 63) == 0) {
+    int qdone = 0;
+    for (;;) {
+        __syncthreads();
+        if (wave == 0) {
+            const int t = next_group(queue, home, qdone);
+            if (lane == 0) job = t;
+        }
+        __syncthreads();
+        const int g = uniform(job);
+        if (g < 0) break;
+        const int2 gr = grp[g];
+        const int p = gr.x + lane;
+        const bool valid = p < gr.y && active[p];
+        if (ballot(valid) == 0) continue;   // the whole block
+        double rpx = 0, rpy = 0, rpz = 0, invhp = 1.0, zo_p = 0.0;
+        double gx = 0, gy = 0, gz = 0, gp = 0;
+        if (valid) {
+            const double4 a = rec[2 * (size_t)p], b = rec[2 * (size_t)p + 1];
+            rpx = a.x; rpy = a.y; rpz = a.z;
+            invhp = b.y;
+            zo_p = b.z;
+        }
+        // one leaf, its records at a (wave-uniform)
+        auto leaf_pairs = [&](const double4 *src, int first, int count, bool mine) {
+            for (int i = 0; i < count; i++) {
+                const double4 a = src[2 * i], b = src[2 * i + 1];
+                const bool act = mine && first + i != p;
+                unsigned in_ = 0;
+                if (act)
+                    in_ = pair_fp64(kg, t4, invhp, zo_p, a.x - rpx, a.y - rpy, a.z - rpz, a.w,
+                                    b.w, b.y, b.z, gx, gy, gz, gp);
+                npp += lanes(act);
+                nin_p += lanes(in_ & 1);
+                nin_j += lanes(in_ & 2);
+            }
+        };
+        const int len = uniform(near.len[g]);
+        if (len != NEAR_DROPPED) {
+            for (int e0 = wave * PF_STAGE; e0 < len; e0 += PF_WAVES * PF_STAGE) {
+                const int nb = min(PF_STAGE, len - e0);
+                const size_t at = near.slot(g, e0);   // a batch lies in one page
+                const int e = lane / LEAFMAX, i = lane % LEAFMAX;
+                const int dl = e < nb ? near.leaf[at + e] : 0;
+                const unsigned long long ml = e < nb ? near.mask[at + e] : 0ull;
+                if (i < (dl & 15)) {
+                    const size_t j = (size_t)(dl >> 4) + i;
+                    stage[2 * lane] = rec[2 * j];
+                    stage[2 * lane + 1] = rec[2 * j + 1];
+                }
+                wave_lds_fence();
+                for (int k = 0; k < nb; k++) {
+                    const int d = __builtin_amdgcn_readlane(dl, k * LEAFMAX);
+                    const unsigned long long m =
+                        (unsigned)__builtin_amdgcn_readlane((int)ml, k * LEAFMAX) |
+                        (unsigned long long)(unsigned)__builtin_amdgcn_readlane(
+                            (int)(ml >> 32), k * LEAFMAX) << 32;
+                    leaf_pairs(stage + 2 * LEAFMAX * k, d >> 4, d & 15,
+                               __builtin_amdgcn_inverse_ballot_w64(m));
+                }
+                wave_lds_fence();   // every read before the next batch's writes
+            }
+        } else {
+            // the group's walk again; the wave takes its own batches
+            double afactor = 0.0;
+            if (valid && MACT != SERENX_MAC_GEOMETRIC)
+                afactor = mac_afactor<MACT>(agm[p], gpot[p]);
+            const int2 rr = valid ? root_range[cid[p]] : make_int2(nc, nc);
+            unsigned lv = 0;
+            int e = 0;
+            (void)group_walk(
+                gn, nc, valid, rr.x, rr.y, lv,
+                [&](const GNode &nd, bool) -> int {
+                    const double dr[3] = {rpx - nd.r[0], rpy - nd.r[1], rpz - nd.r[2]};
+                    const double drsqd = dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2];
+                    bool accept;
+                    if (MACT == SERENX_MAC_GEOMETRIC)
+                        accept = drsqd > nd.dminsqd;
+                    else
+                        accept = drsqd > nd.mac * afactor && drsqd > nd.dminsqd;
+                    accept = accept && nd.leaf != 1;
+                    if (accept) return WALK_SKIP;
+                    return nd.leaf > 0 ? WALK_LEAF : WALK_DESCEND;
+                },
+                [&](const GNode &nd, bool mine) {
+                    if (e / PF_STAGE % PF_WAVES == wave)
+                        leaf_pairs(rec + 2 * (size_t)nd.first, nd.first, nd.leaf, mine);
+                    e++;
+                });
+        }
+        // every wave is done with its stage and with the previous |a|
+        __syncthreads();
+        double *sums = reinterpret_cast<double *>(stage_all);   // [wave][component][lane]
+        sums[(wave * 4 + 0) * WAVE + lane] = gx;
+        sums[(wave * 4 + 1) * WAVE + lane] = gy;
+        sums[(wave * 4 + 2) * WAVE + lane] = gz;
+        sums[(wave * 4 + 3) * WAVE + lane] = gp;
+        __syncthreads();
+        if (wave == 0 && valid) {
+            gx = ax[p]; gy = ay[p]; gz = az[p]; gp = cp[p];   // the cell sums
+            for (int w = 0; w < PF_WAVES; w++) {
+                gx += sums[(w * 4 + 0) * WAVE + lane];
+                gy += sums[(w * 4 + 1) * WAVE + lane];
+                gz += sums[(w * 4 + 2) * WAVE + lane];
+                gp += sums[(w * 4 + 3) * WAVE + lane];
+            }
+            ax[p] = gx;   // the gravity acceleration; k_add_grav adds it to a
+            ay[p] = gy;
+            az[p] = gz;
+            gpot[p] = gp;
+            if (MACT != SERENX_MAC_GEOMETRIC) agm[p] = sqrt(gx * gx + gy * gy + gz * gz);
+        }
+    }
+    if (lane == 0) {
         unsigned long long *ic = ctr_row(icount);
         atomicAdd(ic + 1, (unsigned long long)npp);
         atomicAdd(ic + 2, (unsigned long long)nin_p);
@@ -666,10 +571,11 @@ __device__ __forceinline__ void pair_f32(const KGeomF &kg, const float4 *__restr
 template <int OCT>
 __device__ __forceinline__ void cell_fp32(const GNodeF &g, const float dr[3], float &ax,
                                           float &ay, float &az, float &pot) {
-#pragma clang fp contract(fast)
-    const float drsqd = dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2];
+#pragma clang fp contract(off)
+    const float drsqd =
+        __builtin_fmaf(dr[2], dr[2], __builtin_fmaf(dr[0], dr[0], dr[1] * dr[1]));
     const float ir = __builtin_amdgcn_rsqf(drsqd + 1.0e-30f);
-    cell_terms_s<OCT, float>(dr[0], dr[1], dr[2], ir, g.m, g.q, g.s, ax, ay, az, pot);
+    cell_terms_s<OCT>(dr[0], dr[1], dr[2], ir, g.m, g.q, g.s, ax, ay, az, pot);
 }
 
 // Cell terms are summed in FP32 over batches of CELL_BATCH cell visits of the
@@ -705,6 +611,691 @@ __device__ __forceinline__ bool group_accepts(const GNodeF &nd, unsigned long lo
     return nd.leaf != 1 && (vmask & ~ok) == 0;       // :128-136; every lane accepts
 }
 
+// ---- the list walk ---------------------------------------------------------
+// Phase 1 of the walk (traversal, cell terms, near lists) by a block of
+// LW_WAVES waves per group, in three steps:
+//  1. the tree is opened level by level, one cell per lane: the lane tests its
+//     cell's MAC against the sphere that holds the group's targets and, where
+//     that does not decide it, against every target (in LDS); it appends an
+//     opened branch's children to the block's list of cells to visit;
+//  2. two bit maps over the cloud's cells (accepted cells, opened leaves) give
+//     every entry its rank in DFS order, so both lists come out in the order
+//     of a walk, whatever order the lanes appended in;
+//  3. each wave forms the terms of its share of the accepted cells, one
+//     target per lane, the nodes through the scalar cache.
+//
+// Why: a wave that walks alone visits a cell in 0.4 to 1 us (scalar load, test,
+// vote and term one after the other), so a launch took as long as its largest
+// walk: 16.6 ms on a uniform sphere of 131,071 particles whose central groups,
+// where |a| -> 0, visit 15,000 cells.  Here 64 tests run at once and the cells
+// to come are known before their terms are formed: 3.8 ms there; 300 -> 62 us
+// on 2,048 particles (FP64, quadrupole), 1,454 -> 385 us on an r^-2 sphere of
+// 16,384 and 5.3 -> 1.1 ms on a uniform one of 65,536 (mixed).  Bound by the
+// vector ALU: on the 1M r^-2 sphere 89 instructions per accepted cell and
+// wave, and 1.1e9 of 8.1e9 in steps 1 and 2 (2.2e9 with every cell tested
+// against every target, without the sphere).
+//
+// Results.  The accepted cells, their order and (mixed) their batches of
+// CELL_BATCH are the serial walk's; the waves' FP64 sums are added in wave
+// order at the end.  A group's sums depend only on its own cloud.
+//
+// A window of the cloud's DFS range is walked at a time: at most LW_BITS
+// cells, halved when the block's LW_CAP entries overflow (cells outside the
+// window are dropped untested, its ancestors are tested and not counted).
+constexpr int LW_TB = LW_WAVES * WAVE;
+
+struct ListWalk {
+    double x[WAVE], y[WAVE], z[WAVE], af[WAVE];   // targets
+    unsigned bits[2][LW_BITS / 32];               // accepted cells, opened leaves
+    int pre[2][LW_BITS / 128];                    // their ranks at every 128th cell
+    unsigned short und[LW_CAP];                   // entries of a level left to all targets
+    double c[3], rad, afmin, afmax;               // sphere of the targets, range of af
+    int job, cnt[3], nund[3], page0;
+    unsigned long long wsum[LW_WAVES];
+};
+// the waves' sums take the place of the accepted cells' bits at the end
+static_assert(sizeof(unsigned) * LW_BITS / 32 >= sizeof(double) * 4 * LW_TB, "sums fit");
+
+// Walks that one wave began and left to the list walk (k_grav_cells_*): their
+// groups, where each goes on, their number and how many have been taken.
+// A null group: the list walk takes every group of the queue from its root.
+struct LongWalks {
+    int *group, *at, *n, *taken;
+    int budget;      // visits of a walk by one wave
+    int alone;       // clouds of at most this many particles are left whole
+};
+
+struct ListScratch {
+    int *ids;                    // BFS ids of the cells to visit, then the outcome bits
+    unsigned long long *in;      // lanes that visit the cell, then those that accept it
+    unsigned long long *open;    // lanes that open it
+    int *list;                   // accepted cells in DFS order
+    unsigned long long *mask;    // the lanes that accept them
+    int cap;
+};
+constexpr int LW_ACC = 1 << 30, LW_LEAF = (int)(1u << 31), LW_ID = LW_ACC - 1;
+
+// MAC tests of one cell against N targets from t0 on; bit k of the result:
+// target t0 + k accepts.  The reference's arithmetic (BHgrav_accel.F90:154-158).
+template <int MACT, int N>
+__device__ __forceinline__ unsigned mac_bits(const ListWalk &L, int t0, const GMac &nd,
+                                             double mac) {
+    unsigned b = 0;
+#pragma unroll 8
+    for (int k = 0; k < N; k++) {
+        const int t = t0 + k;
+        const double dx = L.x[t] - nd.r[0], dy = L.y[t] - nd.r[1], dz = L.z[t] - nd.r[2];
+        const double d2 = dist2_unfused(dx, dy, dz);
+        bool ok = d2 > nd.dminsqd;
+        if (MACT != SERENX_MAC_GEOMETRIC) ok = ok && d2 > mac * L.af[t];
+        b = __builtin_amdgcn_alignbit(ok ? 1u : 0u, b, 1);
+    }
+    return b >> (32 - N);
+}
+
+// number of set bits before a bit
+__device__ __forceinline__ int lw_rank(const ListWalk &L, int which, int bit) {
+    const int w = bit >> 5, g = w >> 2;
+    int r = L.pre[which][g];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const unsigned v = L.bits[which][4 * g + k];
+        if (4 * g + k < w) r += __popc(v);
+        if (4 * g + k == w) r += __popc(v & ((1u << (bit & 31)) - 1u));
+    }
+    return r;
+}
+
+// What one walk of a block counts and needs in every level
+struct LevelState {
+    int ws, we;          // window
+    unsigned nvalid;
+    unsigned vis, lvis, ncell;
+    int hi, slot;        // end of the level's entries, its counter
+};
+
+// The outcome of an entry on the lanes with lead set: am, om are the lanes of
+// the group that accept the cell and that open it (mixed: 1 or 0).  The
+// children of opened branches are appended, with one counter update per wave.
+template <bool MIXED>
+__device__ __forceinline__ void lw_outcome(ListWalk &L, const ListScratch &sc, LevelState &st,
+                                           bool lead, int e, int id, const GMac &nd,
+                                           unsigned long long in, unsigned long long am,
+                                           unsigned long long om) {
+    const int lane = (int)(threadIdx.x & (WAVE - 1));
+    int kids = 0;
+    if (lead) {
+        int f = id;
+        if (nd.c >= st.ws) {
+            st.vis++;
+            st.lvis += MIXED ? st.nvalid : (unsigned)__popcll(in);
+            st.ncell += MIXED ? (am ? st.nvalid : 0u) : (unsigned)__popcll(am);
+            const int bit = nd.c - st.ws;
+            if (am) {
+                f |= LW_ACC;
+                atomicOr(&L.bits[0][bit >> 5], 1u << (bit & 31));
+            }
+            if (om && nd.k > 0) {
+                f |= LW_LEAF;
+                atomicOr(&L.bits[1][bit >> 5], 1u << (bit & 31));
+            }
+        }
+        sc.ids[e] = f;
+        if (!MIXED) {
+            sc.in[e] = am;
+            sc.open[e] = om;
+        }
+        if (om && nd.k < 0) kids = -nd.k;
+    }
+    if (!any_lane(kids != 0)) return;
+    int at = kids;
+#pragma unroll
+    for (int d = 1; d < WAVE; d *= 2) {
+        const int v = __shfl_up(at, d, WAVE);
+        if (lane >= d) at += v;
+    }
+    int base = 0;
+    if (lane == WAVE - 1) base = atomicAdd(&L.cnt[st.slot], at);
+    base = st.hi + __shfl(base, WAVE - 1, WAVE) + at - kids;
+    for (int k = 0; k < kids; k++)
+        if (base + k < sc.cap) {
+            sc.ids[base + k] = nd.fc + k;
+            if (!MIXED) sc.in[base + k] = om;
+        }
+}
+
+// One level's entries from lo on, one per lane, against the targets' sphere.
+// Every target lies within rad of c, so its distance from the cell lies within
+// rad of c's: the cell is accepted by all (opened by all) when that holds
+// with 1e-9 to spare, which is far more than the tests' rounding.  Mixed: a
+// cell that the first or the last target refuses is opened.  The other
+// entries go to L.und.
+template <bool MIXED, int MACT>
+__device__ __forceinline__ void lw_sphere(ListWalk &L, const ListScratch &sc, LevelState &st,
+                                          const GMac *__restrict__ gmac, double macscale, int lo) {
+    const int lane = (int)(threadIdx.x & (WAVE - 1));
+    const double rad = L.rad;
+    for (int e = lo + (int)threadIdx.x; any_lane(e < st.hi); e += LW_TB) {
+        bool has = e < st.hi;
+        GMac nd{};
+        int id = 0;
+        if (has) {
+            id = sc.ids[e];
+            nd = gmac[id];
+        }
+        has = has && nd.c < st.we && nd.next > st.ws;
+        unsigned long long in = 1;
+        if (!MIXED && has) in = sc.in[e];
+        const double mac = nd.mac * macscale;
+        const double dx = L.c[0] - nd.r[0], dy = L.c[1] - nd.r[1], dz = L.c[2] - nd.r[2];
+        const double d2 = dx * dx + dy * dy + dz * dz;
+        double far2 = nd.dminsqd, near2 = nd.dminsqd;   // largest and smallest limit on d^2
+        bool fine = true;
+        if (MACT != SERENX_MAC_GEOMETRIC) {
+            far2 = fmax(far2, mac * L.afmax);
+            near2 = fmax(near2, mac * L.afmin);
+            fine = mac < 1.0e300;
+        }
+        const double sf = (sqrt(far2) + rad) * (1.0 + 1.0e-9);
+        const double sn = (sqrt(near2) - rad) * (1.0 - 1.0e-9);
+        const bool all = fine && d2 > sf * sf;
+        bool none = (fine && sn > 0.0 && d2 < sn * sn) || nd.k == 1;   // :128-136
+        if (MIXED) {
+#pragma unroll
+            for (int t = 0; t < WAVE; t += WAVE - 1) {
+                const double q2 = dist2_unfused(L.x[t] - nd.r[0], L.y[t] - nd.r[1],
+                                                L.z[t] - nd.r[2]);
+                bool ok = q2 > nd.dminsqd;
+                if (MACT != SERENX_MAC_GEOMETRIC) ok = ok && q2 > mac * L.af[t];
+                none = none || !ok;
+            }
+        }
+        const bool und = has && !none && !all;
+        lw_outcome<MIXED>(L, sc, st, has && !und, e, id, nd, in, none ? 0ull : in,
+                          none ? in : 0ull);
+        const unsigned long long um = ballot(und);
+        if (um) {
+            int base = 0;
+            if (lane == 0) base = atomicAdd(&L.nund[st.slot], __popcll(um));
+            base = __shfl(base, 0, WAVE);
+            if (und)
+                L.und[base + __popcll(um & ((1ull << lane) - 1ull))] = (unsigned short)e;
+        }
+    }
+}
+
+// The nu entries of L.und against every target, S lanes per entry
+template <bool MIXED, int MACT, int S>
+__device__ __forceinline__ void lw_targets(ListWalk &L, const ListScratch &sc, LevelState &st,
+                                           const GMac *__restrict__ gmac, double macscale,
+                                           int nu) {
+    const int sub = (int)threadIdx.x % S;
+    for (int u = (int)threadIdx.x / S; any_lane(u < nu); u += LW_TB / S) {
+        const bool has = u < nu;
+        GMac nd{};
+        int id = 0, e = 0;
+        unsigned long long in = 1, acc;
+        if (has) {
+            e = L.und[u];
+            id = sc.ids[e];
+            nd = gmac[id];
+            if (!MIXED) in = sc.in[e];
+        }
+        const double mac = nd.mac * macscale;
+        constexpr int N = WAVE / S;
+        if (S == 1) {
+            acc = (unsigned long long)mac_bits<MACT, 32>(L, 0, nd, mac) |
+                  (unsigned long long)mac_bits<MACT, 32>(L, 32, nd, mac) << 32;
+        } else {
+            acc = (unsigned long long)mac_bits<MACT, (N < 32 ? N : 32)>(L, sub * N, nd, mac)
+                  << (sub * N);
+#pragma unroll
+            for (int d = 1; d < S; d *= 2) acc |= __shfl_xor(acc, d, WAVE);
+        }
+        if (MIXED) acc = acc == ~0ull ? 1 : 0;
+        lw_outcome<MIXED>(L, sc, st, has && sub == 0, e, id, nd, in, in & acc, in & ~acc);
+    }
+}
+
+template <bool MIXED, int OCT, int MACT>
+__global__ void __launch_bounds__(LW_TB) k_grav_list(
+    int nc, const GMac *__restrict__ gmac, double macscale, const GNode *__restrict__ gn,
+    const GNodeF *__restrict__ gnf, const double *__restrict__ x,
+    const double *__restrict__ y, const double *__restrict__ z, const int *__restrict__ cid,
+    const int2 *__restrict__ root_range, const uint8_t *__restrict__ active,
+    const double *__restrict__ gpot, const double *__restrict__ agm, double *__restrict__ cx,
+    double *__restrict__ cy, double *__restrict__ cz, double *__restrict__ cp, NearList near,
+    ListScratch all, unsigned long long *__restrict__ icount,
+    unsigned long long *__restrict__ wstat, GroupQueue queue, int *__restrict__ cost,
+    const int2 *__restrict__ grp, LongWalks lw) {
+    __shared__ ListWalk L;
+    // the walk is the critical path while the SPH kernels run beside it: its
+    // waves take issue priority over theirs on shared SIMDs
+    __builtin_amdgcn_s_setprio(2);
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = uniform(tid / WAVE);
+    ListScratch sc = all;
+    sc.ids += (size_t)blockIdx.x * all.cap;
+    sc.in += (size_t)blockIdx.x * all.cap;
+    sc.open += (size_t)blockIdx.x * all.cap;
+    sc.list += (size_t)blockIdx.x * (all.cap + CELL_BATCH);
+    sc.mask += (size_t)blockIdx.x * (all.cap + CELL_BATCH);
+    LevelState st{};   // counts per thread
+    const int home = blockIdx.x % NXCD;
+    int qdone = 0;
+    for (;;) {
+        __syncthreads();   // the previous group's use of L
+        if (wave == 0) {
+            int g = -1;
+            if (!lw.group) {
+                g = next_group(queue, home, qdone);
+            } else if (lane == 0) {
+                const int t = atomicAdd(lw.taken, 1);
+                if (t < *lw.n) g = lw.group[t];
+            }
+            if (lane == 0) L.job = g;
+        }
+        __syncthreads();
+        const int g = uniform(L.job);
+        if (g < 0) break;
+        const int2 gr = grp[g];
+        const int p = gr.x + lane;
+        const bool valid = p < gr.y && active[p];
+        const unsigned long long vmask = ballot(valid);
+        if (vmask == 0) {
+            if (tid == 0) {
+                cost[g] = 0;
+                near.len[g] = 0;
+            }
+            continue;
+        }
+        const unsigned nvalid = (unsigned)__popcll(vmask);
+        // the other lanes repeat the first valid lane's target: they change
+        // no vote and store nothing
+        const int q = valid ? p : gr.x + __ffsll((long long)vmask) - 1;
+        const double rpx = x[q], rpy = y[q], rpz = z[q];
+        if (wave == 0) {
+            const double af =
+                MACT != SERENX_MAC_GEOMETRIC ? mac_afactor<MACT>(agm[q], gpot[q]) : 0.0;
+            L.x[lane] = rpx;
+            L.y[lane] = rpy;
+            L.z[lane] = rpz;
+            L.af[lane] = af;
+            double lo[4] = {rpx, rpy, rpz, af}, hi[4] = {rpx, rpy, rpz, af};
+#pragma unroll
+            for (int d = 1; d < WAVE; d *= 2)
+#pragma unroll
+                for (int k = 0; k < (MACT != SERENX_MAC_GEOMETRIC ? 4 : 3); k++) {
+                    lo[k] = fmin(lo[k], __shfl_xor(lo[k], d, WAVE));
+                    hi[k] = fmax(hi[k], __shfl_xor(hi[k], d, WAVE));
+                }
+            double r2 = 0.0, slack = 0.0;   // slack: the rounding of the centre
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                const double half = 0.5 * (hi[k] - lo[k]);
+                r2 += half * half;
+                slack += 1.0e-15 * fmax(fabs(lo[k]), fabs(hi[k]));
+                if (lane == 0) L.c[k] = lo[k] + half;
+            }
+            // an infinite or undefined factor decides nothing by the sphere
+            const bool odd = any_lane(!(af < 1.0e300));
+            if (lane == 0) {
+                L.rad = odd ? 1.0e300 : sqrt(r2) * (1.0 + 1.0e-9) + slack;
+                L.afmin = lo[3];
+                L.afmax = hi[3];
+            }
+        }
+        const int root = uniform(cid[q]);   // BFS id of the cloud's root
+        const int2 rr = root_range[root];
+        double gx = 0, gy = 0, gz = 0, gp = 0;   // the wave's share of the terms
+        int len = 0, carry = 0;                  // near list so far; cells left of a batch
+        int npage = 0;                           // pages of the near list
+        bool dropped = false;                    // the near list did not fit
+        int gvis = 0;
+        int ws = rr.x;
+        if (lw.group) {   // the rest of a walk that one wave began
+            ws = uniform(lw.at[g]);
+            len = uniform(near.len[g]);
+            dropped = len == NEAR_DROPPED;
+            if (dropped) len = 0;
+            npage = (len + PL_PAGE - 1) / PL_PAGE;
+            gvis = uniform(cost[g]);
+            if (wave == 0 && valid) {
+                gx = cx[p];
+                gy = cy[p];
+                gz = cz[p];
+                gp = cp[p];
+            }
+        }
+        int we = min(rr.y, ws + LW_BITS);
+        while (ws < rr.y) {
+            const int words = (we - ws + 127) / 128 * 4;
+            for (int i = tid; i < words; i += LW_TB) L.bits[0][i] = L.bits[1][i] = 0u;
+            if (tid == 0) {
+                sc.ids[0] = root;
+                if (!MIXED) sc.in[0] = vmask;
+                for (int k = 0; k < 3; k++) L.cnt[k] = L.nund[k] = 0;
+            }
+            st.ws = ws;
+            st.we = we;
+            st.nvalid = nvalid;
+            __syncthreads();
+            // step 1.  Three counters in turn: one is cleared only after
+            // every wave has read it
+            int lo = 0, hi = 1, slot = 0;
+            const LevelState st0 = st;
+            while (lo < hi && hi <= sc.cap) {
+                st.hi = hi;
+                st.slot = slot;
+                lw_sphere<MIXED, MACT>(L, sc, st, gmac, macscale, lo);
+                __syncthreads();
+                const int nu = uniform(L.nund[slot]);
+                if (nu) {
+                    // the more lanes an entry has, the sooner it is done and
+                    // the more is spent on it besides the tests
+                    if (nu * 8 <= LW_TB)
+                        lw_targets<MIXED, MACT, 8>(L, sc, st, gmac, macscale, nu);
+                    else if (nu * 2 <= LW_TB)
+                        lw_targets<MIXED, MACT, 2>(L, sc, st, gmac, macscale, nu);
+                    else
+                        lw_targets<MIXED, MACT, 1>(L, sc, st, gmac, macscale, nu);
+                    __syncthreads();
+                }
+                lo = hi;
+                hi = hi + uniform(L.cnt[slot]);
+                const int old = slot == 0 ? 2 : slot - 1;
+                if (tid == 0) L.cnt[old] = L.nund[old] = 0;
+                slot = slot == 2 ? 0 : slot + 1;
+            }
+            if (hi > sc.cap) {   // too many entries: a window of half the cells
+                st = st0;
+                we = ws + (we - ws) / 2;
+                __syncthreads();
+                continue;
+            }
+            gvis += hi;
+            // step 2
+            int nacc = 0, nleaf = 0;
+            {
+                unsigned long long run = 0;   // accepted | leaves << 32, of groups of 128 cells
+                for (int k0 = 0; k0 < words / 4; k0 += LW_TB) {
+                    const int k = k0 + tid;
+                    unsigned long long v = 0;
+                    if (k < words / 4) {
+                        int a = 0, b = 0;
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            a += __popc(L.bits[0][4 * k + i]);
+                            b += __popc(L.bits[1][4 * k + i]);
+                        }
+                        v = (unsigned)a | (unsigned long long)(unsigned)b << 32;
+                    }
+                    unsigned long long s = v;
+#pragma unroll
+                    for (int d = 1; d < WAVE; d *= 2) {
+                        const unsigned long long o = __shfl_up(s, d, WAVE);
+                        if (lane >= d) s += o;
+                    }
+                    if (lane == WAVE - 1) L.wsum[wave] = s;
+                    __syncthreads();
+                    unsigned long long before = run, sum = 0;
+#pragma unroll
+                    for (int w = 0; w < LW_WAVES; w++) {
+                        if (w < wave) before += L.wsum[w];
+                        sum += L.wsum[w];
+                    }
+                    if (k < words / 4) {
+                        const unsigned long long ex = before + s - v;
+                        L.pre[0][k] = (int)(unsigned)ex;
+                        L.pre[1][k] = (int)(ex >> 32);
+                    }
+                    run += sum;
+                    __syncthreads();
+                }
+                nacc = uniform((int)(unsigned)run);
+                nleaf = uniform((int)(run >> 32));
+            }
+            // pages for the leaves of this window
+            const int pages = (len + nleaf + PL_PAGE - 1) / PL_PAGE;
+            if (len + nleaf > near.cap) dropped = true;
+            if (!dropped && pages > npage) {
+                if (tid == 0) L.page0 = atomicAdd(near.next, pages - npage);
+                __syncthreads();
+                const int first = uniform(L.page0);
+                if (first + pages - npage > near.npage)
+                    dropped = true;
+                else
+                    for (int i = npage + tid; i < pages; i += LW_TB)
+                        near.page[(size_t)g * PL_PAGES + i] = first + i - npage;
+                npage = pages;
+                __syncthreads();
+            }
+            for (int e = tid; e < hi; e += LW_TB) {
+                const int f = sc.ids[e];
+                if (!(f & (LW_ACC | LW_LEAF))) continue;
+                const GMac &nd = gmac[f & LW_ID];
+                const int bit = nd.c - ws;
+                if (f & LW_ACC) {
+                    const int r = carry + lw_rank(L, 0, bit);
+                    sc.list[r] = nd.c;
+                    if (!MIXED) sc.mask[r] = sc.in[e];
+                }
+                if ((f & LW_LEAF) && !dropped) {
+                    const size_t at = near.slot(g, len + lw_rank(L, 1, bit));
+                    near.leaf[at] = (nd.fc << 4) | nd.k;
+                    near.mask[at] = MIXED ? vmask : sc.open[e];
+                }
+            }
+            len += nleaf;
+            __syncthreads();
+            // step 3: whole batches, the last window's remainder too; each
+            // wave takes a run of them
+            const int have = carry + nacc;
+            const bool last = we >= rr.y;
+            const int nb = last ? (have + CELL_BATCH - 1) / CELL_BATCH : have / CELL_BATCH;
+            const int i0 = (int)((long long)nb * wave / LW_WAVES) * CELL_BATCH;
+            const int i1 = min(have, (int)((long long)nb * (wave + 1) / LW_WAVES) * CELL_BATCH);
+            for (int j0 = i0; j0 < i1; j0 += WAVE) {
+                const int m = min(WAVE, i1 - j0);
+                const int mine = sc.list[j0 + min(lane, m - 1)];
+                unsigned mlo = 0, mhi = 0;
+                if (!MIXED) {
+                    const unsigned long long mm = sc.mask[j0 + min(lane, m - 1)];
+                    mlo = (unsigned)mm;
+                    mhi = (unsigned)(mm >> 32);
+                }
+                if (MIXED) {
+                    for (int b0 = 0; b0 < m; b0 += CELL_BATCH) {
+                        float bx = 0.0f, by = 0.0f, bz = 0.0f, bp = 0.0f;
+                        const int be = min(m, b0 + CELL_BATCH);
+                        for (int i = b0; i < be; i++) {
+                            const GNodeF nd = gnf[__builtin_amdgcn_readlane(mine, i)];
+                            const float dr[3] = {(float)(rpx - nd.r[0]), (float)(rpy - nd.r[1]),
+                                                 (float)(rpz - nd.r[2])};
+                            cell_fp32<OCT>(nd, dr, bx, by, bz, bp);
+                        }
+                        gx += (double)bx; gy += (double)by; gz += (double)bz; gp += (double)bp;
+                    }
+                } else {
+                    for (int i = 0; i < m; i++) {
+                        const GNode nd = gn[__builtin_amdgcn_readlane(mine, i)];
+                        const unsigned long long mm =
+                            (unsigned)__builtin_amdgcn_readlane((int)mlo, i) |
+                            (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)mhi, i)
+                                << 32;
+                        const double dr[3] = {rpx - nd.r[0], rpy - nd.r[1], rpz - nd.r[2]};
+                        const double d2 = dist2_unfused(dr[0], dr[1], dr[2]);
+                        if (__builtin_amdgcn_inverse_ballot_w64(mm)) cell_fp64<OCT>(nd, dr, d2, gx, gy, gz, gp);
+                    }
+                }
+            }
+            // the cells of an unfinished batch come first in the next window
+            carry = have - min(have, nb * CELL_BATCH);
+            int keep = 0;
+            unsigned long long keepm = 0;
+            if (tid < carry) {
+                keep = sc.list[nb * CELL_BATCH + tid];
+                if (!MIXED) keepm = sc.mask[nb * CELL_BATCH + tid];
+            }
+            __syncthreads();
+            if (tid < carry) {
+                sc.list[tid] = keep;
+                if (!MIXED) sc.mask[tid] = keepm;
+            }
+            ws = we;
+            we = min(rr.y, ws + LW_BITS);
+        }
+        // the waves' sums, added in wave order
+        double *sum = reinterpret_cast<double *>(L.bits[0]);   // [component][wave][lane]
+        sum[(0 * LW_WAVES + wave) * WAVE + lane] = gx;
+        sum[(1 * LW_WAVES + wave) * WAVE + lane] = gy;
+        sum[(2 * LW_WAVES + wave) * WAVE + lane] = gz;
+        sum[(3 * LW_WAVES + wave) * WAVE + lane] = gp;
+        __syncthreads();
+        if (wave < 4) {
+            double s = sum[wave * LW_WAVES * WAVE + lane];
+#pragma unroll
+            for (int w = 1; w < LW_WAVES; w++) s += sum[(wave * LW_WAVES + w) * WAVE + lane];
+            if (valid) (wave == 0 ? cx : wave == 1 ? cy : wave == 2 ? cz : cp)[p] = s;
+        }
+        if (tid == 0) {
+            cost[g] = gvis;
+            near.len[g] = dropped ? NEAR_DROPPED : len;
+        }
+    }
+#pragma unroll
+    for (int d = 1; d < WAVE; d *= 2) {
+        st.ncell += __shfl_xor(st.ncell, d, WAVE);
+        st.vis += __shfl_xor(st.vis, d, WAVE);
+        st.lvis += __shfl_xor(st.lvis, d, WAVE);
+    }
+    if (lane == 0) atomicAdd(ctr_row(icount) + 0, (unsigned long long)st.ncell);
+    wave_stats(wstat, 0, st.vis, st.lvis);
+}
+
+// ---- the walk of one wave --------------------------------------------------
+// In a cloud of more than LW_ALONE particles a wave walks for its group alone,
+// up to LW_BUDGET visits; the list walk takes what is left, from the cell where
+// the wave stopped.  With that many groups the waves hide each other's
+// latency, and the walk by one wave issues slightly fewer instructions and
+// leaves the SPH kernels beside it more room: an evaluation of r^-2 spheres
+// takes (waves / list walk, ms) 22.8 / 28.3 at 1M, 12.7 / 13.8 at 524k, 9.7 /
+// 10.9 at 400k (mixed), 10.6 / 11.5 at 300k and 8.4 / 8.6 at 200k (FP64).  Where
+// a few groups walk far, the list walk wins up to 400k and beyond: uniform
+// 18.1 / 14.8 at 524k, 14.8 / 11.2 at 400k (mixed), Plummer 18.7 / 12.7 at 300k
+// (FP64).  The line lies where the two gains balance; the budget keeps the
+// long walks of a large uniform cloud from their waves (1M: 75 -> 30 ms;
+// budgets of 3,000, 8,192 and 16,384 differ by 2 % there, and 3,000 costs the
+// r^-2 sphere 10 %).
+// The near list of the group that a wave walks (wave-uniform): entries found
+// and the page that takes the next ones, -1 once none could be had
+struct NearWriter {
+    int len = 0, page = 0;
+    __device__ __forceinline__ void append(const NearList &L, int g, int first, int count,
+                                           unsigned long long mask) {
+        if (len % PL_PAGE == 0 && page >= 0) {
+            int pg = L.npage;
+            if (len < PL_PAGES * PL_PAGE && (threadIdx.x & 63) == 0) pg = atomicAdd(L.next, 1);
+            page = uniform(pg);
+            if (page >= L.npage)
+                page = -1;
+            else if ((threadIdx.x & 63) == 0)
+                L.page[(size_t)g * PL_PAGES + len / PL_PAGE] = page;
+        }
+        if (page >= 0 && (threadIdx.x & 63) == 0) {
+            const size_t at = (size_t)page * PL_PAGE + len % PL_PAGE;
+            L.leaf[at] = (first << 4) | count;
+            L.mask[at] = mask;
+        }
+        len++;
+    }
+    __device__ __forceinline__ int stored(const NearList &L) const {
+        return page < 0 || len > L.cap ? NEAR_DROPPED : len;
+    }
+};
+
+// visits that one wave may make for its group: none in a small cloud
+__device__ __forceinline__ unsigned walk_budget(const LongWalks &lw, bool valid, int p,
+                                                const int *__restrict__ cid,
+                                                const int *__restrict__ cloud_off) {
+    const unsigned long long vm = ballot(valid);
+    if (vm == 0) return 0;
+    const int k = __builtin_amdgcn_readlane(valid ? cid[p] : 0, __ffsll((long long)vm) - 1);
+    return cloud_off[k + 1] - cloud_off[k] > lw.alone ? (unsigned)lw.budget : 0u;
+}
+
+template <int OCT, int MACT>
+__global__ void __launch_bounds__(256) k_grav_cells_fp64(
+    int n, int nc, const GNode *__restrict__ gn, const double *__restrict__ x,
+    const double *__restrict__ y, const double *__restrict__ z, const int *__restrict__ cid,
+    const int2 *__restrict__ root_range, const uint8_t *__restrict__ active,
+    const double *__restrict__ gpot, const double *__restrict__ agm, double *__restrict__ cx,
+    double *__restrict__ cy, double *__restrict__ cz, double *__restrict__ cp, NearList near,
+    unsigned long long *__restrict__ icount, unsigned long long *__restrict__ wstat,
+    GroupQueue queue, int *__restrict__ cost, const int2 *__restrict__ grp,
+    const int *__restrict__ cloud_off, LongWalks lw) {
+    // the walk is the critical path while the SPH kernels run beside it: its
+    // waves take issue priority over theirs on shared SIMDs
+    __builtin_amdgcn_s_setprio(2);
+    unsigned ncell = 0, vis = 0, lvis = 0;   // wave totals
+    const int home = blockIdx.x % NXCD;
+    int qdone = 0;
+    for (int g = next_group(queue, home, qdone); g >= 0; g = next_group(queue, home, qdone)) {
+        const int2 gr = grp[g];
+        const int p = gr.x + (int)(threadIdx.x & (WAVE - 1));
+        const bool valid = p < gr.y && active[p];
+        double rpx = 0, rpy = 0, rpz = 0, afactor = 0.0;
+        if (valid) {
+            rpx = x[p]; rpy = y[p]; rpz = z[p];
+            if (MACT != SERENX_MAC_GEOMETRIC) afactor = mac_afactor<MACT>(agm[p], gpot[p]);
+        }
+        double gx = 0, gy = 0, gz = 0, gp = 0;
+        NearWriter nw;
+        const int2 rr = valid ? root_range[cid[p]] : make_int2(nc, nc);
+        const unsigned budget = walk_budget(lw, valid, p, cid, cloud_off);
+        unsigned gv = 0;
+        int resume = valid ? rr.x : nc;
+        int c = uniform(wave_min_int(resume));
+        while (c < nc && gv < budget) {
+            gv++;
+            group_step(gn, nc, rr.y, c, resume, lvis,
+            [&](const GNode &nd, bool here) -> int {
+                const double dr[3] = {rpx - nd.r[0], rpy - nd.r[1], rpz - nd.r[2]};
+                const double drsqd = dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2];
+                bool accept;
+                if (MACT == SERENX_MAC_GEOMETRIC)
+                    accept = drsqd > nd.dminsqd;
+                else
+                    accept = drsqd > nd.mac * afactor && drsqd > nd.dminsqd;
+                accept = accept && nd.leaf != 1;                   // :128-136, no MAC test
+                ncell += lanes(here && accept);
+                if (here && accept) cell_fp64<OCT>(nd, dr, drsqd, gx, gy, gz, gp);
+                if (accept) return WALK_SKIP;
+                return nd.leaf > 0 ? WALK_LEAF : WALK_DESCEND;     // :242-258
+            },
+            [&](const GNode &nd, bool mine) {
+                nw.append(near, g, nd.first, nd.leaf, ballot(mine));
+            });
+        }
+        vis += gv;
+        if ((threadIdx.x & 63) == 0) {
+            cost[g] = (int)gv;
+            near.len[g] = nw.stored(near);
+            if (c < nc) {
+                lw.at[g] = c;
+                lw.group[atomicAdd(lw.n, 1)] = g;
+            }
+        }
+        if (valid) {
+            cx[p] = gx;
+            cy[p] = gy;
+            cz[p] = gz;
+            cp[p] = gp;
+        }
+    }
+    if ((threadIdx.x & 63) == 0) atomicAdd(ctr_row(icount) + 0, (unsigned long long)ncell);
+    wave_stats(wstat, 0, vis, lvis);
+}
+
 template <int OCT, int MACT>
 __global__ void __launch_bounds__(256) k_grav_cells_mixed(
     int n, int nc, const GNodeF *__restrict__ gn, const double *__restrict__ x,
@@ -713,7 +1304,8 @@ __global__ void __launch_bounds__(256) k_grav_cells_mixed(
     const double *__restrict__ gpot, const double *__restrict__ agm, double *__restrict__ ox,
     double *__restrict__ oy, double *__restrict__ oz, double *__restrict__ op, NearList near,
     unsigned long long *__restrict__ icount, unsigned long long *__restrict__ wstat,
-    GroupQueue queue, int *__restrict__ cost, const int2 *__restrict__ grp) {
+    GroupQueue queue, int *__restrict__ cost, const int2 *__restrict__ grp,
+    const int *__restrict__ cloud_off, LongWalks lw) {
     __builtin_amdgcn_s_setprio(2);
     unsigned ncell = 0, vis = 0, lvis = 0;   // wave totals
     const int home = blockIdx.x % NXCD;
@@ -729,7 +1321,8 @@ __global__ void __launch_bounds__(256) k_grav_cells_mixed(
         }
         double cx = 0.0, cy = 0.0, cz = 0.0, cp = 0.0;   // cell terms
         float bx = 0.0f, by = 0.0f, bz = 0.0f, bp = 0.0f; // current batch of cell terms
-        int nbatch = 0, len = 0;                          // wave-uniform
+        int nbatch = 0;                                   // wave-uniform
+        NearWriter nw;
         unsigned gv = 0;
         // the walk covers the tree of the group's cloud (groups never straddle
         // clouds); every valid lane takes part at every cell, and the cell
@@ -739,7 +1332,9 @@ __global__ void __launch_bounds__(256) k_grav_cells_mixed(
         const int2 rr = valid ? root_range[cid[p]] : make_int2(nc, nc);
         int c = uniform(wave_min_int(valid ? rr.x : nc));
         const int cend = uniform(wave_max_int(valid ? rr.y : 0));
-        while (c < cend) {
+        const unsigned budget = walk_budget(lw, valid, p, cid, cloud_off);
+        int stop = budget ? cend : c;   // the walk ends here
+        while (c < stop) {
             const GNodeF nd = gn[c];
             gv++;
             lvis += nvalid;
@@ -752,10 +1347,11 @@ __global__ void __launch_bounds__(256) k_grav_cells_mixed(
                     cx += (double)bx; cy += (double)by; cz += (double)bz; cp += (double)bp;
                     bx = by = bz = bp = 0.0f;
                     nbatch = 0;
+                    if (gv >= budget) stop = 0;   // only between batches
                 }
                 c = nd.next;
             } else if (nd.leaf > 0) {
-                near_append(near, g, len, nd.first, nd.leaf, vmask);
+                nw.append(near, g, nd.first, nd.leaf, vmask);
                 c = nd.next;
             } else {
                 c = c + 1;
@@ -765,7 +1361,11 @@ __global__ void __launch_bounds__(256) k_grav_cells_mixed(
         vis += gv;
         if ((threadIdx.x & 63) == 0) {
             cost[g] = (int)gv;
-            near.len[g] = len;
+            near.len[g] = nw.stored(near);
+            if (c < cend) {
+                lw.at[g] = c;
+                lw.group[atomicAdd(lw.n, 1)] = g;
+            }
         }
         if (valid) {
             ox[p] = cx;
@@ -778,13 +1378,21 @@ __global__ void __launch_bounds__(256) k_grav_cells_mixed(
     wave_stats(wstat, 0, vis, lvis);
 }
 
-// leaves of a near list staged in LDS at once by the mixed pair phase
-constexpr int PL_STAGE = 32;
+// The mixed pair phase: a block of PM_WAVES waves takes a group; each wave
+// has all its targets, one per lane, and takes the list's batches of PL_STAGE
+// leaves (staged in LDS) in turn.  The waves' compensated sums are added in
+// wave order at the end, in FP64.  One wave per group left the longest lists
+// (5,000 to 20,000 leaves at the centre of a uniform sphere) to one wave:
+// r^-2 sphere of 16,384 particles 957 -> 163 us, uniform sphere of 1M 27.3 ->
+// 4.6 ms, r^-2 sphere of 1M, which fills the device, 3.1 ms either way.
+constexpr int PL_STAGE = 16;
+constexpr int PM_WAVES = 8;
+constexpr int PM_TB = PM_WAVES * WAVE;
 
 template <int MACT, bool QUINTIC>
 __device__ __forceinline__ void pairs_group_mixed(
-    int g, int n, int nc, const GNodeF *__restrict__ gn, const float4 *__restrict__ rec,
-    float4 *__restrict__ stage,
+    int g, int wave, int n, int nc, const GNodeF *__restrict__ gn, const float4 *__restrict__ rec,
+    float4 *__restrict__ stage, double *__restrict__ sums,
     const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
     const double *__restrict__ h, const double *__restrict__ zeta,
     const int *__restrict__ cid, const int2 *__restrict__ root_range,
@@ -800,7 +1408,7 @@ __device__ __forceinline__ void pairs_group_mixed(
     const int2 gr = grp[g];
     const int p = gr.x + lane;
     const bool valid = p < gr.y && active[p];
-    if (ballot(valid) == 0) return;
+    if (ballot(valid) == 0) return;   // the whole block
     double rpx = 0, rpy = 0, rpz = 0, afactor = 0.0;
     PairTarget tp{1.0f, 1.0f, 0.0f, 0.0f, 0.0f};
     if (valid) {
@@ -869,16 +1477,17 @@ __device__ __forceinline__ void pairs_group_mixed(
         }
     };
     const int len = uniform(near.len[g]);
-    if (len <= near.cap) {
+    if (len != NEAR_DROPPED) {
         // the near list in batches of PL_STAGE leaves: lane l copies the
         // records of the batch's leaf l into the wave's LDS stage (all the
         // batch's loads in flight at once), then the wave forms the pairs
         // leaf by leaf in list order from LDS
-        for (int e0 = 0; e0 < len; e0 += PL_STAGE) {
+        for (int e0 = wave * PL_STAGE; e0 < len; e0 += PM_WAVES * PL_STAGE) {
             const int nb = min(PL_STAGE, len - e0);
+            const size_t at = near.slot(g, e0);   // a batch lies in one page
             int dl = 0;
             if (lane < nb) {
-                dl = near.leaf[(size_t)g * near.stride + e0 + lane];
+                dl = near.leaf[at + lane];
                 const int f = dl >> 4, k = dl & 15;
                 float4 *dst = stage + 2 * LEAFMAX * lane;
                 for (int i = 0; i < k; i++) {
@@ -893,7 +1502,7 @@ __device__ __forceinline__ void pairs_group_mixed(
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             for (int e = 0; e < nb; e++) {
                 const int d = __builtin_amdgcn_readlane(dl, e);
-                const unsigned long long m = near.mask[(size_t)g * near.stride + e0 + e];
+                const unsigned long long m = near.mask[at + e];
                 leaf_pairs_staged(stage + 2 * LEAFMAX * e, d >> 4, d & 15,
                                   valid && ((m >> lane) & 1ull));
             }
@@ -903,7 +1512,9 @@ __device__ __forceinline__ void pairs_group_mixed(
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
     } else {
-        // the list did not fit: the same wave-uniform walk again, pairs only
+        // the list was not stored: the same wave-uniform walk again, pairs of
+        // the wave's batches only
+        int e = 0;
         const int2 rr = valid ? root_range[cid[p]] : make_int2(nc, nc);
         int c = uniform(wave_min_int(valid ? rr.x : nc));
         const int cend = uniform(wave_max_int(valid ? rr.y : 0));
@@ -914,19 +1525,33 @@ __device__ __forceinline__ void pairs_group_mixed(
             if (group_accepts<MACT>(nd, vmask, rpx, rpy, rpz, afactor, d0, d1, d2)) {
                 c = nd.next;
             } else if (nd.leaf > 0) {
-                leaf_pairs(nd.first, nd.leaf, valid);
+                if (e / PL_STAGE % PM_WAVES == wave) leaf_pairs(nd.first, nd.leaf, valid);
+                e++;
                 c = nd.next;
             } else {
                 c = c + 1;
             }
         }
     }
-    if (valid) {
-        const double gx = ax[p] + px.value(), gy = ay[p] + py.value(), gz = az[p] + pz.value();
+    // every wave is done with its stage and with the previous |a|
+    __syncthreads();
+    sums[(wave * 4 + 0) * WAVE + lane] = px.value();
+    sums[(wave * 4 + 1) * WAVE + lane] = py.value();
+    sums[(wave * 4 + 2) * WAVE + lane] = pz.value();
+    sums[(wave * 4 + 3) * WAVE + lane] = pq.value();
+    __syncthreads();
+    if (wave == 0 && valid) {
+        double gx = ax[p], gy = ay[p], gz = az[p], gp = cpot[p];
+        for (int w = 0; w < PM_WAVES; w++) {
+            gx += sums[(w * 4 + 0) * WAVE + lane];
+            gy += sums[(w * 4 + 1) * WAVE + lane];
+            gz += sums[(w * 4 + 2) * WAVE + lane];
+            gp += sums[(w * 4 + 3) * WAVE + lane];
+        }
         ax[p] = gx;   // the gravity acceleration; k_add_grav adds it to a
         ay[p] = gy;
         az[p] = gz;
-        gpot[p] = cpot[p] + pq.value();
+        gpot[p] = gp;
         if (MACT != SERENX_MAC_GEOMETRIC) agm[p] = sqrt(gx * gx + gy * gy + gz * gz);
     }
     npp_out += npp;
@@ -935,7 +1560,7 @@ __device__ __forceinline__ void pairs_group_mixed(
 }
 
 template <int MACT, bool QUINTIC>
-__global__ void __launch_bounds__(256) k_grav_pairs_mixed(
+__global__ void __launch_bounds__(PM_TB) k_grav_pairs_mixed(
     int n, int nc, const GNodeF *__restrict__ gn, const float4 *__restrict__ rec,
     const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
     const double *__restrict__ h, const double *__restrict__ zeta,
@@ -949,16 +1574,30 @@ __global__ void __launch_bounds__(256) k_grav_pairs_mixed(
     // persistent over the walk's queue: the groups of each XCD range
     // longest-first (by the previous walk's cost), as phase 1 takes them
     __builtin_amdgcn_s_setprio(2);
-    // each wave's LDS stage: PL_STAGE leaves of LEAFMAX two-float4 records
-    __shared__ float4 stage_all[(256 / WAVE) * PL_STAGE * LEAFMAX * 2];
-    float4 *stage = stage_all + (threadIdx.x / WAVE) * (PL_STAGE * LEAFMAX * 2);
+    // each wave's LDS stage: PL_STAGE leaves of LEAFMAX two-float4 records;
+    // in its place at the end, the waves' sums
+    __shared__ float4 stage_all[PM_WAVES * PL_STAGE * LEAFMAX * 2];
+    static_assert(sizeof(stage_all) >= sizeof(double) * 4 * PM_TB, "sums fit");
+    __shared__ int job;
+    const int wave = uniform((int)(threadIdx.x / WAVE));
+    float4 *stage = stage_all + wave * (PL_STAGE * LEAFMAX * 2);
     unsigned npp = 0, nin_p = 0, nin_j = 0;   // wave totals
     const int home = blockIdx.x % NXCD;
     int qdone = 0;
-    for (int g = next_group(queue, home, qdone); g >= 0; g = next_group(queue, home, qdone))
-        pairs_group_mixed<MACT, QUINTIC>(g, n, nc, gn, rec, stage, x, y, z, h, zeta, cid,
-                                         root_range, active, t4, ax, ay, az, cpot, gpot, agm,
+    for (;;) {
+        __syncthreads();
+        if (wave == 0) {
+            const int t = next_group(queue, home, qdone);
+            if (threadIdx.x == 0) job = t;
+        }
+        __syncthreads();
+        const int g = uniform(job);
+        if (g < 0) break;
+        pairs_group_mixed<MACT, QUINTIC>(g, wave, n, nc, gn, rec, stage,
+                                         reinterpret_cast<double *>(stage_all), x, y, z, h, zeta,
+                                         cid, root_range, active, t4, ax, ay, az, cpot, gpot, agm,
                                          near, icount, grp, ngrp, npp, nin_p, nin_j);
+    }
     if ((threadIdx.x & 63) == 0) {
         unsigned long long *ic = ctr_row(icount);
         atomicAdd(ic + 1, (unsigned long long)npp);
@@ -1030,7 +1669,7 @@ __global__ void __launch_bounds__(256) k_direct(KGeom kg, int n, int nt,
         if (valid) {
             for (int k = 0; k < lim; k++) {
                 if (base + k == p || base + k < lo || base + k >= hi) continue;
-                pair_fp64(kg, t4, invhp, zo_p, sx[k] - rpx, sy[k] - rpy, sz[k] - rpz, sm[k],
+                (void)pair_fp64(kg, t4, invhp, zo_p, sx[k] - rpx, sy[k] - rpy, sz[k] - rpz, sm[k],
                           sh[k], sih[k], szt[k], gx, gy, gz, gp);
             }
         }
@@ -1060,29 +1699,24 @@ int pair_cap(const Ctx &c) {
     return c.pair_blocks > 0 ? c.pair_blocks : c.walk_queue;
 }
 
-// Blocks of the walk launch: with the work queue, at most cap per CU and as
-// many as the device holds at once (each wave then takes group after
-// group); without it, one wave per group.
+// Blocks of a walk launch that has `groups` groups per block at a time: as many
+// as the device holds at once and at most cap per CU, where the knob counts
+// blocks of TB threads.
 template <class K>
-int walk_blocks(Ctx &c, K kernel, int cap, int parts = 1) {
-    const int per_wave = (c.gq.ngroups * parts + 3) / 4;
-    if (c.walk_queue == 0) return std::max(per_wave, 1);
+int walk_blocks(Ctx &c, K kernel, int cap, int tb, int groups = 1) {
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, TB, 0) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, tb, 0) != hipSuccess ||
         per_cu <= 0)
         per_cu = 1;
-    per_cu = std::min(per_cu, cap);
-    return std::max(1, std::min(per_wave, per_cu * c.ncu));
+    if (c.walk_queue != 0) per_cu = std::min(per_cu, std::max(1, cap * TB / tb));
+    return std::max(1, std::min((c.gq.ngroups + groups - 1) / groups, per_cu * c.ncu));
 }
 
-// The lists share pl_entries slots: each of the ngrp groups gets an equal
-// share, at most PL_CAP.  One cloud has at most n / 64 + 1 groups and gets
-// PL_CAP entries per group; a forest of many small clouds, whose groups walk
-// small trees, gets fewer.
+// near_cap bounds a group's list; its largest value leaves that to the pool
 NearList near_list(Ctx &c) {
-    const size_t share = c.pl_entries / (size_t)std::max(c.ngrp, 1);
-    const int stride = (int)std::min<size_t>(PL_CAP, share);
-    return NearList{c.pl_leaf, c.pl_mask, c.pl_len, std::min(c.near_cap, stride), stride};
+    const int cap = c.near_cap < PL_CAP ? c.near_cap : PL_PAGES * PL_PAGE;
+    return NearList{c.pl_leaf, c.pl_mask, c.pl_page, c.gq.ctr + 2 * NXCD, c.pl_len, cap,
+                    c.pl_npage};
 }
 
 // phase 1 of the walk (traversal and cell terms), persistent over the
@@ -1090,19 +1724,33 @@ NearList near_list(Ctx &c) {
 template <int OCT, int MACT>
 void launch_cells(Ctx &c, hipStream_t s, int cap) {
     GroupQueue q{c.gq.ctr, c.gq.order, c.gq.ngroups};
-    if (c.opt.precision == SERENX_MIXED) {
-        auto k = k_grav_cells_mixed<OCT, MACT>;
-        hipLaunchKernelGGL(k, dim3(walk_blocks(c, k, cap)), dim3(TB), 0, s, c.n, c.nc, c.gnf,
+    const bool mixed = c.opt.precision == SERENX_MIXED;
+    int most = 0;   // particles of the largest cloud
+    for (int i = 0; i < c.ncloud; i++)
+        most = std::max(most, c.cloud_off_h[i + 1] - c.cloud_off_h[i]);
+    const bool waves = most > LW_ALONE;
+    int *cont = c.gq.ctr + 2 * NXCD + 1;
+    const LongWalks lw{waves ? c.lw_group : nullptr, c.lw_at, cont, cont + 1, LW_BUDGET, LW_ALONE};
+    if (waves && mixed) {
+        auto kw = k_grav_cells_mixed<OCT, MACT>;
+        hipLaunchKernelGGL(kw, dim3(walk_blocks(c, kw, cap, TB, TB / WAVE)), dim3(TB), 0, s, c.n, c.nc, c.gnf,
                            c.x, c.y, c.z, c.cid, c.root_range, c.active, c.gpot, c.agm, c.gax,
                            c.gay, c.gaz, c.gpc, near_list(c), c.icount, c.wstat, q, c.gq.cost,
-                           c.grp);
-    } else {
-        auto k = k_grav_cells_fp64<OCT, MACT>;
-        hipLaunchKernelGGL(k, dim3(walk_blocks(c, k, cap)), dim3(TB), 0, s, c.n, c.nc, c.gn,
+                           c.grp, c.cloud_off, lw);
+    } else if (waves) {
+        auto kw = k_grav_cells_fp64<OCT, MACT>;
+        hipLaunchKernelGGL(kw, dim3(walk_blocks(c, kw, cap, TB, TB / WAVE)), dim3(TB), 0, s, c.n, c.nc, c.gn,
                            c.x, c.y, c.z, c.cid, c.root_range, c.active, c.gpot, c.agm, c.gax,
                            c.gay, c.gaz, c.gpc, near_list(c), c.icount, c.wstat, q, c.gq.cost,
-                           c.grp);
+                           c.grp, c.cloud_off, lw);
     }
+    auto k = mixed ? k_grav_list<true, OCT, MACT> : k_grav_list<false, OCT, MACT>;
+    const int nb = std::min(walk_blocks(c, k, cap, LW_TB), c.lw_blocks);
+    const ListScratch sc{c.lw_ids, c.lw_in, c.lw_open, c.lw_list, c.lw_mask, c.lw_cap};
+    hipLaunchKernelGGL(k, dim3(nb), dim3(LW_TB), 0, s, c.nc, c.gmac,
+                       mixed ? mixed_mac_scale(c) : 1.0, c.gn, c.gnf, c.x, c.y, c.z, c.cid,
+                       c.root_range, c.active, c.gpot, c.agm, c.gax, c.gay, c.gaz, c.gpc,
+                       near_list(c), sc, c.icount, c.wstat, q, c.gq.cost, c.grp, lw);
 }
 
 // phase 2 (pair terms), persistent over the same queue order (its second
@@ -1112,15 +1760,15 @@ void launch_pairs(Ctx &c, const double4 *rec, hipStream_t s, int cap) {
     GroupQueue q{c.gq.ctr + NXCD, c.gq.order, c.gq.ngroups};
     if (c.opt.precision == SERENX_MIXED) {
         auto k = k_grav_pairs_mixed<MACT, QUINTIC>;
-        hipLaunchKernelGGL(k, dim3(walk_blocks(c, k, cap)), dim3(TB), 0, s, c.n, c.nc, c.gnf,
-                           reinterpret_cast<const float4 *>(rec), c.x, c.y, c.z, c.h, c.zeta,
-                           c.cid, c.root_range, c.active,
+        hipLaunchKernelGGL(k, dim3(walk_blocks(c, k, cap, PM_TB)), dim3(PM_TB), 0, s, c.n, c.nc,
+                           c.gnf, reinterpret_cast<const float4 *>(rec), c.x, c.y, c.z, c.h,
+                           c.zeta, c.cid, c.root_range, c.active,
                            reinterpret_cast<const float4 *>(c.ktab + KT_G4F_OFF), c.gax, c.gay,
                            c.gaz, c.gpc, c.gpot, c.agm, near_list(c), c.icount, c.grp, c.ngrp, q);
     } else {
         auto k = k_grav_pairs_fp64<MACT, QUINTIC>;
-        hipLaunchKernelGGL(k, dim3(walk_blocks(c, k, cap, PAIR_LPT)), dim3(TB), 0, s, c.nc, c.gn,
-                           rec, c.cid, c.root_range, c.active,
+        hipLaunchKernelGGL(k, dim3(walk_blocks(c, k, cap, PF_TB)), dim3(PF_TB), 0, s, c.nc,
+                           c.gn, rec, c.cid, c.root_range, c.active,
                            reinterpret_cast<const double4 *>(c.ktab + KT_G4_OFF), c.gax, c.gay,
                            c.gaz, c.gpc, c.gpot, c.agm, near_list(c), c.icount, c.grp, q);
     }
@@ -1160,7 +1808,7 @@ int prepare_queue(Ctx &c) {
         SX_TRY(sort_queue(c));
     }
     q.order_ready = false;   // used by this walk
-    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, c.gstream, 2 * NXCD, q.ctr);
+    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, c.gstream, 2 * NXCD + 3, q.ctr);
     SX_HIP(hipGetLastError());
     return SERENX_OK;
 }

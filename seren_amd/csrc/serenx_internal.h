@@ -65,11 +65,24 @@ constexpr int HL_SLOTS = 96;
 // standard SPH: r^2 values of the h_gather band kept per particle for the
 // selection of the pp_gather-th neighbour (more are narrowed by bisection)
 constexpr int BAND_MAX = 64;
-// near-field list entries per group of the gravity walk (a longer list makes
-// the group repeat its walk in the pair phase).  Groups deep in a 1M uniform
-// sphere under the relative MAC at 1e-4 open more than 2048 leaves; 4096
-// entries (48 KB per group, 768 B per particle) hold them.
+// near-field lists of the gravity walk: pages of PL_PAGE entries that the
+// groups take from one pool as they need them, up to PL_PAGES a group (a
+// longer list, or an empty pool, makes the group repeat its walk in the pair
+// phase).  The pool holds PL_CAP entries per group (768 B per particle): a
+// mean group opens about 700 leaves, while a few groups at the centre of a
+// uniform sphere, where |a| -> 0, open 5,000 to 20,000 under the relative MAC.
 constexpr int PL_CAP = 4096;
+constexpr int PL_PAGE = 256;
+constexpr int PL_PAGES = 128;
+// The list walk (grav.hip: k_grav_list): waves of a block, cells of a window
+// (bits of its two maps in LDS) and entries a block visits in one window
+constexpr int LW_WAVES = 8;
+constexpr int LW_BITS = 131072;
+// clouds of more particles are walked by one wave per group, which leaves a
+// walk to the list walk after LW_BUDGET visits (grav.hip has the reasons)
+constexpr int LW_ALONE = 393216;
+constexpr int LW_BUDGET = 8192;
+constexpr int LW_CAP = 8192;
 // leaves a wave of the neighbour walk records for the rows of its particles
 // above pp_limit (a longer list makes such a particle walk the tree alone)
 constexpr int NB_CAP = 512;
@@ -178,6 +191,18 @@ static_assert(offsetof(GNodeF, q) <= 64 && sizeof(GNodeF) == 128, "GNodeF layout
 static_assert(sizeof(HNode) == 64, "HNode layout");
 static_assert(sizeof(BNode) == 64, "BNode layout");
 
+// What the gravity walk's MAC test needs of a cell, in BFS order (a branch's
+// children are consecutive, so the lanes of a wave test a front of cells, one
+// each, with contiguous loads).
+struct __attribute__((aligned(64))) GMac {
+    double r[3];      // centre of mass
+    double dminsqd;
+    double mac;
+    int c, next;      // DFS index of the cell and of the one after its subtree
+    int fc;           // branch: first child (BFS id); leaf: first particle
+    int k;            // > 0: particles of a leaf; < 0: minus the children of a branch
+};
+
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
@@ -232,11 +257,18 @@ struct Ctx {
     double *grec = nullptr;      // gravity source records, 8 doubles per particle
     double *gax = nullptr, *gay = nullptr, *gaz = nullptr;   // gravity acceleration
     double *gpc = nullptr;       // potential of the walk's cell terms (phase 1)
-    // near-field lists of the walk: per group of 64 particles, up to PL_CAP
-    // leaves (first << 4 | count) and the masks of the lanes that opened them
-    int *pl_leaf = nullptr, *pl_len = nullptr;
+    // near-field lists of the walk: per group of 64 particles, the leaves it
+    // opened (first << 4 | count) and the masks of the lanes that opened them,
+    // in pages of the pool, PL_PAGES page numbers per group
+    int *pl_leaf = nullptr, *pl_len = nullptr, *pl_page = nullptr;
     unsigned long long *pl_mask = nullptr;
-    size_t pl_entries = 0;       // slots of pl_leaf and pl_mask
+    int pl_npage = 0;            // pages of the pool
+    // the list walk's scratch: LW_CAP entries (fewer for a small context) for
+    // each of lw_blocks blocks
+    int *lw_ids = nullptr, *lw_list = nullptr;
+    unsigned long long *lw_in = nullptr, *lw_open = nullptr, *lw_mask = nullptr;
+    int *lw_group = nullptr, *lw_at = nullptr;   // walks that waves left to it, by number
+    int lw_blocks = 0, lw_cap = 0;
     // groups of the gravity walk: [start, end) of up to 64 consecutive
     // particles of one cloud (each cloud's groups start at its first
     // particle, so a cloud is grouped the same alone and in a forest)
@@ -290,6 +322,7 @@ struct Ctx {
     GNodeF *gnf = nullptr;
     HNode *hn = nullptr;
     BNode *bn = nullptr;         // hydro nodes by BFS id (h solve and lists by waves)
+    GMac *gmac = nullptr;        // gravity MAC data by BFS id
     int *c_first = nullptr, *c_last = nullptr;   // children of a branch: [first, last) BFS ids
     int nc = 0, ltot = 0;
     int level_off[LMAX + 2] = {0};
@@ -316,7 +349,9 @@ struct Ctx {
     // work queue of the persistent gravity walk (walk.h: GroupQueue)
     struct WalkQueue {
         int ngroups = 0;
-        int *ctr = nullptr;          // 2 NXCD counters (one set per walk phase)
+        int *ctr = nullptr;          // 2 NXCD counters (one set per walk phase), the
+                                     // next free page of the near-list pool, the
+                                     // walks left to the list walk and those taken
         int *cost = nullptr;         // per group: cells its last walk visited
         int *order = nullptr;        // group ids by range, then decreasing cost
         uint64_t *keys = nullptr, *keys2 = nullptr;
@@ -429,10 +464,11 @@ inline size_t walk_max_groups(int n, int pp_gather) {
     return ((size_t)n + WAVE - 1) / WAVE + (size_t)forest_max_clouds(n, pp_gather);
 }
 // near-list slots of a context for n particles: PL_CAP for each group of a
-// single cloud (at most n / 64 + 1 groups), shared by all groups otherwise
+// single cloud (at most n / 64 + 1 groups)
 // waves of a one-thread-per-particle launch over n particles
 inline size_t particle_waves(int n) { return (((size_t)n + 255) / 256) * 4; }
 inline size_t near_list_entries(int n) { return (((size_t)n + WAVE - 1) / WAVE + 1) * PL_CAP; }
+static_assert(PL_CAP % PL_PAGE == 0, "whole pages");
 
 int diag_blocks(int n, int *per_block);
 int diagnostics(Ctx &c, double *partial, double *dout);
@@ -447,6 +483,7 @@ int ensure_tree_buffers(Ctx &c);
 int build_tree(Ctx &c);          // bbox, keys, sort, cells, DFS, permutation
 int stock_tree(Ctx &c);          // BHgrav_stock + BHhydro_stock (fused)
 int refresh_f32_nodes(Ctx &c);   // mixed-precision node copy of the stocked tree
+double mixed_mac_scale(const Ctx &c);   // the mixed walk's factor on the MAC term
 int hguess(Ctx &c);              // BHhydro_hguess
 int update_hmax(Ctx &c);         // BHhydro_update_hmax
 int eval_pow_third(Ctx &c, int n, const double *x, double *y);   // device x**ONETHIRD

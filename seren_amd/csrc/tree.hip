@@ -419,7 +419,8 @@ __device__ __forceinline__ void octupole_shift_exact(double *sc, const double *c
 __global__ void __launch_bounds__(256) k_stock(
     int nc, int base, int cnt, const int *__restrict__ bfs2dfs, GNode *__restrict__ gn,
     double *__restrict__ gs,
-    HNode *__restrict__ hn, BNode *__restrict__ bn, const int *__restrict__ c_first,
+    HNode *__restrict__ hn, BNode *__restrict__ bn, GMac *__restrict__ gmac,
+    const int *__restrict__ c_first,
     const int *__restrict__ c_last, const int *__restrict__ c_parent,
     double *__restrict__ bbmin, double *__restrict__ bbmax,
     double *__restrict__ hmaxs, const double *__restrict__ x, const double *__restrict__ y,
@@ -625,6 +626,14 @@ __global__ void __launch_bounds__(256) k_stock(
     b.fc = leaf > 0 ? first : c_first[base + j];
     b.k = leaf > 0 ? leaf : c_first[base + j] - c_last[base + j];
     b.parent = c_parent[base + j];
+    GMac &w = gmac[base + j];
+    for (int k = 0; k < 3; k++) w.r[k] = gr[k];
+    w.dminsqd = dminsqd;
+    w.mac = macv;
+    w.c = c;
+    w.next = next;
+    w.fc = b.fc;
+    w.k = b.k;
 }
 
 // macscale multiplies the multipole-MAC term for the mixed walk's own
@@ -756,6 +765,7 @@ int ensure_tree_buffers(Ctx &c) {
     SX_TRY(dalloc(&c.gnf, cc));
     SX_TRY(dalloc(&c.hn, cc));
     SX_TRY(dalloc(&c.bn, cc));
+    SX_TRY(dalloc(&c.gmac, cc));
     SX_TRY(dalloc(&c.c_first, cc));
     SX_TRY(dalloc(&c.c_last, cc));
     // temporary storage for sort and scans
@@ -980,7 +990,7 @@ int build_tree(Ctx &c) {
 // turns abserror into the mixed walk's tolerance: the term is proportional to
 // abserror^(-1/3) (GADGET), abserror^(-1/2) (GADGET2) or abserror^(-2/3)
 // (EIGEN).  The geometric MAC has no tolerance to trade.
-static double mixed_mac_scale(const Ctx &c) {
+double mixed_mac_scale(const Ctx &c) {
     const double am = c.mixed_abserror, a0 = c.opt.abserror;
     if (!(am > 0.0) || !(a0 > 0.0) || am == a0) return 1.0;
     const double r = a0 / am;
@@ -1000,7 +1010,7 @@ int stock_tree(Ctx &c) {
         const int cnt = c.level_cnt[L];
         if (cnt == 0) continue;
         hipLaunchKernelGGL(k_stock, dim3(nblk(cnt)), dim3(TB), 0, s, c.nc, c.level_off[L], cnt,
-                           c.bfs2dfs, c.gn, c.gs, c.hn, c.bn, c.c_first, c.c_last,
+                           c.bfs2dfs, c.gn, c.gs, c.hn, c.bn, c.gmac, c.c_first, c.c_last,
                            c.c_parent, c.bbmin, c.bbmax, c.hmaxs, c.x, c.y, c.z, c.m,
                            c.h, oct, c.opt.mac, c.opt.thetamaxsqd, c.opt.abserror, c.daux,
                            c.kg.range);
