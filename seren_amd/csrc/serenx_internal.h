@@ -164,7 +164,7 @@ struct __attribute__((aligned(64))) HNode {
 struct __attribute__((aligned(64))) BNode {
     double r[3];
     double rmax;
-    double hrangemax; // KERNRANGE max(h) over the subtree (k_hmax_bfs)
+    double hrangemax; // KERNRANGE max(h) over the subtree (k_pack_xyzh)
     float half[3];
     int fc;           // branch: first child (BFS id); leaf: first particle
     int k;            // > 0: particles of a leaf; < 0: minus the children of a branch
