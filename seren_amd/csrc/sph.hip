@@ -1243,6 +1243,22 @@ __global__ void k_pack_hydro(int n, const double *__restrict__ x, const double *
 // hydro_gradh.F90:87-297 (AB viscosity, beta := 2 alpha).  ENERGY: the
 // INTERNAL_ENERGY terms, du/dt = sum 0.5 m_j visc W_mean (dv.dr) / |dr|
 // (:258-259) - P div v / (Omega rho) (:326-332)
+//
+// HYD_LPP lanes take a particle, each every HYD_LPP-th neighbour; their sums
+// are added in a fixed tree.  One lane per particle went through its row in a
+// chain of gather, square root and divisions, and the longest row held the
+// launch: 115 -> 35 us at 2,048 particles, 650 -> 90 us on a Plummer sphere of
+// 2,053 (rows of thousands), 569 -> 326 us on an r^-2 sphere of 300,007, where
+// eight gathers of a particle in flight hide the L2 misses that bound it.
+constexpr int HYD_LPP = 8;
+
+// the sum over the lanes of a particle, on each of them
+__device__ __forceinline__ double hyd_sum(double v) {
+#pragma unroll
+    for (int d = 1; d < HYD_LPP; d *= 2) v += __shfl_xor(v, d, WAVE);
+    return v;
+}
+
 template <bool ENERGY>
 __global__ void __launch_bounds__(256) k_hydro(
     KGeom kg, int n, const double4 *__restrict__ rec, const uint8_t *__restrict__ active,
@@ -1251,7 +1267,7 @@ __global__ void __launch_bounds__(256) k_hydro(
     double *__restrict__ ax, double *__restrict__ ay, double *__restrict__ az,
     const double *__restrict__ press, const double *__restrict__ divv,
     const double *__restrict__ omega, double *__restrict__ dudt) {
-    const int p = xcd_block() * blockDim.x + threadIdx.x;
+    const int t = xcd_block() * blockDim.x + threadIdx.x, p = t / HYD_LPP, sub = t % HYD_LPP;
     if (p >= n || !active[p]) return;
     const double *w1 = ktab + T_W1 * KT;
     const double4 *rp = rec + 4 * (size_t)p;
@@ -1265,7 +1281,7 @@ __global__ void __launch_bounds__(256) k_hydro(
     double dudt_diss = 0.0;
     const int nn = pptot[p];
     const int *lst = (nn <= pp_limit) ? pplist + (size_t)p * pp_limit : ovf_list + ovf_off[p];
-    for (int i = 0; i < nn; i++) {
+    for (int i = sub; i < nn; i += HYD_LPP) {
         const double4 *rq = rec + 4 * (size_t)lst[i];
         const double4 q0 = rq[0], q1 = rq[1], q2 = rq[2];
         double wmean = 0.0;
@@ -1314,9 +1330,14 @@ __global__ void __launch_bounds__(256) k_hydro(
             if (ENERGY) dudt_diss = dudt_diss + 0.5 * mpp * visc * wmean * dvdr * invdrmag;
         }
     }
-    ax[p] = ahx + adx;
-    ay[p] = ahy + ady;
-    az[p] = ahz + adz;
+    ahx = hyd_sum(ahx) + hyd_sum(adx);
+    ahy = hyd_sum(ahy) + hyd_sum(ady);
+    ahz = hyd_sum(ahz) + hyd_sum(adz);
+    if (ENERGY) dudt_diss = hyd_sum(dudt_diss);
+    if (sub != 0) return;
+    ax[p] = ahx;
+    ay[p] = ahy;
+    az[p] = ahz;
     if (ENERGY) dudt[p] = (0.0 + dudt_diss) - press[p] * divv[p] / omega[p] / rho_p;
 }
 
@@ -1366,6 +1387,13 @@ __global__ void k_pack_hydro_mixed(int n, const double *__restrict__ x,
 // accelerations are summed in FP32 over the particle's neighbours (tens of
 // terms) and stored in FP64.  ENERGY: du/dt as k_hydro, the P div v term in
 // FP64.
+//
+// HYD_LPP lanes take a particle, each every HYD_LPP-th neighbour.  The factors
+// of eight neighbours' terms then go through LDS to the lanes that add them in
+// list order, one lane per sum (three of the pressure force, three of the
+// viscous one, du/dt), so the FP32 sums are those of one lane; every
+// multiply-add is written out for the same reason.  r^-2 spheres: 120 -> 30 us
+// at 16,384 particles, 1,408 -> 686 us at 1M (10 M record gathers of 64 B).
 template <bool ENERGY>
 __global__ void __launch_bounds__(256) k_hydro_mixed(
     KGeom kg, int n, const HydroRecF *__restrict__ rec, const uint8_t *__restrict__ active,
@@ -1375,70 +1403,106 @@ __global__ void __launch_bounds__(256) k_hydro_mixed(
     const double *__restrict__ press, const double *__restrict__ divv,
     const double *__restrict__ omega, const double *__restrict__ rho,
     double *__restrict__ dudt) {
-#pragma clang fp contract(fast)
-    const int p = xcd_block() * blockDim.x + threadIdx.x;
-    if (p >= n || !active[p]) return;
-    const HydroRecF s = rec[p];
+#pragma clang fp contract(off)
+    static_assert(HYD_LPP == 8, "eight lanes, seven sums");
+    // per wave [f_p, f_pp, f_visc, e, ux, uy, uz, 1/|r|][lane], one column of
+    // padding: the eight lanes of a particle read one lane's entries
+    __shared__ float xch_all[256 / WAVE][8][WAVE + 1];
+    float(*xch)[WAVE + 1] = xch_all[threadIdx.x / WAVE];
+    const int t = xcd_block() * blockDim.x + threadIdx.x, p = t / HYD_LPP, sub = t % HYD_LPP;
+    const int lane = (int)(threadIdx.x & (WAVE - 1));
+    const bool valid = p < n && active[p];
+    if (ballot(valid) == 0) return;
+    HydroRecF s{};
+    int nn = 0;
+    const int *lst = nullptr;
+    if (valid) {
+        s = rec[p];
+        nn = pptot[p];
+        lst = (nn <= pp_limit) ? pplist + (size_t)p * pp_limit : ovf_list + ovf_off[p];
+    }
     const double rpx = s.x, rpy = s.y, rpz = s.z;
-    const float hp = s.h, vpx = s.vx, vpy = s.vy, vpz = s.vz;
-    const float rho_p = s.rho, pfactor_p = s.pf, sound_p = s.sound, invhp = s.invh,
-                hfactor_p = s.hfac;
+    const float hp = s.h;
     const float rangesqd = (float)kg.rangesqd, range = (float)kg.range, half = (float)kg.half;
-    const float beta = 2.0f * alpha;
-    const float lim_p = rangesqd * hp * hp, rng_p = range * hp;
-    float ahx = 0.0f, ahy = 0.0f, ahz = 0.0f, adx = 0.0f, ady = 0.0f, adz = 0.0f;
-    float dudt_diss = 0.0f;
-    const int nn = pptot[p];
-    const int *lst = (nn <= pp_limit) ? pplist + (size_t)p * pp_limit : ovf_list + ovf_off[p];
-    for (int i = 0; i < nn; i++) {
-        const HydroRecF q = rec[lst[i]];
-        const float hpp = q.h, mpp = q.m;
-        float ux = (float)(q.x - rpx), uy = (float)(q.y - rpy), uz = (float)(q.z - rpz);
-        const float dr2 = ux * ux + uy * uy + uz * uz;
-        if (dr2 >= lim_p && dr2 >= rangesqd * hpp * hpp) continue;
-        const float ir = __builtin_amdgcn_rsqf(dr2 + 1.0e-30f);
-        const float drmag = dr2 * ir;
-        const float dvx = q.vx - vpx, dvy = q.vy - vpy, dvz = q.vz - vpz;
-        const float dvdr = dvx * ux + dvy * uy + dvz * uz;
-        ux = ux * ir;
-        uy = uy * ir;
-        uz = uz * ir;
-        float wmean = 0.0f;
-        if (drmag < rng_p) {
-            const float wk = w1[min((int)(half * drmag * invhp), KERNTOT)];
-            wmean = 0.5f * hfactor_p * wk;
-            const float f = mpp * pfactor_p * hfactor_p * wk;
-            ahx = ahx + f * ux;
-            ahy = ahy + f * uy;
-            ahz = ahz + f * uz;
+    const float beta = alpha + alpha;
+    const float lim_p = hp * (hp * rangesqd), rng_p = hp * range;
+    // this lane's sum: its factors' rows
+    const int arow = sub < 3 ? 0 : sub < 6 ? 2 : 3;
+    const int urow = sub < 3 ? 4 + sub : sub < 6 ? 1 + sub : 7;
+    float acc = 0.0f;
+    for (int i0 = 0; any_lane(i0 < nn); i0 += HYD_LPP) {
+        float f1 = 0.0f, f2 = 0.0f, f3 = 0.0f, e = 0.0f, ux = 0.0f, uy = 0.0f, uz = 0.0f,
+              ir = 0.0f;
+        if (i0 + sub < nn) {
+            const HydroRecF q = rec[lst[i0 + sub]];
+            const float hpp = q.h, mpp = q.m;
+            const float ex = (float)(q.x - rpx), ey = (float)(q.y - rpy), ez = (float)(q.z - rpz);
+            const float dr2 = __builtin_fmaf(ez, ez, __builtin_fmaf(ex, ex, ey * ey));
+            if (!(dr2 >= lim_p) || !(dr2 >= hpp * (hpp * rangesqd))) {
+                ir = __builtin_amdgcn_rsqf(dr2 + 1.0e-30f);
+                const float drmag = dr2 * ir;
+                const float dvx = q.vx - s.vx, dvy = q.vy - s.vy, dvz = q.vz - s.vz;
+                const float dvdr = __builtin_fmaf(dvz, ez, __builtin_fmaf(dvx, ex, dvy * ey));
+                ux = ir * ex;
+                uy = ir * ey;
+                uz = ir * ez;
+                float wmean = 0.0f;
+                if (drmag < rng_p) {
+                    const float wk = w1[min((int)(s.invh * (drmag * half)), KERNTOT)];
+                    wmean = (0.5f * s.hfac) * wk;
+                    f1 = (s.hfac * (s.pf * mpp)) * wk;
+                }
+                if (drmag < hpp * range) {
+                    const float wk = w1[min((int)((drmag * half) * q.invh), KERNTOT)];
+                    wmean = __builtin_fmaf(0.5f * q.hfac, wk, wmean);
+                    f2 = ((mpp * q.pf) * q.hfac) * wk;
+                }
+                if (dvdr < 0.0f) {
+                    const float hs = hp + hpp;
+                    const float vsignal = 0.5f * (s.sound + q.sound);
+                    const float den =
+                        __builtin_fmaf(hs, hs * (0.25f * (float)ETA_SQD), drmag * drmag);
+                    const float mu = ((0.5f * hs) * dvdr) * __builtin_amdgcn_rcpf(den);
+                    const float visc =
+                        __builtin_amdgcn_rcpf(0.5f * (s.rho + q.rho)) *
+                        __builtin_fmaf(mu, beta * mu, -((alpha * vsignal) * mu));
+                    f3 = (mpp * visc) * wmean;
+                    if (ENERGY) e = dvdr * (((0.5f * mpp) * visc) * wmean);
+                }
+            }
         }
-        if (drmag < range * hpp) {
-            const float wk = w1[min((int)(half * drmag * q.invh), KERNTOT)];
-            wmean = wmean + 0.5f * q.hfac * wk;
-            const float f = mpp * q.pf * q.hfac * wk;
-            ahx = ahx + f * ux;
-            ahy = ahy + f * uy;
-            ahz = ahz + f * uz;
+        xch[0][lane] = f1;
+        xch[1][lane] = f2;
+        xch[2][lane] = f3;
+        if (ENERGY) xch[3][lane] = e;
+        xch[4][lane] = ux;
+        xch[5][lane] = uy;
+        xch[6][lane] = uz;
+        if (ENERGY) xch[7][lane] = ir;
+        wave_lds_fence();
+        // a neighbour without a term adds 0 u, which leaves the sum (never -0)
+        // as it is
+        const int l0 = lane & ~(HYD_LPP - 1);
+        float fa[HYD_LPP], fb[HYD_LPP], fu[HYD_LPP];
+#pragma unroll
+        for (int k = 0; k < HYD_LPP; k++) {
+            fa[k] = xch[arow][l0 + k];
+            fb[k] = xch[1][l0 + k];
+            fu[k] = xch[urow][l0 + k];
         }
-        if (dvdr < 0.0f) {
-            const float hs = hp + hpp;
-            const float vsignal = 0.5f * (sound_p + q.sound);
-            const float mu = 0.5f * hs * dvdr *
-                             __builtin_amdgcn_rcpf(drmag * drmag + 0.25f * (float)ETA_SQD * hs * hs);
-            const float visc = (-alpha * vsignal * mu + beta * mu * mu) *
-                               __builtin_amdgcn_rcpf(0.5f * (rho_p + q.rho));
-            const float f = mpp * visc * wmean;
-            adx = adx + f * ux;
-            ady = ady + f * uy;
-            adz = adz + f * uz;
-            if (ENERGY) dudt_diss = dudt_diss + 0.5f * mpp * visc * wmean * dvdr * ir;
+        wave_lds_fence();
+#pragma unroll
+        for (int k = 0; k < HYD_LPP; k++) {
+            acc = __builtin_fmaf(fu[k], fa[k], acc);
+            acc = __builtin_fmaf(fu[k], sub < 3 ? fb[k] : 0.0f, acc);
         }
     }
-    ax[p] = (double)(ahx + adx);
-    ay[p] = (double)(ahy + ady);
-    az[p] = (double)(ahz + adz);
-    if (ENERGY)
-        dudt[p] = (0.0 + (double)dudt_diss) - press[p] * divv[p] / omega[p] / rho[p];
+    // the pressure force's lane takes the viscous one's sum; lane 6 has du/dt
+    const float ad = __shfl(acc, lane + 3, WAVE), du = __shfl(acc, lane + 6, WAVE);
+    if (!valid || sub > 2) return;
+    (sub == 0 ? ax : sub == 1 ? ay : az)[p] = (double)(ad + acc);
+    if (ENERGY && sub == 0)
+        dudt[p] = (0.0 + (double)du) - press[p] * divv[p] / omega[p] / rho[p];
 }
 
 // thermal.F90:108-113 (INTERNAL_ENERGY, ideal gas): P = (gamma - 1) rho u,
@@ -1736,6 +1800,7 @@ __global__ void k_pack_hydro_std(int n, const double *__restrict__ x, const doub
 // averaged over h_p and h_pp (wmean) weighs both the pressure term
 // (P_p/rho_p^2 + P_pp/rho_pp^2) and the viscous term.  ENERGY adds du/dt,
 // the same pair terms projected on dv.dr / |dr| (hydro.F90:206-208, :262-264).
+// HYD_LPP lanes per particle, as k_hydro.
 template <bool ENERGY>
 __global__ void __launch_bounds__(256) k_hydro_std(
     KGeom kg, int n, const double4 *__restrict__ rec, const uint8_t *__restrict__ active,
@@ -1743,7 +1808,7 @@ __global__ void __launch_bounds__(256) k_hydro_std(
     const int *__restrict__ ovf_list, int pp_limit, const double *__restrict__ ktab, double alpha,
     double *__restrict__ ax, double *__restrict__ ay, double *__restrict__ az,
     double *__restrict__ dudt_out) {
-    const int p = xcd_block() * blockDim.x + threadIdx.x;
+    const int t = xcd_block() * blockDim.x + threadIdx.x, p = t / HYD_LPP, sub = t % HYD_LPP;
     if (p >= n || !active[p]) return;
     const double *w1 = ktab + T_W1 * KT;
     const double4 *rp = rec + 4 * (size_t)p;
@@ -1755,7 +1820,7 @@ __global__ void __launch_bounds__(256) k_hydro_std(
     double ahx = 0.0, ahy = 0.0, ahz = 0.0, adx = 0.0, ady = 0.0, adz = 0.0, dudt = 0.0;
     const int nn = pptot[p];
     const int *lst = (nn <= pp_limit) ? pplist + (size_t)p * pp_limit : ovf_list + ovf_off[p];
-    for (int i = 0; i < nn; i++) {
+    for (int i = sub; i < nn; i += HYD_LPP) {
         const double4 *rq = rec + 4 * (size_t)lst[i];
         const double4 q0 = rq[0], q1 = rq[1], q2 = rq[2];
         const double hpp = q0.w, mpp = q1.w, rho_pp = q2.x;
@@ -1795,9 +1860,14 @@ __global__ void __launch_bounds__(256) k_hydro_std(
             if (ENERGY) dudt = dudt + 0.5 * mpp * visc * wmean * dvdr * invdrmag;
         }
     }
-    ax[p] = ahx + adx;
-    ay[p] = ahy + ady;
-    az[p] = ahz + adz;
+    ahx = hyd_sum(ahx) + hyd_sum(adx);
+    ahy = hyd_sum(ahy) + hyd_sum(ady);
+    ahz = hyd_sum(ahz) + hyd_sum(adz);
+    if (ENERGY) dudt = hyd_sum(dudt);
+    if (sub != 0) return;
+    ax[p] = ahx;
+    ay[p] = ahy;
+    az[p] = ahz;
     if (ENERGY) dudt_out[p] = dudt;
 }
 
@@ -2022,11 +2092,11 @@ int hydro_forces(Ctx &c) {
         hipLaunchKernelGGL(k_pack_hydro_std, dim3(nblk(c.n)), dim3(TB), 0, c.stream, c.n, c.x,
                            c.y, c.z, c.h, c.vx, c.vy, c.vz, c.m, c.rho, c.press, c.sound, rec);
         if (c.opt.thermal == SERENX_THERMAL_ENERGY_EQN)
-            hipLaunchKernelGGL(k_hydro_std<true>, dim3(nblk(c.n)), dim3(TB), 0, c.stream, c.kg,
+            hipLaunchKernelGGL(k_hydro_std<true>, dim3(nblk((long)c.n * HYD_LPP)), dim3(TB), 0, c.stream, c.kg,
                                c.n, rec, c.active, c.pptot, c.pplist, c.ovf_off, c.ovf_list,
                                c.pp_limit, c.ktab, c.opt.alpha, c.ax, c.ay, c.az, c.dudt);
         else
-            hipLaunchKernelGGL(k_hydro_std<false>, dim3(nblk(c.n)), dim3(TB), 0, c.stream, c.kg,
+            hipLaunchKernelGGL(k_hydro_std<false>, dim3(nblk((long)c.n * HYD_LPP)), dim3(TB), 0, c.stream, c.kg,
                                c.n, rec, c.active, c.pptot, c.pplist, c.ovf_off, c.ovf_list,
                                c.pp_limit, c.ktab, c.opt.alpha, c.ax, c.ay, c.az, c.dudt);
         SX_HIP(hipGetLastError());
@@ -2040,12 +2110,12 @@ int hydro_forces(Ctx &c) {
                            c.y, c.z, c.h, c.vx, c.vy, c.vz, c.m, c.rho, c.omega, c.press, c.sound,
                            rf);
         if (c.opt.thermal == SERENX_THERMAL_ENERGY_EQN)
-            hipLaunchKernelGGL(k_hydro_mixed<true>, dim3(nblk(c.n)), dim3(TB), 0, c.stream, c.kg,
+            hipLaunchKernelGGL(k_hydro_mixed<true>, dim3(nblk((long)c.n * HYD_LPP)), dim3(TB), 0, c.stream, c.kg,
                                c.n, rf, c.active, c.pptot, c.pplist, c.ovf_off, c.ovf_list,
                                c.pp_limit, w1f, (float)c.opt.alpha, c.ax, c.ay, c.az, c.press,
                                c.divv, c.omega, c.rho, c.dudt);
         else
-            hipLaunchKernelGGL(k_hydro_mixed<false>, dim3(nblk(c.n)), dim3(TB), 0, c.stream, c.kg,
+            hipLaunchKernelGGL(k_hydro_mixed<false>, dim3(nblk((long)c.n * HYD_LPP)), dim3(TB), 0, c.stream, c.kg,
                                c.n, rf, c.active, c.pptot, c.pplist, c.ovf_off, c.ovf_list,
                                c.pp_limit, w1f, (float)c.opt.alpha, c.ax, c.ay, c.az, c.press,
                                c.divv, c.omega, c.rho, c.dudt);
@@ -2056,11 +2126,11 @@ int hydro_forces(Ctx &c) {
                        c.h, c.vx, c.vy, c.vz, c.m, c.rho, c.omega, c.press, c.sound, rec);
     SX_HIP(hipGetLastError());
     if (c.opt.thermal == SERENX_THERMAL_ENERGY_EQN)
-        hipLaunchKernelGGL(k_hydro<true>, dim3(nblk(c.n)), dim3(TB), 0, c.stream, c.kg, c.n, rec,
+        hipLaunchKernelGGL(k_hydro<true>, dim3(nblk((long)c.n * HYD_LPP)), dim3(TB), 0, c.stream, c.kg, c.n, rec,
                            c.active, c.pptot, c.pplist, c.ovf_off, c.ovf_list, c.pp_limit, c.ktab,
                            c.opt.alpha, c.ax, c.ay, c.az, c.press, c.divv, c.omega, c.dudt);
     else
-        hipLaunchKernelGGL(k_hydro<false>, dim3(nblk(c.n)), dim3(TB), 0, c.stream, c.kg, c.n, rec,
+        hipLaunchKernelGGL(k_hydro<false>, dim3(nblk((long)c.n * HYD_LPP)), dim3(TB), 0, c.stream, c.kg, c.n, rec,
                            c.active, c.pptot, c.pplist, c.ovf_off, c.ovf_list, c.pp_limit, c.ktab,
                            c.opt.alpha, c.ax, c.ay, c.az, c.press, c.divv, c.omega, c.dudt);
     SX_HIP(hipGetLastError());
