@@ -415,6 +415,9 @@ struct Ctx {
     bool bound = false;
     std::vector<double> hbuf;   // staging for host-state transfers
     std::vector<int> hibuf;
+    char *pin = nullptr;         // pinned transfer buffer (capi.hip), grown as needed
+    size_t pin_bytes = 0, pin_used = 0;
+    hipEvent_t pin_ev[16] = {};  // its slots' copies done (two per worker thread)
 };
 
 // Zeroes nwords 32-bit words at p on stream s with a fill kernel (capi.hip).
