@@ -205,39 +205,58 @@ __device__ __forceinline__ double rsqrt_fp64(double a) {
 // the components of H); S is formed as 2 (r.H) / 3 (Euler's identity for a
 // homogeneous cubic).  q = [xx xy yy zx zy zz]; oc holds H's coefficients on
 // the monomials (xx xy xz yy zz yz), stocked per node.
-template <int OCT, class T>
-__device__ __forceinline__ void cell_terms(T x, T y, T z, T ir, T m, const T *q, const T *oc,
-                                           T &ax, T &ay, T &az, T &pot) {
-#pragma clang fp contract(fast)
-    const T ir2 = ir * ir;
-    const T ir3 = ir2 * ir;
-    const T ir5 = ir3 * ir2;
-    const T ir7 = ir5 * ir2;
-    const T Qx = q[0] * x + q[1] * y + q[3] * z;
-    const T Qy = q[1] * x + q[2] * y + q[4] * z;
-    const T Qz = q[3] * x + q[4] * y + q[5] * z;
-    const T t5 = (x * Qx + y * Qy + z * Qz) * ir5;   // (r.Q.r) / r^5
-    T crad = -(m * ir3) - T(2.5) * t5 * ir2;
-    T phi = m * ir + T(0.5) * t5;
-    T gx = ax + Qx * ir5, gy = ay + Qy * ir5, gz = az + Qz * ir5;
+//
+// The factors of the terms, so that a wave can form them and another add them
+// (add_cell): a += Q ir5 + H ir7 + crad r, phi.  Every multiply-add is written
+// out, as in cell_terms_s.
+struct CellFactors {
+    double Q[3], ir5, H[3], ir7, crad, phi;
+};
+
+template <int OCT>
+__device__ __forceinline__ CellFactors cell_factors(double x, double y, double z, double ir,
+                                                    double m, const double *q,
+                                                    const double *oc) {
+#pragma clang fp contract(off)
+    CellFactors f;
+    const double ir2 = ir * ir;
+    const double ir3 = ir * ir2;
+    f.ir5 = ir2 * ir3;
+    f.ir7 = ir2 * f.ir5;
+    f.Q[0] = __fma_rn(q[3], z, __fma_rn(q[1], y, q[0] * x));
+    f.Q[1] = __fma_rn(q[4], z, __fma_rn(q[2], y, q[1] * x));
+    f.Q[2] = __fma_rn(q[5], z, __fma_rn(q[4], y, q[3] * x));
+    // (r.Q.r) / r^5
+    const double t5 = f.ir5 * __fma_rn(z, f.Q[2], __fma_rn(y, f.Q[1], x * f.Q[0]));
+    f.crad = __fma_rn(ir2, -2.5 * t5, -(m * ir3));
+    f.phi = __fma_rn(m, ir, 0.5 * t5);
+    f.H[0] = f.H[1] = f.H[2] = 0.0;
     if (OCT) {
-        const T xx = x * x, yy = y * y, zz = z * z;
-        const T xy = x * y, xz = x * z, yz = y * z;
-        const T Hx = oc[0] * xx + oc[1] * xy + oc[2] * xz + oc[3] * yy + oc[4] * zz + oc[5] * yz;
-        const T Hy = oc[6] * xx + oc[7] * xy + oc[8] * xz + oc[9] * yy + oc[10] * zz + oc[11] * yz;
-        const T Hz =
-            oc[12] * xx + oc[13] * xy + oc[14] * xz + oc[15] * yy + oc[16] * zz + oc[17] * yz;
-        const T rh = (x * Hx + y * Hy + z * Hz) * ir7;   // (r.H) / r^7
-        crad = crad - T(7.0 / 3.0) * rh * ir2;
-        phi = phi + T(1.0 / 3.0) * rh;
-        gx = gx + Hx * ir7;
-        gy = gy + Hy * ir7;
-        gz = gz + Hz * ir7;
+        const double xx = x * x, yy = y * y, zz = z * z;
+        const double xy = x * y, xz = x * z, yz = y * z;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const double *o = oc + 6 * k;
+            f.H[k] = __fma_rn(
+                o[5], yz,
+                __fma_rn(o[4], zz,
+                         __fma_rn(o[3], yy, __fma_rn(o[2], xz, __fma_rn(o[1], xy, o[0] * xx)))));
+        }
+        // (r.H) / r^7
+        const double rh = f.ir7 * __fma_rn(z, f.H[2], __fma_rn(y, f.H[1], x * f.H[0]));
+        f.crad = __fma_rn(ir2, (-7.0 / 3.0) * rh, f.crad);
+        f.phi = __fma_rn(1.0 / 3.0, rh, f.phi);
     }
-    ax = gx + crad * x;
-    ay = gy + crad * y;
-    az = gz + crad * z;
-    pot = pot + phi;
+    return f;
+}
+
+// one component of the acceleration
+template <int OCT>
+__device__ __forceinline__ double add_cell(double a, double Q, double ir5, double H, double ir7,
+                                           double crad, double x) {
+    a = __fma_rn(ir5, Q, a);
+    if (OCT) a = __fma_rn(ir7, H, a);
+    return __fma_rn(x, crad, a);
 }
 
 // The same terms from the moments themselves (the FP32 walk, whose nodes keep
@@ -298,8 +317,12 @@ __device__ __forceinline__ void cell_terms_s(float x, float y, float z, float ir
 template <int OCT>
 __device__ __forceinline__ void cell_fp64(const GNode &g, const double dr[3], double drsqd,
                                           double &ax, double &ay, double &az, double &pot) {
-    const double ir = rsqrt_fp64(drsqd + SMALL_NUMBER);
-    cell_terms<OCT, double>(dr[0], dr[1], dr[2], ir, g.m, g.q, g.oc, ax, ay, az, pot);
+    const CellFactors f =
+        cell_factors<OCT>(dr[0], dr[1], dr[2], rsqrt_fp64(drsqd + SMALL_NUMBER), g.m, g.q, g.oc);
+    ax = add_cell<OCT>(ax, f.Q[0], f.ir5, f.H[0], f.ir7, f.crad, dr[0]);
+    ay = add_cell<OCT>(ay, f.Q[1], f.ir5, f.H[1], f.ir7, f.crad, dr[1]);
+    az = add_cell<OCT>(az, f.Q[2], f.ir5, f.H[2], f.ir7, f.crad, dr[2]);
+    pot = pot + f.phi;
 }
 
 // Near-field lists: per group, the leaves its walk opened, in DFS order, as
@@ -320,6 +343,12 @@ struct NearList {
     }
 };
 constexpr int NEAR_DROPPED = 0x7FFFFFFF;
+
+// Ordered FP64 sums (clouds of up to LW_ORDERED particles): waves of a block,
+// in the pair phase targets of a wave and lanes of a target
+constexpr int OW_WAVES = 16, OW_TB = OW_WAVES * WAVE;
+constexpr int OW_T = WAVE / OW_WAVES, OW_L = WAVE / OW_T;
+static_assert(OW_L == 2 * LEAFMAX, "two leaves on a target's lanes");
 
 // The walk in two phases, so that the traversal and the cell terms -- which
 // need only the positions, the tree stocked with the previous h (Q2:
@@ -353,24 +382,37 @@ constexpr int NEAR_DROPPED = 0x7FFFFFFF;
 // wave (the same MAC decisions: they read the stocked tree and the previous
 // |a| and potential, which the block overwrites only when all its waves are
 // done), so the batches and the sums are the same.
+//
+// ORDERED: clouds of up to LW_ORDERED particles, whose terms are added in list
+// order (see k_grav_list): a wave has OW_T targets with OW_L lanes each, which
+// take the particles of the target's next two leaves and send their factors
+// through LDS to the lanes that add them: 349 us on an r^-2 sphere of 4,096
+// (153 us with the sums in wave order), bound by the steps of the target with
+// the most leaves; with 16 targets and four lanes each 361 us, with a leaf per
+// wave and the adding left to four waves 456 us.
 constexpr int PF_STAGE = WAVE / LEAFMAX;
 constexpr int PF_WAVES = 8;
 constexpr int PF_TB = PF_WAVES * WAVE;
 
-template <int MACT, bool QUINTIC>
-__global__ void __launch_bounds__(PF_TB) k_grav_pairs_fp64(
+template <int MACT, bool QUINTIC, bool ORDERED>
+__global__ void __launch_bounds__(ORDERED ? OW_TB : PF_TB) k_grav_pairs_fp64(
     int nc, const GNode *__restrict__ gn, const double4 *__restrict__ rec,
     const int *__restrict__ cid, const int2 *__restrict__ root_range,
     const uint8_t *__restrict__ active, const double4 *__restrict__ t4,
     double *__restrict__ ax, double *__restrict__ ay, double *__restrict__ az,
     const double *__restrict__ cp, double *__restrict__ gpot, double *__restrict__ agm,
     NearList near, unsigned long long *__restrict__ icount, const int2 *__restrict__ grp,
-    GroupQueue queue) {
+    const int *__restrict__ cloud_off, GroupQueue queue) {
     // persistent over the walk's queue: the groups of each XCD range
     // longest-first (by the previous walk's cost), as phase 1 takes them
     __builtin_amdgcn_s_setprio(2);
-    // per wave: the records of a batch; in their place at the end, the sums
-    __shared__ double4 stage_all[PF_WAVES][2 * WAVE];
+    // per wave: the records of a batch; in their place at the end, the sums.
+    // Ordered sums: per component, the lanes' factor pairs (one slot of padding)
+    __shared__ union {
+        double4 stage[ORDERED ? 1 : PF_WAVES][2 * WAVE];
+        double2 xch[ORDERED ? OW_WAVES : 1][4][WAVE + 1];
+    } lds;
+    auto &stage_all = lds.stage;
     __shared__ int job;
     constexpr KGeom kg = walk_geom<QUINTIC>();
     const int lane = (int)(threadIdx.x & (WAVE - 1));
@@ -415,7 +457,111 @@ __global__ void __launch_bounds__(PF_TB) k_grav_pairs_fp64(
             }
         };
         const int len = uniform(near.len[g]);
-        if (len != NEAR_DROPPED) {
+        const int root = __builtin_amdgcn_readlane(valid ? cid[p] : 0,
+                                                   __ffsll((long long)ballot(valid)) - 1);
+        if ((cloud_off[root + 1] - cloud_off[root] <= LW_ORDERED) != ORDERED)
+            continue;   // the other launch's group
+        constexpr bool ordered = ORDERED;
+        if (ordered && len == NEAR_DROPPED && valid && wave == 0) {
+            gx = ax[p]; gy = ay[p]; gz = az[p]; gp = cp[p];   // wave 0 walks alone
+        }
+        if (ordered && len != NEAR_DROPPED) {
+            // the wave's targets go through their own leaves, a target's lanes
+            // on the leaf's particles; the factors of the terms go through LDS
+            // to the lane that adds a component (0-2, potential 3, in gx)
+            double2(*xch)[WAVE + 1] = lds.xch[wave];
+            const int sub = lane % OW_L, l0 = lane & ~(OW_L - 1);
+            const int tg = wave * OW_T + lane / OW_L, pt = gr.x + tg;
+            const bool mine = pt < gr.y && active[pt];
+            double qx = 0.0, qy = 0.0, qz = 0.0, ihq = 1.0, zoq = 0.0;
+            if (mine) {
+                const double4 a = rec[2 * (size_t)pt], b = rec[2 * (size_t)pt + 1];
+                qx = a.x; qy = a.y; qz = a.z;
+                ihq = b.y;
+                zoq = b.z;
+                if (sub < 4) gx = (sub == 0 ? ax : sub == 1 ? ay : sub == 2 ? az : cp)[pt];
+            }
+            for (int e0 = 0; e0 < len; e0 += WAVE) {
+                const bool have = e0 + lane < len;
+                const size_t at = near.slot(g, e0) + lane;   // a chunk lies in one page
+                const int d = have ? near.leaf[at] : 0;
+                const unsigned long long m = have ? near.mask[at] : 0ull;
+                // the chunk's leaves that the lane's target opened
+                const unsigned mm = (unsigned)(m >> (wave * OW_T));
+                unsigned long long word = 0;
+#pragma unroll
+                for (int t = 0; t < OW_T; t++) {
+                    const unsigned long long b = ballot((mm >> t) & 1u);
+                    if (lane / OW_L == t) word = b;
+                }
+                if (!mine) word = 0;
+                // the lane's source of the target's next two leaves, if any
+                auto next = [&](int &j) -> bool {
+                    const unsigned long long rest = word & (word - 1);
+                    const unsigned long long own = sub < LEAFMAX ? word : rest;
+                    const int e = own ? __ffsll((long long)own) - 1 : 0;
+                    const int de = __shfl(d, e, WAVE), i = sub % LEAFMAX;
+                    const bool act = own != 0 && i < (de & 15);
+                    j = act ? (de >> 4) + i : gr.x;
+                    word = rest & (rest - 1);
+                    return act && j != pt;
+                };
+                bool more = any_lane(word != 0);
+                int j;
+                bool act = next(j);
+                double4 a = rec[2 * (size_t)j], b = rec[2 * (size_t)j + 1];
+                while (more) {
+                    more = any_lane(word != 0);
+                    // the next sources' records are in flight while these are used
+                    int jn;
+                    const bool actn = next(jn);
+                    const double4 an = rec[2 * (size_t)jn], bn = rec[2 * (size_t)jn + 1];
+                    double dx = 0.0, dy = 0.0, dz = 0.0, f = 0.0, hm = 0.0, dpot = 0.0;
+                    unsigned in_ = 0;
+                    if (act) {
+                        dx = a.x - qx;
+                        dy = a.y - qy;
+                        dz = a.z - qz;
+                        hm = 0.5 * a.w;
+                        in_ = pair_terms(kg, t4, ihq, zoq, dx, dy, dz, a.w, b.w, b.y, b.z, f,
+                                         dpot);
+                    }
+                    npp += lanes(act);
+                    nin_p += lanes(in_ & 1);
+                    nin_j += lanes(in_ & 2);
+                    // a lane without a source adds 0 * 0, which leaves the sum
+                    // (never -0) as it is
+                    xch[0][lane] = make_double2(f, dx);
+                    xch[1][lane] = make_double2(f, dy);
+                    xch[2][lane] = make_double2(f, dz);
+                    xch[3][lane] = make_double2(hm, dpot);
+                    wave_lds_fence();
+                    if (sub < 4) {
+#pragma unroll
+                        for (int i0 = 0; i0 < OW_L; i0 += 4) {
+                            double2 t[4];
+#pragma unroll
+                            for (int i = 0; i < 4; i++) t[i] = xch[sub][l0 + i0 + i];
+#pragma unroll
+                            for (int i = 0; i < 4; i++) gx = __fma_rn(t[i].x, t[i].y, gx);
+                        }
+                    }
+                    wave_lds_fence();
+                    a = an;
+                    b = bn;
+                    act = actn;
+                }
+            }
+            const double sx = __shfl(gx, l0, WAVE), sy = __shfl(gx, l0 + 1, WAVE),
+                         sz = __shfl(gx, l0 + 2, WAVE);
+            __syncthreads();   // every wave is done
+            if (mine && sub < 4) {
+                (sub == 0 ? ax : sub == 1 ? ay : sub == 2 ? az : gpot)[pt] = gx;
+                if (MACT != SERENX_MAC_GEOMETRIC && sub == 0)
+                    agm[pt] = sqrt(sx * sx + sy * sy + sz * sz);
+            }
+            continue;
+        } else if (len != NEAR_DROPPED) {
             for (int e0 = wave * PF_STAGE; e0 < len; e0 += PF_WAVES * PF_STAGE) {
                 const int nb = min(PF_STAGE, len - e0);
                 const size_t at = near.slot(g, e0);   // a batch lies in one page
@@ -462,26 +608,28 @@ __global__ void __launch_bounds__(PF_TB) k_grav_pairs_fp64(
                     return nd.leaf > 0 ? WALK_LEAF : WALK_DESCEND;
                 },
                 [&](const GNode &nd, bool mine) {
-                    if (e / PF_STAGE % PF_WAVES == wave)
+                    if ((ordered ? 0 : e / PF_STAGE % PF_WAVES) == wave)
                         leaf_pairs(rec + 2 * (size_t)nd.first, nd.first, nd.leaf, mine);
                     e++;
                 });
         }
         // every wave is done with its stage and with the previous |a|
         __syncthreads();
-        double *sums = reinterpret_cast<double *>(stage_all);   // [wave][component][lane]
+        double *sums = reinterpret_cast<double *>(&lds);   // [wave][component][lane]
         sums[(wave * 4 + 0) * WAVE + lane] = gx;
         sums[(wave * 4 + 1) * WAVE + lane] = gy;
         sums[(wave * 4 + 2) * WAVE + lane] = gz;
         sums[(wave * 4 + 3) * WAVE + lane] = gp;
         __syncthreads();
         if (wave == 0 && valid) {
-            gx = ax[p]; gy = ay[p]; gz = az[p]; gp = cp[p];   // the cell sums
-            for (int w = 0; w < PF_WAVES; w++) {
-                gx += sums[(w * 4 + 0) * WAVE + lane];
-                gy += sums[(w * 4 + 1) * WAVE + lane];
-                gz += sums[(w * 4 + 2) * WAVE + lane];
-                gp += sums[(w * 4 + 3) * WAVE + lane];
+            if (!ordered) {
+                gx = ax[p]; gy = ay[p]; gz = az[p]; gp = cp[p];   // the cell sums
+                for (int w = 0; w < PF_WAVES; w++) {
+                    gx += sums[(w * 4 + 0) * WAVE + lane];
+                    gy += sums[(w * 4 + 1) * WAVE + lane];
+                    gz += sums[(w * 4 + 2) * WAVE + lane];
+                    gp += sums[(w * 4 + 3) * WAVE + lane];
+                }
             }
             ax[p] = gx;   // the gravity acceleration; k_add_grav adds it to a
             ay[p] = gy;
@@ -535,7 +683,8 @@ __device__ __forceinline__ void pair_f32(const KGeomF &kg, const float4 *__restr
                                          float zi2, float &ax, float &ay, float &az, float &pot,
                                          unsigned &nin_p, unsigned &nin_j) {
 #pragma clang fp contract(fast)
-    const float d2 = dx * dx + dy * dy + dz * dz;
+    // written out: which product the compiler rounds depends on the caller
+    const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dx, dx, dy * dy));
     const float ir = __builtin_amdgcn_rsqf(d2 + 1.0e-30f);
     const float dr = d2 * ir;
     const float ir2 = ir * ir;
@@ -637,25 +786,36 @@ __device__ __forceinline__ bool group_accepts(const GNodeF &nd, unsigned long lo
 //
 // Results.  The accepted cells, their order and (mixed) their batches of
 // CELL_BATCH are the serial walk's; the waves' FP64 sums are added in wave
-// order at the end.  A group's sums depend only on its own cloud.
+// order at the end.  A group's sums depend only on its own cloud.  In clouds of
+// up to LW_ORDERED particles the terms themselves are added in the walk's
+// order, so their results are those of a walk by one wave bit for bit: small
+// clouds are the ones followed over many steps, and a collapsing core of 4,096
+// particles makes 1e-8 of a last bit in 60 steps.  Mixed: the sums of a batch
+// go through LDS to four waves, one component each.  FP64: a launch of its own
+// with 16 waves a block; a round of 16 cells' factors (6.6 KB a cell) goes
+// through LDS to four waves that add them: 311 us on an r^-2 sphere of 4,096
+// particles, 188 us with the sums in wave order, 849 us by one wave.
 //
 // A window of the cloud's DFS range is walked at a time: at most LW_BITS
 // cells, halved when the block's LW_CAP entries overflow (cells outside the
 // window are dropped untested, its ancestors are tested and not counted).
 constexpr int LW_TB = LW_WAVES * WAVE;
 
+template <int NW>
 struct ListWalk {
+    // cells of a window (a block of ordered sums, whose factors need the room,
+    // walks small clouds)
+    static constexpr int CELLS = NW == LW_WAVES ? LW_BITS : LW_BITS / 4;
     double x[WAVE], y[WAVE], z[WAVE], af[WAVE];   // targets
-    unsigned bits[2][LW_BITS / 32];               // accepted cells, opened leaves
-    int pre[2][LW_BITS / 128];                    // their ranks at every 128th cell
+    unsigned bits[2][CELLS / 32];                 // accepted cells, opened leaves
+    int pre[2][CELLS / 128];                    // their ranks at every 128th cell
     unsigned short und[LW_CAP];                   // entries of a level left to all targets
     double c[3], rad, afmin, afmax;               // sphere of the targets, range of af
     int job, cnt[3], nund[3], page0;
-    unsigned long long wsum[LW_WAVES];
+    unsigned long long wsum[NW];
 };
 // the waves' sums take the place of the accepted cells' bits at the end
 static_assert(sizeof(unsigned) * LW_BITS / 32 >= sizeof(double) * 4 * LW_TB, "sums fit");
-
 // Walks that one wave began and left to the list walk (k_grav_cells_*): their
 // groups, where each goes on, their number and how many have been taken.
 // A null group: the list walk takes every group of the queue from its root.
@@ -677,8 +837,8 @@ constexpr int LW_ACC = 1 << 30, LW_LEAF = (int)(1u << 31), LW_ID = LW_ACC - 1;
 
 // MAC tests of one cell against N targets from t0 on; bit k of the result:
 // target t0 + k accepts.  The reference's arithmetic (BHgrav_accel.F90:154-158).
-template <int MACT, int N>
-__device__ __forceinline__ unsigned mac_bits(const ListWalk &L, int t0, const GMac &nd,
+template <int MACT, int N, int NW>
+__device__ __forceinline__ unsigned mac_bits(const ListWalk<NW> &L, int t0, const GMac &nd,
                                              double mac) {
     unsigned b = 0;
 #pragma unroll 8
@@ -694,7 +854,8 @@ __device__ __forceinline__ unsigned mac_bits(const ListWalk &L, int t0, const GM
 }
 
 // number of set bits before a bit
-__device__ __forceinline__ int lw_rank(const ListWalk &L, int which, int bit) {
+template <int NW>
+__device__ __forceinline__ int lw_rank(const ListWalk<NW> &L, int which, int bit) {
     const int w = bit >> 5, g = w >> 2;
     int r = L.pre[which][g];
 #pragma unroll
@@ -717,8 +878,8 @@ struct LevelState {
 // The outcome of an entry on the lanes with lead set: am, om are the lanes of
 // the group that accept the cell and that open it (mixed: 1 or 0).  The
 // children of opened branches are appended, with one counter update per wave.
-template <bool MIXED>
-__device__ __forceinline__ void lw_outcome(ListWalk &L, const ListScratch &sc, LevelState &st,
+template <bool MIXED, int NW>
+__device__ __forceinline__ void lw_outcome(ListWalk<NW> &L, const ListScratch &sc, LevelState &st,
                                            bool lead, int e, int id, const GMac &nd,
                                            unsigned long long in, unsigned long long am,
                                            unsigned long long om) {
@@ -770,12 +931,12 @@ __device__ __forceinline__ void lw_outcome(ListWalk &L, const ListScratch &sc, L
 // with 1e-9 to spare, which is far more than the tests' rounding.  Mixed: a
 // cell that the first or the last target refuses is opened.  The other
 // entries go to L.und.
-template <bool MIXED, int MACT>
-__device__ __forceinline__ void lw_sphere(ListWalk &L, const ListScratch &sc, LevelState &st,
+template <bool MIXED, int MACT, int NW>
+__device__ __forceinline__ void lw_sphere(ListWalk<NW> &L, const ListScratch &sc, LevelState &st,
                                           const GMac *__restrict__ gmac, double macscale, int lo) {
     const int lane = (int)(threadIdx.x & (WAVE - 1));
     const double rad = L.rad;
-    for (int e = lo + (int)threadIdx.x; any_lane(e < st.hi); e += LW_TB) {
+    for (int e = lo + (int)threadIdx.x; any_lane(e < st.hi); e += NW * WAVE) {
         bool has = e < st.hi;
         GMac nd{};
         int id = 0;
@@ -825,12 +986,12 @@ __device__ __forceinline__ void lw_sphere(ListWalk &L, const ListScratch &sc, Le
 }
 
 // The nu entries of L.und against every target, S lanes per entry
-template <bool MIXED, int MACT, int S>
-__device__ __forceinline__ void lw_targets(ListWalk &L, const ListScratch &sc, LevelState &st,
+template <bool MIXED, int MACT, int S, int NW>
+__device__ __forceinline__ void lw_targets(ListWalk<NW> &L, const ListScratch &sc, LevelState &st,
                                            const GMac *__restrict__ gmac, double macscale,
                                            int nu) {
     const int sub = (int)threadIdx.x % S;
-    for (int u = (int)threadIdx.x / S; any_lane(u < nu); u += LW_TB / S) {
+    for (int u = (int)threadIdx.x / S; any_lane(u < nu); u += NW * WAVE / S) {
         const bool has = u < nu;
         GMac nd{};
         int id = 0, e = 0;
@@ -857,8 +1018,10 @@ __device__ __forceinline__ void lw_targets(ListWalk &L, const ListScratch &sc, L
     }
 }
 
-template <bool MIXED, int OCT, int MACT>
-__global__ void __launch_bounds__(LW_TB) k_grav_list(
+// (four waves per SIMD: two blocks of a CU hide each other's barriers)
+template <bool MIXED, bool ORDERED, int OCT, int MACT>
+__global__ void __launch_bounds__(ORDERED ? OW_TB : LW_TB)
+__attribute__((amdgpu_waves_per_eu(4))) k_grav_list(
     int nc, const GMac *__restrict__ gmac, double macscale, const GNode *__restrict__ gn,
     const GNodeF *__restrict__ gnf, const double *__restrict__ x,
     const double *__restrict__ y, const double *__restrict__ z, const int *__restrict__ cid,
@@ -867,8 +1030,11 @@ __global__ void __launch_bounds__(LW_TB) k_grav_list(
     double *__restrict__ cy, double *__restrict__ cz, double *__restrict__ cp, NearList near,
     ListScratch all, unsigned long long *__restrict__ icount,
     unsigned long long *__restrict__ wstat, GroupQueue queue, int *__restrict__ cost,
-    const int2 *__restrict__ grp, LongWalks lw) {
-    __shared__ ListWalk L;
+    const int2 *__restrict__ grp, const int *__restrict__ cloud_off, LongWalks lw) {
+    constexpr int NW = ORDERED ? OW_WAVES : LW_WAVES, NT = NW * WAVE;
+    __shared__ ListWalk<NW> L;
+    // a round's factors [wave][dx, Q, H, ir5, ir7, crad, phi][lane]
+    __shared__ double xc[ORDERED ? NW : 1][13][ORDERED ? WAVE : 1];
     // the walk is the critical path while the SPH kernels run beside it: its
     // waves take issue priority over theirs on shared SIMDs
     __builtin_amdgcn_s_setprio(2);
@@ -951,6 +1117,8 @@ __global__ void __launch_bounds__(LW_TB) k_grav_list(
         int npage = 0;                           // pages of the near list
         bool dropped = false;                    // the near list did not fit
         int gvis = 0;
+        const bool ordered = cloud_off[root + 1] - cloud_off[root] <= LW_ORDERED;
+        if (!MIXED && ordered != ORDERED) continue;   // the other launch's group
         int ws = rr.x;
         if (lw.group) {   // the rest of a walk that one wave began
             ws = uniform(lw.at[g]);
@@ -959,17 +1127,17 @@ __global__ void __launch_bounds__(LW_TB) k_grav_list(
             if (dropped) len = 0;
             npage = (len + PL_PAGE - 1) / PL_PAGE;
             gvis = uniform(cost[g]);
-            if (wave == 0 && valid) {
+            if (wave == 0 && valid && !ordered) {   // (ordered walks begin here)
                 gx = cx[p];
                 gy = cy[p];
                 gz = cz[p];
                 gp = cp[p];
             }
         }
-        int we = min(rr.y, ws + LW_BITS);
+        int we = min(rr.y, ws + L.CELLS);
         while (ws < rr.y) {
             const int words = (we - ws + 127) / 128 * 4;
-            for (int i = tid; i < words; i += LW_TB) L.bits[0][i] = L.bits[1][i] = 0u;
+            for (int i = tid; i < words; i += NT) L.bits[0][i] = L.bits[1][i] = 0u;
             if (tid == 0) {
                 sc.ids[0] = root;
                 if (!MIXED) sc.in[0] = vmask;
@@ -992,9 +1160,9 @@ __global__ void __launch_bounds__(LW_TB) k_grav_list(
                 if (nu) {
                     // the more lanes an entry has, the sooner it is done and
                     // the more is spent on it besides the tests
-                    if (nu * 8 <= LW_TB)
+                    if (nu * 8 <= NT)
                         lw_targets<MIXED, MACT, 8>(L, sc, st, gmac, macscale, nu);
-                    else if (nu * 2 <= LW_TB)
+                    else if (nu * 2 <= NT)
                         lw_targets<MIXED, MACT, 2>(L, sc, st, gmac, macscale, nu);
                     else
                         lw_targets<MIXED, MACT, 1>(L, sc, st, gmac, macscale, nu);
@@ -1017,7 +1185,7 @@ __global__ void __launch_bounds__(LW_TB) k_grav_list(
             int nacc = 0, nleaf = 0;
             {
                 unsigned long long run = 0;   // accepted | leaves << 32, of groups of 128 cells
-                for (int k0 = 0; k0 < words / 4; k0 += LW_TB) {
+                for (int k0 = 0; k0 < words / 4; k0 += NT) {
                     const int k = k0 + tid;
                     unsigned long long v = 0;
                     if (k < words / 4) {
@@ -1039,7 +1207,7 @@ __global__ void __launch_bounds__(LW_TB) k_grav_list(
                     __syncthreads();
                     unsigned long long before = run, sum = 0;
 #pragma unroll
-                    for (int w = 0; w < LW_WAVES; w++) {
+                    for (int w = 0; w < NW; w++) {
                         if (w < wave) before += L.wsum[w];
                         sum += L.wsum[w];
                     }
@@ -1064,12 +1232,12 @@ __global__ void __launch_bounds__(LW_TB) k_grav_list(
                 if (first + pages - npage > near.npage)
                     dropped = true;
                 else
-                    for (int i = npage + tid; i < pages; i += LW_TB)
+                    for (int i = npage + tid; i < pages; i += NT)
                         near.page[(size_t)g * PL_PAGES + i] = first + i - npage;
                 npage = pages;
                 __syncthreads();
             }
-            for (int e = tid; e < hi; e += LW_TB) {
+            for (int e = tid; e < hi; e += NT) {
                 const int f = sc.ids[e];
                 if (!(f & (LW_ACC | LW_LEAF))) continue;
                 const GMac &nd = gmac[f & LW_ID];
@@ -1092,9 +1260,85 @@ __global__ void __launch_bounds__(LW_TB) k_grav_list(
             const int have = carry + nacc;
             const bool last = we >= rr.y;
             const int nb = last ? (have + CELL_BATCH - 1) / CELL_BATCH : have / CELL_BATCH;
-            const int i0 = (int)((long long)nb * wave / LW_WAVES) * CELL_BATCH;
-            const int i1 = min(have, (int)((long long)nb * (wave + 1) / LW_WAVES) * CELL_BATCH);
-            for (int j0 = i0; j0 < i1; j0 += WAVE) {
+            const int i0 = (int)((long long)nb * wave / NW) * CELL_BATCH;
+            const int i1 = min(have, (int)((long long)nb * (wave + 1) / NW) * CELL_BATCH);
+            if (ordered) {
+                const int n1 = min(have, nb * CELL_BATCH);
+                float(*xb)[4][WAVE] = reinterpret_cast<float(*)[4][WAVE]>(L.bits);
+                for (int j0 = 0; j0 < n1; j0 += WAVE) {
+                    const int m = min(WAVE, n1 - j0);
+                    const int mine = sc.list[j0 + min(lane, m - 1)];
+                    if (MIXED) {
+                        // wave w < 3 has component w of the acceleration, wave 3
+                        // the potential (in gx); WAVE entries are at most LW_WAVES
+                        // batches
+                        static_assert(WAVE == CELL_BATCH * LW_WAVES, "a batch a wave");
+                        float bx = 0.0f, by = 0.0f, bz = 0.0f, bp = 0.0f;
+                        const int b0 = wave * CELL_BATCH;
+                        for (int i = b0; i < min(m, b0 + CELL_BATCH); i++) {
+                            const GNodeF nd = gnf[__builtin_amdgcn_readlane(mine, i)];
+                            const float dr[3] = {(float)(rpx - nd.r[0]), (float)(rpy - nd.r[1]),
+                                                 (float)(rpz - nd.r[2])};
+                            cell_fp32<OCT>(nd, dr, bx, by, bz, bp);
+                        }
+                        xb[wave][0][lane] = bx;
+                        xb[wave][1][lane] = by;
+                        xb[wave][2][lane] = bz;
+                        xb[wave][3][lane] = bp;
+                        __syncthreads();
+                        if (wave < 4)
+                            for (int b = 0; b * CELL_BATCH < m; b++)
+                                gx += (double)xb[b][wave][lane];
+                        __syncthreads();
+                    } else {
+                        // wave w < 3: component w, wave 3: the potential (gx)
+                        const unsigned long long mm = sc.mask[j0 + min(lane, m - 1)];
+                        for (int r = 0; r < m; r += NW) {
+                            if (r + wave < m) {
+                                const GNode nd = gn[__builtin_amdgcn_readlane(mine, r + wave)];
+                                const double dr[3] = {rpx - nd.r[0], rpy - nd.r[1],
+                                                      rpz - nd.r[2]};
+                                const double d2 = dist2_unfused(dr[0], dr[1], dr[2]);
+                                const CellFactors f =
+                                    cell_factors<OCT>(dr[0], dr[1], dr[2],
+                                                      rsqrt_fp64(d2 + SMALL_NUMBER), nd.m, nd.q,
+                                                      nd.oc);
+#pragma unroll
+                                for (int k = 0; k < 3; k++) {
+                                    xc[wave][k][lane] = dr[k];
+                                    xc[wave][3 + k][lane] = f.Q[k];
+                                    if (OCT) xc[wave][6 + k][lane] = f.H[k];
+                                }
+                                xc[wave][9][lane] = f.ir5;
+                                xc[wave][10][lane] = f.ir7;
+                                xc[wave][11][lane] = f.crad;
+                                xc[wave][12][lane] = f.phi;
+                            }
+                            __syncthreads();
+                            if (wave < 4)
+#pragma unroll
+                                for (int k = 0; k < NW; k++) {
+                                    if (r + k >= m) break;
+                                    const int e = r + k;
+                                    const unsigned long long em =
+                                        (unsigned)__builtin_amdgcn_readlane((int)mm, e) |
+                                        (unsigned long long)(unsigned)__builtin_amdgcn_readlane(
+                                            (int)(mm >> 32), e) << 32;
+                                    if (!__builtin_amdgcn_inverse_ballot_w64(em)) continue;
+                                    if (wave == 3)
+                                        gx = gx + xc[k][12][lane];
+                                    else
+                                        gx = add_cell<OCT>(gx, xc[k][3 + wave][lane],
+                                                           xc[k][9][lane],
+                                                           OCT ? xc[k][6 + wave][lane] : 0.0,
+                                                           xc[k][10][lane], xc[k][11][lane],
+                                                           xc[k][wave][lane]);
+                                }
+                            __syncthreads();
+                        }
+                    }
+                }
+            } else for (int j0 = i0; j0 < i1; j0 += WAVE) {
                 const int m = min(WAVE, i1 - j0);
                 const int mine = sc.list[j0 + min(lane, m - 1)];
                 unsigned mlo = 0, mhi = 0;
@@ -1142,20 +1386,24 @@ __global__ void __launch_bounds__(LW_TB) k_grav_list(
                 if (!MIXED) sc.mask[tid] = keepm;
             }
             ws = we;
-            we = min(rr.y, ws + LW_BITS);
+            we = min(rr.y, ws + L.CELLS);
         }
+        if (ordered) {
+            if (wave < 4 && valid) (wave == 0 ? cx : wave == 1 ? cy : wave == 2 ? cz : cp)[p] = gx;
+        } else {
         // the waves' sums, added in wave order
         double *sum = reinterpret_cast<double *>(L.bits[0]);   // [component][wave][lane]
-        sum[(0 * LW_WAVES + wave) * WAVE + lane] = gx;
-        sum[(1 * LW_WAVES + wave) * WAVE + lane] = gy;
-        sum[(2 * LW_WAVES + wave) * WAVE + lane] = gz;
-        sum[(3 * LW_WAVES + wave) * WAVE + lane] = gp;
+        sum[(0 * NW + wave) * WAVE + lane] = gx;
+        sum[(1 * NW + wave) * WAVE + lane] = gy;
+        sum[(2 * NW + wave) * WAVE + lane] = gz;
+        sum[(3 * NW + wave) * WAVE + lane] = gp;
         __syncthreads();
         if (wave < 4) {
-            double s = sum[wave * LW_WAVES * WAVE + lane];
+            double s = sum[wave * NW * WAVE + lane];
 #pragma unroll
-            for (int w = 1; w < LW_WAVES; w++) s += sum[(wave * LW_WAVES + w) * WAVE + lane];
+            for (int w = 1; w < NW; w++) s += sum[(wave * NW + w) * WAVE + lane];
             if (valid) (wave == 0 ? cx : wave == 1 ? cy : wave == 2 ? cz : cp)[p] = s;
+        }
         }
         if (tid == 0) {
             cost[g] = gvis;
@@ -1387,12 +1635,14 @@ __global__ void __launch_bounds__(256) k_grav_cells_mixed(
 // 4.6 ms, r^-2 sphere of 1M, which fills the device, 3.1 ms either way.
 constexpr int PL_STAGE = 16;
 constexpr int PM_WAVES = 8;
+constexpr int PM_LEAVES = 4;   // leaves per wave and round of ordered sums
 constexpr int PM_TB = PM_WAVES * WAVE;
 
 template <int MACT, bool QUINTIC>
 __device__ __forceinline__ void pairs_group_mixed(
     int g, int wave, int n, int nc, const GNodeF *__restrict__ gn, const float4 *__restrict__ rec,
-    float4 *__restrict__ stage, double *__restrict__ sums,
+    float4 *__restrict__ stage, double *__restrict__ sums, float *__restrict__ xsum,
+    const int *__restrict__ cloud_off,
     const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
     const double *__restrict__ h, const double *__restrict__ zeta,
     const int *__restrict__ cid, const int2 *__restrict__ root_range,
@@ -1453,6 +1703,26 @@ __device__ __forceinline__ void pairs_group_mixed(
             pq.add(bp);
         }
     };
+    // one leaf's sums over the valid lanes, stored (ordered sums)
+    auto leaf_sums = [&](const float4 *src, int first, int count, float *out) {
+        const float ox = (float)(x[first] - rpx), oy = (float)(y[first] - rpy),
+                    oz = (float)(z[first] - rpz);
+        float bx = 0.0f, by = 0.0f, bz = 0.0f, bp = 0.0f;
+        const unsigned long long mm = ballot(valid);
+        for (int i = 0; i < count; i++) {
+            const int j = first + i;
+            const float4 a = src[2 * i], b = src[2 * i + 1];
+            const unsigned sl = (unsigned)(j - gr.x);
+            const unsigned long long mact = mm & ~(sl < WAVE ? 1ull << sl : 0ull);
+            npp += (unsigned)__popcll(mact);
+            pair_f32(kg, t4, tp, valid && j != p, mact, a.x + ox, a.y + oy, a.z + oz, a.w, b.x,
+                     b.y, b.z, b.w, bx, by, bz, bp, nin_p, nin_j);
+        }
+        out[0 * WAVE] = bx;
+        out[1 * WAVE] = by;
+        out[2 * WAVE] = bz;
+        out[3 * WAVE] = bp;
+    };
     // the same terms with the leaf's records read from the wave's LDS stage
     // (src: the leaf's LEAFMAX slots of two float4)
     auto leaf_pairs_staged = [&](const float4 *src, int first, int count, bool mine) {
@@ -1477,7 +1747,37 @@ __device__ __forceinline__ void pairs_group_mixed(
         }
     };
     const int len = uniform(near.len[g]);
-    if (len != NEAR_DROPPED) {
+    const int root =
+        __builtin_amdgcn_readlane(valid ? cid[p] : 0, __ffsll((long long)ballot(valid)) - 1);
+    const bool ordered = cloud_off[root + 1] - cloud_off[root] <= LW_ORDERED;
+    if (ordered && len != NEAR_DROPPED) {
+        // PM_LEAVES leaves per wave and round; their sums go to the four waves
+        // that add them in list order, one component each (px)
+        for (int r = 0; r < len; r += PM_WAVES * PM_LEAVES) {
+            const int e0 = r + wave * PM_LEAVES, nb = max(0, min(PM_LEAVES, len - e0));
+            int dl = 0;
+            if (lane < nb) {
+                dl = near.leaf[near.slot(g, e0) + lane];   // in one page
+                const int f = dl >> 4, k = dl & 15;
+                float4 *dst = stage + 2 * LEAFMAX * lane;
+                for (int i = 0; i < k; i++) {
+                    dst[2 * i] = rec[2 * (size_t)(f + i)];
+                    dst[2 * i + 1] = rec[2 * (size_t)(f + i) + 1];
+                }
+            }
+            wave_lds_fence();
+            for (int e = 0; e < nb; e++) {
+                const int d = __builtin_amdgcn_readlane(dl, e);
+                leaf_sums(stage + 2 * LEAFMAX * e, d >> 4, d & 15,
+                          xsum + ((wave * PM_LEAVES + e) * 4) * WAVE + lane);
+            }
+            __syncthreads();
+            if (wave < 4)
+                for (int e = 0; e < min(PM_WAVES * PM_LEAVES, len - r); e++)
+                    px.add(xsum[(e * 4 + wave) * WAVE + lane]);
+            __syncthreads();
+        }
+    } else if (len != NEAR_DROPPED) {
         // the near list in batches of PL_STAGE leaves: lane l copies the
         // records of the batch's leaf l into the wave's LDS stage (all the
         // batch's loads in flight at once), then the wave forms the pairs
@@ -1525,7 +1825,8 @@ __device__ __forceinline__ void pairs_group_mixed(
             if (group_accepts<MACT>(nd, vmask, rpx, rpy, rpz, afactor, d0, d1, d2)) {
                 c = nd.next;
             } else if (nd.leaf > 0) {
-                if (e / PL_STAGE % PM_WAVES == wave) leaf_pairs(nd.first, nd.leaf, valid);
+                if ((ordered ? 0 : e / PL_STAGE % PM_WAVES) == wave)
+                    leaf_pairs(nd.first, nd.leaf, valid);
                 e++;
                 c = nd.next;
             } else {
@@ -1542,7 +1843,12 @@ __device__ __forceinline__ void pairs_group_mixed(
     __syncthreads();
     if (wave == 0 && valid) {
         double gx = ax[p], gy = ay[p], gz = az[p], gp = cpot[p];
-        for (int w = 0; w < PM_WAVES; w++) {
+        if (ordered && len != NEAR_DROPPED) {   // component w is wave w's px
+            gx += sums[(0 * 4 + 0) * WAVE + lane];
+            gy += sums[(1 * 4 + 0) * WAVE + lane];
+            gz += sums[(2 * 4 + 0) * WAVE + lane];
+            gp += sums[(3 * 4 + 0) * WAVE + lane];
+        } else for (int w = 0; w < (ordered ? 1 : PM_WAVES); w++) {
             gx += sums[(w * 4 + 0) * WAVE + lane];
             gy += sums[(w * 4 + 1) * WAVE + lane];
             gz += sums[(w * 4 + 2) * WAVE + lane];
@@ -1570,7 +1876,7 @@ __global__ void __launch_bounds__(PM_TB) k_grav_pairs_mixed(
     const double *__restrict__ cpot, double *__restrict__ gpot, double *__restrict__ agm,
     NearList near, unsigned long long *__restrict__ icount, const int2 *__restrict__ grp,
     int ngrp,
-    GroupQueue queue) {
+    const int *__restrict__ cloud_off, GroupQueue queue) {
     // persistent over the walk's queue: the groups of each XCD range
     // longest-first (by the previous walk's cost), as phase 1 takes them
     __builtin_amdgcn_s_setprio(2);
@@ -1578,6 +1884,7 @@ __global__ void __launch_bounds__(PM_TB) k_grav_pairs_mixed(
     // in its place at the end, the waves' sums
     __shared__ float4 stage_all[PM_WAVES * PL_STAGE * LEAFMAX * 2];
     static_assert(sizeof(stage_all) >= sizeof(double) * 4 * PM_TB, "sums fit");
+    __shared__ float xsum[PM_WAVES * PM_LEAVES * 4 * WAVE];
     __shared__ int job;
     const int wave = uniform((int)(threadIdx.x / WAVE));
     float4 *stage = stage_all + wave * (PL_STAGE * LEAFMAX * 2);
@@ -1594,7 +1901,8 @@ __global__ void __launch_bounds__(PM_TB) k_grav_pairs_mixed(
         const int g = uniform(job);
         if (g < 0) break;
         pairs_group_mixed<MACT, QUINTIC>(g, wave, n, nc, gn, rec, stage,
-                                         reinterpret_cast<double *>(stage_all), x, y, z, h, zeta,
+                                         reinterpret_cast<double *>(stage_all), xsum, cloud_off, x,
+                                         y, z, h, zeta,
                                          cid, root_range, active, t4, ax, ay, az, cpot, gpot, agm,
                                          near, icount, grp, ngrp, npp, nin_p, nin_j);
     }
@@ -1719,15 +2027,23 @@ NearList near_list(Ctx &c) {
                     c.pl_npage};
 }
 
+// particles of the smallest and the largest cloud
+void cloud_sizes(const Ctx &c, int &least, int &most) {
+    least = most = c.cloud_off_h[1] - c.cloud_off_h[0];
+    for (int i = 1; i < c.ncloud; i++) {
+        least = std::min(least, c.cloud_off_h[i + 1] - c.cloud_off_h[i]);
+        most = std::max(most, c.cloud_off_h[i + 1] - c.cloud_off_h[i]);
+    }
+}
+
 // phase 1 of the walk (traversal and cell terms), persistent over the
 // queue, on stream s with at most cap blocks per CU
 template <int OCT, int MACT>
 void launch_cells(Ctx &c, hipStream_t s, int cap) {
     GroupQueue q{c.gq.ctr, c.gq.order, c.gq.ngroups};
     const bool mixed = c.opt.precision == SERENX_MIXED;
-    int most = 0;   // particles of the largest cloud
-    for (int i = 0; i < c.ncloud; i++)
-        most = std::max(most, c.cloud_off_h[i + 1] - c.cloud_off_h[i]);
+    int least, most;
+    cloud_sizes(c, least, most);
     const bool waves = most > LW_ALONE;
     int *cont = c.gq.ctr + 2 * NXCD + 1;
     const LongWalks lw{waves ? c.lw_group : nullptr, c.lw_at, cont, cont + 1, LW_BUDGET, LW_ALONE};
@@ -1744,13 +2060,26 @@ void launch_cells(Ctx &c, hipStream_t s, int cap) {
                            c.gay, c.gaz, c.gpc, near_list(c), c.icount, c.wstat, q, c.gq.cost,
                            c.grp, c.cloud_off, lw);
     }
-    auto k = mixed ? k_grav_list<true, OCT, MACT> : k_grav_list<false, OCT, MACT>;
-    const int nb = std::min(walk_blocks(c, k, cap, LW_TB), c.lw_blocks);
     const ListScratch sc{c.lw_ids, c.lw_in, c.lw_open, c.lw_list, c.lw_mask, c.lw_cap};
-    hipLaunchKernelGGL(k, dim3(nb), dim3(LW_TB), 0, s, c.nc, c.gmac,
-                       mixed ? mixed_mac_scale(c) : 1.0, c.gn, c.gnf, c.x, c.y, c.z, c.cid,
-                       c.root_range, c.active, c.gpot, c.agm, c.gax, c.gay, c.gaz, c.gpc,
-                       near_list(c), sc, c.icount, c.wstat, q, c.gq.cost, c.grp, lw);
+    auto launch = [&](auto k, int tb, const GroupQueue &gq, const LongWalks &walks) {
+        const int nb = std::min(walk_blocks(c, k, cap, tb), c.lw_blocks);
+        hipLaunchKernelGGL(k, dim3(nb), dim3(tb), 0, s, c.nc, c.gmac,
+                           mixed ? mixed_mac_scale(c) : 1.0, c.gn, c.gnf, c.x, c.y, c.z, c.cid,
+                           c.root_range, c.active, c.gpot, c.agm, c.gax, c.gay, c.gaz, c.gpc,
+                           near_list(c), sc, c.icount, c.wstat, gq, c.gq.cost, c.grp,
+                           c.cloud_off, walks);
+    };
+    if (mixed) {
+        launch(k_grav_list<true, false, OCT, MACT>, LW_TB, q, lw);
+        return;
+    }
+    if (most > LW_ORDERED) launch(k_grav_list<false, false, OCT, MACT>, LW_TB, q, lw);
+    if (least <= LW_ORDERED) {
+        LongWalks lo = lw;
+        lo.taken = cont + 2;
+        launch(k_grav_list<false, true, OCT, MACT>, OW_TB, GroupQueue{cont + 3, q.order, q.ngroups},
+               lo);
+    }
 }
 
 // phase 2 (pair terms), persistent over the same queue order (its second
@@ -1764,13 +2093,22 @@ void launch_pairs(Ctx &c, const double4 *rec, hipStream_t s, int cap) {
                            c.gnf, reinterpret_cast<const float4 *>(rec), c.x, c.y, c.z, c.h,
                            c.zeta, c.cid, c.root_range, c.active,
                            reinterpret_cast<const float4 *>(c.ktab + KT_G4F_OFF), c.gax, c.gay,
-                           c.gaz, c.gpc, c.gpot, c.agm, near_list(c), c.icount, c.grp, c.ngrp, q);
+                           c.gaz, c.gpc, c.gpot, c.agm, near_list(c), c.icount, c.grp, c.ngrp,
+                           c.cloud_off, q);
     } else {
-        auto k = k_grav_pairs_fp64<MACT, QUINTIC>;
-        hipLaunchKernelGGL(k, dim3(walk_blocks(c, k, cap, PF_TB)), dim3(PF_TB), 0, s, c.nc,
-                           c.gn, rec, c.cid, c.root_range, c.active,
-                           reinterpret_cast<const double4 *>(c.ktab + KT_G4_OFF), c.gax, c.gay,
-                           c.gaz, c.gpc, c.gpot, c.agm, near_list(c), c.icount, c.grp, q);
+        int least, most;
+        cloud_sizes(c, least, most);
+        auto launch = [&](auto k, int tb, const GroupQueue &gq) {
+            hipLaunchKernelGGL(k, dim3(walk_blocks(c, k, cap, tb)), dim3(tb), 0, s, c.nc, c.gn, rec,
+                               c.cid, c.root_range, c.active,
+                               reinterpret_cast<const double4 *>(c.ktab + KT_G4_OFF), c.gax, c.gay,
+                               c.gaz, c.gpc, c.gpot, c.agm, near_list(c), c.icount, c.grp,
+                               c.cloud_off, gq);
+        };
+        if (most > LW_ORDERED) launch(k_grav_pairs_fp64<MACT, QUINTIC, false>, PF_TB, q);
+        if (least <= LW_ORDERED)
+            launch(k_grav_pairs_fp64<MACT, QUINTIC, true>, OW_TB,
+                   GroupQueue{c.gq.ctr + 3 * NXCD + 6, q.order, q.ngroups});
     }
 }
 
@@ -1808,7 +2146,7 @@ int prepare_queue(Ctx &c) {
         SX_TRY(sort_queue(c));
     }
     q.order_ready = false;   // used by this walk
-    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, c.gstream, 2 * NXCD + 3, q.ctr);
+    hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, c.gstream, 4 * NXCD + 6, q.ctr);
     SX_HIP(hipGetLastError());
     return SERENX_OK;
 }

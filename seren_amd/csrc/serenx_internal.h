@@ -81,6 +81,10 @@ constexpr int LW_BITS = 131072;
 // clouds of more particles are walked by one wave per group, which leaves a
 // walk to the list walk after LW_BUDGET visits (grav.hip has the reasons)
 constexpr int LW_ALONE = 393216;
+// clouds of at most this many particles have their terms added in walk order
+// (grav.hip; twice the time of a walk there, and nothing to gain by it where a
+// cloud is not followed through a collapse)
+constexpr int LW_ORDERED = 6144;
 constexpr int LW_BUDGET = 8192;
 constexpr int LW_CAP = 8192;
 // leaves a wave of the neighbour walk records for the rows of its particles
@@ -349,9 +353,10 @@ struct Ctx {
     // work queue of the persistent gravity walk (walk.h: GroupQueue)
     struct WalkQueue {
         int ngroups = 0;
-        int *ctr = nullptr;          // 2 NXCD counters (one set per walk phase), the
-                                     // next free page of the near-list pool, the
-                                     // walks left to the list walk and those taken
+        // counters: NXCD of each walk phase, then the next free page of the
+        // near-list pool, the walks left to the list walk and those taken (two
+        // launches), and NXCD of each phase for the clouds with ordered sums
+        int *ctr = nullptr;
         int *cost = nullptr;         // per group: cells its last walk visited
         int *order = nullptr;        // group ids by range, then decreasing cost
         uint64_t *keys = nullptr, *keys2 = nullptr;

@@ -1244,19 +1244,56 @@ __global__ void k_pack_hydro(int n, const double *__restrict__ x, const double *
 // INTERNAL_ENERGY terms, du/dt = sum 0.5 m_j visc W_mean (dv.dr) / |dr|
 // (:258-259) - P div v / (Omega rho) (:326-332)
 //
-// HYD_LPP lanes take a particle, each every HYD_LPP-th neighbour; their sums
-// are added in a fixed tree.  One lane per particle went through its row in a
-// chain of gather, square root and divisions, and the longest row held the
-// launch: 115 -> 35 us at 2,048 particles, 650 -> 90 us on a Plummer sphere of
-// 2,053 (rows of thousands), 569 -> 326 us on an r^-2 sphere of 300,007, where
-// eight gathers of a particle in flight hide the L2 misses that bound it.
+// HYD_LPP lanes take a particle, each every HYD_LPP-th neighbour.  The factors
+// of eight neighbours' terms then go through LDS to the lanes that add them in
+// list order, one lane per sum (three of the pressure force, three of the
+// viscous one, du/dt), so the sums are those of one lane bit for bit.
+//
+// One lane per particle went through its row in a chain of gather, square root
+// and divisions, and the longest row held the launch: 115 -> 40 us at 2,048 particles,
+// 650 -> 95 us on a Plummer sphere of 2,053 (rows of thousands), 569 -> 337 us on
+// an r^-2 sphere of 300,007, where eight gathers of a particle in flight hide
+// the L2 misses that bound it.
 constexpr int HYD_LPP = 8;
 
-// the sum over the lanes of a particle, on each of them
-__device__ __forceinline__ double hyd_sum(double v) {
+// per wave [f_p, f_pp, f_visc, e1, e2, ux, uy, uz][lane], one column of
+// padding: the eight lanes of a particle read one lane's entries
+using HydXch = double[8][WAVE + 1];
+
+// The calling lane's sum with eight neighbours' terms f u added in their
+// order: f_p u and f_pp u (lanes 0-2, the components of the pressure force),
+// f_visc u (lanes 3-5), e1 and e2 (lane 6, du/dt).  A neighbour without a
+// term has zeros: they leave the sum (never -0) as it is.
+__device__ __forceinline__ double hyd_add(HydXch &x, int lane, int sub, double acc, double f1,
+                                          double f2, double f3, double e1, double e2, double ux,
+                                          double uy, double uz) {
+    x[0][lane] = f1;
+    x[1][lane] = f2;
+    x[2][lane] = f3;
+    x[3][lane] = e1;
+    x[4][lane] = e2;
+    x[5][lane] = ux;
+    x[6][lane] = uy;
+    x[7][lane] = uz;
+    wave_lds_fence();
+    const int l0 = lane & ~(HYD_LPP - 1);
+    const int ra = sub < 3 ? 0 : sub < 6 ? 2 : 3, rb = sub < 3 ? 1 : 4,
+              ru = 5 + (sub < 3 ? sub : sub < 6 ? sub - 3 : 0);
+    double fa[HYD_LPP], fb[HYD_LPP], fu[HYD_LPP];
 #pragma unroll
-    for (int d = 1; d < HYD_LPP; d *= 2) v += __shfl_xor(v, d, WAVE);
-    return v;
+    for (int k = 0; k < HYD_LPP; k++) {
+        fa[k] = x[ra][l0 + k];
+        fb[k] = x[rb][l0 + k];
+        fu[k] = x[ru][l0 + k];
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (int k = 0; k < HYD_LPP; k++) {
+        const double u = sub < 6 ? fu[k] : 1.0;
+        acc = acc + fa[k] * u;
+        acc = acc + (sub >= 3 && sub < 6 ? 0.0 : fb[k] * u);
+    }
+    return acc;
 }
 
 template <bool ENERGY>
@@ -1267,8 +1304,13 @@ __global__ void __launch_bounds__(256) k_hydro(
     double *__restrict__ ax, double *__restrict__ ay, double *__restrict__ az,
     const double *__restrict__ press, const double *__restrict__ divv,
     const double *__restrict__ omega, double *__restrict__ dudt) {
-    const int t = xcd_block() * blockDim.x + threadIdx.x, p = t / HYD_LPP, sub = t % HYD_LPP;
-    if (p >= n || !active[p]) return;
+    __shared__ HydXch xch_all[256 / WAVE];
+    HydXch &xch = xch_all[threadIdx.x / WAVE];
+    const int t = xcd_block() * blockDim.x + threadIdx.x, sub = t % HYD_LPP;
+    const int lane = (int)(threadIdx.x & (WAVE - 1));
+    const bool valid = t / HYD_LPP < n && active[t / HYD_LPP];
+    if (ballot(valid) == 0) return;
+    const int p = valid ? t / HYD_LPP : 0;   // (lanes without a particle: an empty row)
     const double *w1 = ktab + T_W1 * KT;
     const double4 *rp = rec + 4 * (size_t)p;
     const double4 r0 = rp[0], r1 = rp[1], r2 = rp[2], r3 = rp[3];
@@ -1277,68 +1319,58 @@ __global__ void __launch_bounds__(256) k_hydro(
     const double rho_p = r2.x, pfactor_p = r2.y, sound_p = r2.z, invhp = r2.w;
     const double hfactor_p = r3.x;
     const double beta = 2.0 * alpha;
-    double ahx = 0.0, ahy = 0.0, ahz = 0.0, adx = 0.0, ady = 0.0, adz = 0.0;
-    double dudt_diss = 0.0;
-    const int nn = pptot[p];
+    double acc = 0.0;
+    const int nn = valid ? pptot[p] : 0;
     const int *lst = (nn <= pp_limit) ? pplist + (size_t)p * pp_limit : ovf_list + ovf_off[p];
-    for (int i = sub; i < nn; i += HYD_LPP) {
-        const double4 *rq = rec + 4 * (size_t)lst[i];
-        const double4 q0 = rq[0], q1 = rq[1], q2 = rq[2];
-        double wmean = 0.0;
-        const double hpp = q0.w, mpp = q1.w, rho_pp = q2.x;
-        double ux = q0.x - rpx, uy = q0.y - rpy, uz = q0.z - rpz;
-        double drmag = ux * ux + uy * uy + uz * uz;
-        if (drmag >= kg.rangesqd * hp * hp && drmag >= kg.rangesqd * hpp * hpp) continue;
-        drmag = sqrt(drmag) + SMALL_NUMBER;
-        const double dvx = q1.x - vpx, dvy = q1.y - vpy, dvz = q1.z - vpz;
-        const double dvdr = dvx * ux + dvy * uy + dvz * uz;
-        const double invdrmag = 1.0 / drmag;
-        ux = ux * invdrmag;
-        uy = uy * invdrmag;
-        uz = uz * invdrmag;
-        if (drmag < kg.range * hp) {
-            int kern = (int)(kg.half * drmag * invhp);
-            kern = min(kern, KERNTOT);
-            const double wk = w1[kern];
-            wmean = 0.5 * hfactor_p * wk;
-            const double f = mpp * pfactor_p * hfactor_p * wk;
-            ahx = ahx + f * ux;
-            ahy = ahy + f * uy;
-            ahz = ahz + f * uz;
+    for (int i0 = 0; any_lane(i0 < nn); i0 += HYD_LPP) {
+        double f1 = 0.0, f2 = 0.0, f3 = 0.0, e1 = 0.0, ux = 0.0, uy = 0.0, uz = 0.0;
+        if (i0 + sub < nn) {
+            const double4 *rq = rec + 4 * (size_t)lst[i0 + sub];
+            const double4 q0 = rq[0], q1 = rq[1], q2 = rq[2];
+            const double hpp = q0.w, mpp = q1.w, rho_pp = q2.x;
+            const double dx = q0.x - rpx, dy = q0.y - rpy, dz = q0.z - rpz;
+            const double drsqd = dx * dx + dy * dy + dz * dz;
+            if (!(drsqd >= kg.rangesqd * hp * hp) || !(drsqd >= kg.rangesqd * hpp * hpp)) {
+                const double drmag = sqrt(drsqd) + SMALL_NUMBER;
+                const double dvx = q1.x - vpx, dvy = q1.y - vpy, dvz = q1.z - vpz;
+                const double dvdr = dvx * dx + dvy * dy + dvz * dz;
+                const double invdrmag = 1.0 / drmag;
+                double wmean = 0.0;
+                ux = dx * invdrmag;
+                uy = dy * invdrmag;
+                uz = dz * invdrmag;
+                if (drmag < kg.range * hp) {
+                    const int kern = min((int)(kg.half * drmag * invhp), KERNTOT);
+                    const double wk = w1[kern];
+                    wmean = 0.5 * hfactor_p * wk;
+                    f1 = mpp * pfactor_p * hfactor_p * wk;
+                }
+                if (drmag < kg.range * hpp) {
+                    const double invhpp = q2.w, hfactor_pp = rq[3].x, pfactor_pp = q2.y;
+                    const int kern = min((int)(kg.half * drmag * invhpp), KERNTOT);
+                    const double wk = w1[kern];
+                    wmean = wmean + 0.5 * hfactor_pp * wk;
+                    f2 = mpp * pfactor_pp * hfactor_pp * wk;
+                }
+                if (dvdr < 0.0) {
+                    const double rhomean = 0.5 * (rho_p + rho_pp);
+                    const double vsignal = 0.5 * (sound_p + q2.z);
+                    const double mu = 0.5 * (hp + hpp) * dvdr /
+                                      (drmag * drmag + 0.25 * ETA_SQD * (hp + hpp) * (hp + hpp));
+                    const double visc = (-alpha * vsignal * mu + beta * mu * mu) / rhomean;
+                    f3 = mpp * visc * wmean;
+                    if (ENERGY) e1 = 0.5 * mpp * visc * wmean * dvdr * invdrmag;
+                }
+            }
         }
-        if (drmag < kg.range * hpp) {
-            const double invhpp = q2.w, hfactor_pp = rq[3].x, pfactor_pp = q2.y;
-            int kern = (int)(kg.half * drmag * invhpp);
-            kern = min(kern, KERNTOT);
-            const double wk = w1[kern];
-            wmean = wmean + 0.5 * hfactor_pp * wk;
-            const double f = mpp * pfactor_pp * hfactor_pp * wk;
-            ahx = ahx + f * ux;
-            ahy = ahy + f * uy;
-            ahz = ahz + f * uz;
-        }
-        const double rhomean = 0.5 * (rho_p + rho_pp);
-        if (dvdr < 0.0) {
-            const double vsignal = 0.5 * (sound_p + q2.z);
-            const double mu = 0.5 * (hp + hpp) * dvdr /
-                              (drmag * drmag + 0.25 * ETA_SQD * (hp + hpp) * (hp + hpp));
-            const double visc = (-alpha * vsignal * mu + beta * mu * mu) / rhomean;
-            const double f = mpp * visc * wmean;
-            adx = adx + f * ux;
-            ady = ady + f * uy;
-            adz = adz + f * uz;
-            if (ENERGY) dudt_diss = dudt_diss + 0.5 * mpp * visc * wmean * dvdr * invdrmag;
-        }
+        acc = hyd_add(xch, lane, sub, acc, f1, f2, f3, e1, 0.0, ux, uy, uz);
     }
-    ahx = hyd_sum(ahx) + hyd_sum(adx);
-    ahy = hyd_sum(ahy) + hyd_sum(ady);
-    ahz = hyd_sum(ahz) + hyd_sum(adz);
-    if (ENERGY) dudt_diss = hyd_sum(dudt_diss);
-    if (sub != 0) return;
-    ax[p] = ahx;
-    ay[p] = ahy;
-    az[p] = ahz;
-    if (ENERGY) dudt[p] = (0.0 + dudt_diss) - press[p] * divv[p] / omega[p] / rho_p;
+    // the pressure force's lane takes the viscous one's sum; lane 6 has du/dt
+    const double ad = __shfl(acc, lane + 3, WAVE), du = __shfl(acc, lane + 6, WAVE);
+    if (!valid || sub > 2) return;
+    (sub == 0 ? ax : sub == 1 ? ay : az)[p] = acc + ad;
+    if (ENERGY && sub == 0)
+        dudt[p] = (0.0 + du) - press[p] * divv[p] / omega[p] / rho_p;
 }
 
 // Mixed-precision hydro record, 64 bytes per particle: the position in FP64
@@ -1808,8 +1840,13 @@ __global__ void __launch_bounds__(256) k_hydro_std(
     const int *__restrict__ ovf_list, int pp_limit, const double *__restrict__ ktab, double alpha,
     double *__restrict__ ax, double *__restrict__ ay, double *__restrict__ az,
     double *__restrict__ dudt_out) {
-    const int t = xcd_block() * blockDim.x + threadIdx.x, p = t / HYD_LPP, sub = t % HYD_LPP;
-    if (p >= n || !active[p]) return;
+    __shared__ HydXch xch_all[256 / WAVE];
+    HydXch &xch = xch_all[threadIdx.x / WAVE];
+    const int t = xcd_block() * blockDim.x + threadIdx.x, sub = t % HYD_LPP;
+    const int lane = (int)(threadIdx.x & (WAVE - 1));
+    const bool valid = t / HYD_LPP < n && active[t / HYD_LPP];
+    if (ballot(valid) == 0) return;
+    const int p = valid ? t / HYD_LPP : 0;   // (lanes without a particle: an empty row)
     const double *w1 = ktab + T_W1 * KT;
     const double4 *rp = rec + 4 * (size_t)p;
     const double4 r0 = rp[0], r1 = rp[1], r2 = rp[2], r3 = rp[3];
@@ -1817,58 +1854,56 @@ __global__ void __launch_bounds__(256) k_hydro_std(
     const double vpx = r1.x, vpy = r1.y, vpz = r1.z;
     const double rho_p = r2.x, pfactor_p = r2.y, sound_p = r2.z, invhp = r2.w;
     const double hfactor_p = r3.x;
-    double ahx = 0.0, ahy = 0.0, ahz = 0.0, adx = 0.0, ady = 0.0, adz = 0.0, dudt = 0.0;
-    const int nn = pptot[p];
+    double acc = 0.0;
+    const int nn = valid ? pptot[p] : 0;
     const int *lst = (nn <= pp_limit) ? pplist + (size_t)p * pp_limit : ovf_list + ovf_off[p];
-    for (int i = sub; i < nn; i += HYD_LPP) {
-        const double4 *rq = rec + 4 * (size_t)lst[i];
-        const double4 q0 = rq[0], q1 = rq[1], q2 = rq[2];
-        const double hpp = q0.w, mpp = q1.w, rho_pp = q2.x;
-        const double dx = q0.x - rpx, dy = q0.y - rpy, dz = q0.z - rpz;
-        const double drsqd = dx * dx + dy * dy + dz * dz;
-        if (drsqd >= kg.rangesqd * hp * hp && drsqd >= kg.rangesqd * hpp * hpp) continue;
-        const double drmag = sqrt(drsqd) + SMALL_NUMBER;
-        const double invdrmag = 1.0 / drmag;
-        const double ux = dx * invdrmag, uy = dy * invdrmag, uz = dz * invdrmag;
-        const double dvx = q1.x - vpx, dvy = q1.y - vpy, dvz = q1.z - vpz;
-        const double dvdr = dvx * dx + dvy * dy + dvz * dz;
-        double wmean = 0.0;
-        if (drmag < kg.range * hp) {
-            const int kern = min((int)(kg.half * drmag * invhp), KERNTOT);
-            wmean = 0.5 * hfactor_p * invhp * w1[kern];
+    for (int i0 = 0; any_lane(i0 < nn); i0 += HYD_LPP) {
+        double f1 = 0.0, f3 = 0.0, e1 = 0.0, e2 = 0.0, ux = 0.0, uy = 0.0, uz = 0.0;
+        if (i0 + sub < nn) {
+            const double4 *rq = rec + 4 * (size_t)lst[i0 + sub];
+            const double4 q0 = rq[0], q1 = rq[1], q2 = rq[2];
+            const double hpp = q0.w, mpp = q1.w, rho_pp = q2.x;
+            const double dx = q0.x - rpx, dy = q0.y - rpy, dz = q0.z - rpz;
+            const double drsqd = dx * dx + dy * dy + dz * dz;
+            if (!(drsqd >= kg.rangesqd * hp * hp) || !(drsqd >= kg.rangesqd * hpp * hpp)) {
+                const double drmag = sqrt(drsqd) + SMALL_NUMBER;
+                const double invdrmag = 1.0 / drmag;
+                ux = dx * invdrmag;
+                uy = dy * invdrmag;
+                uz = dz * invdrmag;
+                const double dvx = q1.x - vpx, dvy = q1.y - vpy, dvz = q1.z - vpz;
+                const double dvdr = dvx * dx + dvy * dy + dvz * dz;
+                double wmean = 0.0;
+                if (drmag < kg.range * hp) {
+                    const int kern = min((int)(kg.half * drmag * invhp), KERNTOT);
+                    wmean = 0.5 * hfactor_p * invhp * w1[kern];
+                }
+                if (drmag < kg.range * hpp) {
+                    const double invhpp = q2.w, hfactor_pp = rq[3].x;
+                    const int kern = min((int)(kg.half * drmag * invhpp), KERNTOT);
+                    wmean = wmean + 0.5 * hfactor_pp * invhpp * w1[kern];
+                }
+                const double pf = pfactor_p + rq[3].y;
+                f1 = mpp * wmean * pf;
+                if (ENERGY) e1 = 0.5 * mpp * wmean * dvdr * invdrmag * pf;
+                if (dvdr < 0.0) {                              // hydro.F90:221-224
+                    const double rhomean = 0.5 * (rho_p + rho_pp);
+                    const double beta = 2 * alpha;
+                    const double vsignal = 0.5 * (sound_p + q2.z);
+                    const double mu = 0.5 * (hp + hpp) * dvdr /
+                                      (drsqd + 0.25 * ETA_SQD * (hp + hpp) * (hp + hpp));
+                    const double visc = (-alpha * vsignal * mu + beta * mu * mu) / rhomean;
+                    f3 = mpp * visc * wmean;
+                    if (ENERGY) e2 = 0.5 * mpp * visc * wmean * dvdr * invdrmag;
+                }
+            }
         }
-        if (drmag < kg.range * hpp) {
-            const double invhpp = q2.w, hfactor_pp = rq[3].x;
-            const int kern = min((int)(kg.half * drmag * invhpp), KERNTOT);
-            wmean = wmean + 0.5 * hfactor_pp * invhpp * w1[kern];
-        }
-        const double pf = pfactor_p + rq[3].y;
-        ahx = ahx + mpp * wmean * pf * ux;
-        ahy = ahy + mpp * wmean * pf * uy;
-        ahz = ahz + mpp * wmean * pf * uz;
-        if (ENERGY) dudt = dudt + 0.5 * mpp * wmean * dvdr * invdrmag * pf;
-        const double rhomean = 0.5 * (rho_p + rho_pp);
-        if (dvdr < 0.0) {                                      // hydro.F90:221-224
-            const double beta = 2 * alpha;
-            const double vsignal = 0.5 * (sound_p + q2.z);
-            const double mu = 0.5 * (hp + hpp) * dvdr /
-                              (drsqd + 0.25 * ETA_SQD * (hp + hpp) * (hp + hpp));
-            const double visc = (-alpha * vsignal * mu + beta * mu * mu) / rhomean;
-            adx = adx + mpp * visc * wmean * ux;
-            ady = ady + mpp * visc * wmean * uy;
-            adz = adz + mpp * visc * wmean * uz;
-            if (ENERGY) dudt = dudt + 0.5 * mpp * visc * wmean * dvdr * invdrmag;
-        }
+        acc = hyd_add(xch, lane, sub, acc, f1, 0.0, f3, e1, e2, ux, uy, uz);
     }
-    ahx = hyd_sum(ahx) + hyd_sum(adx);
-    ahy = hyd_sum(ahy) + hyd_sum(ady);
-    ahz = hyd_sum(ahz) + hyd_sum(adz);
-    if (ENERGY) dudt = hyd_sum(dudt);
-    if (sub != 0) return;
-    ax[p] = ahx;
-    ay[p] = ahy;
-    az[p] = ahz;
-    if (ENERGY) dudt_out[p] = dudt;
+    const double ad = __shfl(acc, lane + 3, WAVE), du = __shfl(acc, lane + 6, WAVE);
+    if (!valid || sub > 2) return;
+    (sub == 0 ? ax : sub == 1 ? ay : az)[p] = acc + ad;
+    if (ENERGY && sub == 0) dudt_out[p] = du;
 }
 
 // sph_update.F90:107-109 (HFIND=CONSTANT): parray(SMOO,1:ptot) = hmin
