@@ -314,9 +314,9 @@ int serenx_serve_info(serenx_ctx *ctx, int32_t ncloud, double *dt, double *time)
  *    autotuner in seren_amd/autotune.py times a few).  A walk with nothing
  *    beside it (serenx_grav_forces) takes all that fit.  0 launches one wave
  *    per group in tree order.  Results do not change.
- *  SERENX_TUNE_NEIB_GROUP: 1 (default) builds the neighbour lists with one
- *    walk per wave that opens every cell any of its particles could need; 0
- *    with the particles' own walks (BHhydro_walk.F90's test per particle).
+ *  SERENX_TUNE_NEIB_GROUP: 1 (default) builds the neighbour lists with searches
+ *    by whole waves, eight particles each; 0 with the particles' own walks
+ *    (BHhydro_walk.F90's test per particle).
  *    The lists are the same.
  *  SERENX_TUNE_HSOLVE_WAVES: waves per SIMD of the grad-h iteration kernel:
  *    8 (registers capped at 64, a few spills), 0 (the compiler's budget,
@@ -329,11 +329,9 @@ int serenx_serve_info(serenx_ctx *ctx, int32_t ncloud, double *dt, double *time)
  *    pair phase with the same MAC decisions (the same leaves in the same
  *    order): results do not change, only speed; tests lower it to drive
  *    that path.
- *  SERENX_TUNE_NEIB_LEAVES: leaves each wave of the neighbour walk records
- *    (in DFS order) for its particles with more than pp_limit neighbours,
- *    0..512 (default 512).  Such a particle's complete row is formed from
- *    that list by the whole wave; when the list did not fit (or at 0) the
- *    particle walks the tree alone.  The rows are the same either way.
+ *  SERENX_TUNE_NEIB_LEAVES: 0..512 (default 512).  Kept for programs that set
+ *    it: rows above pp_limit are searched by whole waves, which keep no list
+ *    of leaves, so the value has no effect.
  *  SERENX_TUNE_PAIR_BLOCKS: blocks per CU of the walk's pair phase, 1..64,
  *    or 0 (default) for SERENX_TUNE_WALK_QUEUE's value; used when the work
  *    queue is on.  Results do not change.

@@ -247,8 +247,6 @@ int ensure_capacity(Ctx &c, int n) {
     SX_TRY(dalloc(&c.pplist, nn * (size_t)c.pp_limit));
     SX_TRY(dalloc(&c.ovf_off, nn));
     SX_TRY(dalloc(&c.ovf_idx, nn));
-    SX_TRY(dalloc(&c.nbl, particle_waves(n) * NB_CAP));
-    SX_TRY(dalloc(&c.nbl_len, particle_waves(n)));
     SX_TRY(dalloc(&c.hq, nn));
     SX_TRY(dalloc(&c.hq_len, 1));
     SX_TRY(dalloc(&c.hrec, nn * 16));
@@ -267,14 +265,15 @@ int ensure_capacity(Ctx &c, int n) {
     SX_TRY(dalloc(&c.pl_page, ng * PL_PAGES));
     // two list-walk blocks fit a CU; a block never visits more cells than the
     // context has (2 n + 2 and the roots of a forest)
-    c.lw_blocks = (int)std::min(ng, (size_t)2 * c.ncu);
+    c.lw_blocks = (int)std::min(((size_t)n + WAVE - 1) / WAVE + 64, (size_t)2 * c.ncu);
     c.lw_cap = (int)std::min((size_t)LW_CAP, 2 * nn + (size_t)forest_max_clouds(n, c.pp_gather));
-    const size_t lw = (size_t)c.lw_blocks * c.lw_cap;
-    SX_TRY(dalloc(&c.lw_ids, lw));
-    SX_TRY(dalloc(&c.lw_list, lw + 8 * (size_t)c.lw_blocks));
-    SX_TRY(dalloc(&c.lw_in, lw));
-    SX_TRY(dalloc(&c.lw_open, lw));
-    SX_TRY(dalloc(&c.lw_mask, lw + 8 * (size_t)c.lw_blocks));
+    // in one allocation: the 8-byte arrays, then the others
+    const size_t lw = (size_t)c.lw_blocks * c.lw_cap, lm = lw + 8 * (size_t)c.lw_blocks;
+    SX_TRY(dalloc(&c.lw_in, 2 * lw + lm + (lw + lm + 1) / 2));
+    c.lw_open = c.lw_in + lw;
+    c.lw_mask = c.lw_open + lw;
+    c.lw_ids = reinterpret_cast<int *>(c.lw_mask + lm);
+    c.lw_list = c.lw_ids + lw;
     SX_TRY(dalloc(&c.lw_group, ng));
     SX_TRY(dalloc(&c.lw_at, ng));
     SX_TRY(dalloc(&c.hlist, (((size_t)n + 255) / 256) * 4 * HL_SLOTS * WAVE));
@@ -307,7 +306,7 @@ void free_all(Ctx &c) {
                     c.press, c.sound, c.divv, c.drhodt, c.ax, c.ay, c.az, c.gpot, c.agm,
                     c.u, c.dudt,
                     c.tmpd, c.hrec, c.hlist, c.porig, c.tmpi, c.active, c.pptot, c.pplist, c.ovf_off,
-                    c.ovf_idx, c.nbl, c.nbl_len, c.hq, c.hq_len, c.bn, c.c_first, c.c_last,
+                    c.ovf_idx, c.hq, c.hq_len, c.bn, c.c_first, c.c_last,
                     c.ovf_list, c.ovf_count, c.khi, c.klo, c.khi2, c.klo2, c.idx, c.idx2,
                     c.cpl, c.pact, c.flag, c.incl, c.cellof, c.ncs, c.off, c.firstlev,
                     c.root, c.bbpart, c.cloud_off, c.cid, c.chunks, c.chunk_first,
@@ -315,7 +314,7 @@ void free_all(Ctx &c) {
                     c.c_level, c.bfs2dfs, c.dfs2bfs, c.dfs_parent, c.bbmin, c.bbmax,
                     c.hmaxs, c.gn, c.gs, c.gnf, c.hn, c.ktab, c.icount, c.wstat, c.band,
                     c.grec, c.gax, c.gay, c.gaz, c.gpc, c.grp, c.pl_leaf, c.pl_mask, c.pl_len, c.pl_page,
-                    c.lw_ids, c.lw_list, c.lw_in, c.lw_open, c.lw_mask, c.lw_group, c.lw_at, c.gmac, c.gq.ctr, c.gq.cost, c.gq.order,
+                    c.lw_in, c.lw_group, c.lw_at, c.gmac, c.gq.ctr, c.gq.cost, c.gq.order,
                     c.gq.vals, c.gq.keys, c.gq.keys2, c.gq.tmp, c.fs_ck, c.fs_ck2, c.fs_pos,
                     c.fs_perm, c.fs_v, c.fs_k};
     for (void *p : ptrs)
@@ -381,7 +380,6 @@ size_t ctx_device_bytes(const Ctx &c) {
     b += near_list_entries(c.cap) * 12;                              // near-field lists
     b += walk_max_groups(c.cap, c.pp_gather) * (PL_PAGES + 2) * (size_t)4; // their pages, left walks
     b += (size_t)c.lw_blocks * (c.lw_cap * (size_t)32 + 96);             // list walk
-    b += particle_waves(c.cap) * (NB_CAP + 1) * 4;                   // neighbour-walk leaves
     b += nn * 4;                                                     // wave h-solve queue
     b += nn * (5 * 4 + 1) + nn * (size_t)c.pp_limit * 4;    // ints, active, neighbour rows
     b += (((size_t)c.cap + 255) / 256) * 4 * HL_SLOTS * WAVE * 4;   // h-solve lists
@@ -494,7 +492,7 @@ int pin_reserve(Ctx &c, size_t bytes) {
 
 // host -> device on the context's stream; src may be reused on return
 int up_bytes(Ctx &c, const void *src, void *dst, size_t bytes) {
-    SX_TRY(pin_reserve(c, bytes));
+    SX_TRY(pin_reserve(c, std::min(bytes, 4 * PIN_PIECE)));
     const char *h = static_cast<const char *>(src);
     char *d = static_cast<char *>(dst);
     while (bytes > 0) {

@@ -87,8 +87,7 @@ constexpr int LW_ALONE = 393216;
 constexpr int LW_ORDERED = 6144;
 constexpr int LW_BUDGET = 8192;
 constexpr int LW_CAP = 8192;
-// leaves a wave of the neighbour walk records for the rows of its particles
-// above pp_limit (a longer list makes such a particle walk the tree alone)
+// largest value of SERENX_TUNE_NEIB_LEAVES
 constexpr int NB_CAP = 512;
 
 // Counters that every wave of a launch updates (walk statistics, interaction
@@ -340,9 +339,6 @@ struct Ctx {
     size_t ovf_cap = 0;
     int *ovf_count = nullptr;     // device scalar: number of overflow particles
     int *ovf_idx = nullptr;       // the overflow particles, in tree order
-    // leaves each wave of the neighbour walk opened (NB_CAP per wave of 64
-    // particles, in DFS order) and their number, for the overflow rows
-    int *nbl = nullptr, *nbl_len = nullptr;
     // particles the lane h solve leaves to the wave solve, and their number
     int *hq = nullptr, *hq_len = nullptr;
 
@@ -369,7 +365,7 @@ struct Ctx {
     int walk_queue = 64;             // SERENX_TUNE_WALK_QUEUE: blocks per CU (0: no queue)
     int pair_blocks = 0;             // SERENX_TUNE_PAIR_BLOCKS: pair phase's (0: walk_queue's)
     int near_cap = PL_CAP;           // SERENX_TUNE_NEAR_CAP: near-list leaves a group may store
-    int nb_cap = NB_CAP;             // SERENX_TUNE_NEIB_LEAVES: leaves a neighbour-walk wave records
+    int nb_cap = NB_CAP;             // SERENX_TUNE_NEIB_LEAVES: kept, of no effect
     bool walk_alone = false;         // no SPH kernels run beside the walk (gravity only)
     int ncu = 1;                     // compute units of the device
 
@@ -473,8 +469,6 @@ inline size_t walk_max_groups(int n, int pp_gather) {
 }
 // near-list slots of a context for n particles: PL_CAP for each group of a
 // single cloud (at most n / 64 + 1 groups)
-// waves of a one-thread-per-particle launch over n particles
-inline size_t particle_waves(int n) { return (((size_t)n + 255) / 256) * 4; }
 inline size_t near_list_entries(int n) { return (((size_t)n + WAVE - 1) / WAVE + 1) * PL_CAP; }
 static_assert(PL_CAP % PL_PAGE == 0, "whole pages");
 

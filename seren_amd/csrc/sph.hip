@@ -421,9 +421,11 @@ __device__ __forceinline__ int wave_prefix(int v, int lane) {
 // WS_CAP is cut: resume then names the first node left out (another call
 // continues there), else it is -1.  Every call moves resume on or ends the
 // search: the node it starts at is expanded until it is a leaf or fails.
-template <class Test>
+// keep(e, node) is called for entry e of the list by the lane that writes it.
+template <class Test, class Keep>
 __device__ __forceinline__ int wave_leaves(WaveSearch &L, const BNode *__restrict__ bn, int root,
-                                           int &resume, unsigned &visits, Test &&test) {
+                                           int &resume, unsigned &visits, Test &&test,
+                                           Keep &&keep) {
     const int lane = (int)(threadIdx.x & (WAVE - 1));
     int len = 0, cur = 0;
     if (resume == root) {
@@ -496,15 +498,23 @@ __device__ __forceinline__ int wave_leaves(WaveSearch &L, const BNode *__restric
     for (int e = lane; e < len; e += WAVE) {
         const BNode &nd = bn[~L.front[cur][e]];
         L.leaf[e] = (nd.fc << 4) | nd.k;
+        keep(e, nd);
     }
     wave_lds_fence();
     return len;
 }
 
+template <class Test>
+__device__ __forceinline__ int wave_leaves(WaveSearch &L, const BNode *__restrict__ bn, int root,
+                                           int &resume, unsigned &visits, Test &&test) {
+    return wave_leaves(L, bn, root, resume, visits, test, [](int, const BNode &) {});
+}
+
 // Calls use(j, record, ok) for the particles of the leaves found, 64 slots
 // at a time in list order: 8 leaves, lane l the particle l & 7 of leaf l >> 3
 // (ok: that particle exists).  The loads of four batches are in flight
-// together.  use returns true to stop.
+// together.  use(j, record, ok, e) has the list entry e too, and returns true to
+// stop.
 template <class Use>
 __device__ __forceinline__ void wave_candidates(const WaveSearch &L, int nleaf,
                                                 const double4 *__restrict__ rec, int p,
@@ -525,7 +535,7 @@ __device__ __forceinline__ void wave_candidates(const WaveSearch &L, int nleaf,
         }
 #pragma unroll
         for (int u = 0; u < U; u++)
-            if (e0 + 8 * u < nleaf && use(j[u], a[u], ok[u])) return;
+            if (e0 + 8 * u < nleaf && use(j[u], a[u], ok[u], e0 + 8 * u + sub)) return;
     }
 }
 
@@ -669,7 +679,7 @@ __global__ void __launch_bounds__(256) k_hsolve_wave(
             bool decided = bisecting && srho >= enough;
             if (!decided) {
                 sweep(kg.range * hp, complete, [&](int m) {
-                    wave_candidates(L, m, rec, p, [&](int j, const double4 &a, bool ok) {
+                    wave_candidates(L, m, rec, p, [&](int j, const double4 &a, bool ok, int) {
                         // :214-231
                         const double ex = a.x - rpx, ey = a.y - rpy, ez = a.z - rpz;
                         const double dsq = ex * ex + ey * ey + ez * ez;
@@ -737,7 +747,7 @@ __global__ void __launch_bounds__(256) k_hsolve_wave(
         double szeta = mp * invhp * invhp * wg[0];
         const bool from_list = complete && !(box && kg.range * hp > kg.range * h_high);
         sweep(kg.range * hp, from_list, [&](int m) {
-            wave_candidates(L, m, rec, p, [&](int j, const double4 &a, bool ok) {
+            wave_candidates(L, m, rec, p, [&](int j, const double4 &a, bool ok, int) {
                 const double ex = a.x - rpx, ey = a.y - rpy, ez = a.z - rpz;
                 const double dsq = ex * ex + ey * ey + ez * ez;
                 const double drmag = sqrt(dsq) + SMALL_NUMBER;
@@ -816,8 +826,7 @@ __global__ void __launch_bounds__(256) k_neib(KGeom kg, bool box, int n, const i
                                               const int *__restrict__ ovf_off,
                                               int *__restrict__ ovf_list,
                                               int *__restrict__ ovf_count,
-                                              unsigned long long *__restrict__ wstat,
-                                              int *__restrict__, int *__restrict__, int) {
+                                              unsigned long long *__restrict__ wstat) {
     // the overflow pass runs over the list of overflow particles (n of them),
     // OVF_PER_WAVE to a wave: their walks are long, and a wave walks the union
     // of its lanes' walks, so a few lanes per wave keep many waves in flight
@@ -879,211 +888,30 @@ __global__ void __launch_bounds__(256) k_neib(KGeom kg, bool box, int n, const i
     if (!OVERFLOW_PASS) wave_stats(wstat, 8, vis, lvis);
 }
 
-// The cell test of the group neighbour walk for one lane (own: the cell is in
-// the lane's cloud).  With fresh boxes, the box test at the larger of the two
-// radii alone: every neighbour j of p in the cell's subtree lies in the box
-// and within max(KERNRANGE h_p, hrangemax) of p, so the cells it passes are
-// a superset of those holding neighbours.  With stale boxes,
-// BHhydro_walk.F90:36-43 for this lane.
-__device__ __forceinline__ bool neib_pass(const HNode &nd, bool box, bool own, double R,
-                                          double rpx, double rpy, double rpz) {
-    const double dx = nd.r[0] - rpx, dy = nd.r[1] - rpy, dz = nd.r[2] - rpz;
-    if (box) {
-        const double Rb = fmax(R, nd.hrangemax);
-        return own && box_dist2(nd, dx, dy, dz) <= Rb * Rb * (1.0 + 1.0e-12);
-    }
-    const double drsqd = dx * dx + dy * dy + dz * dz;
-    const double m1 = (R + nd.rmax) * (R + nd.rmax);
-    const double m2 = (nd.hrangemax + nd.rmax) * (nd.hrangemax + nd.rmax);
-    return own && (drsqd <= m1 || drsqd <= m2);
-}
-
-// The complete row of overflow particle p from the leaves its first-pass
-// wave (particles 64 g .. 64 g + 63) opened, in DFS order: lane l takes
-// leaf e0 + l, applies p's own cell test and the pair test to its
-// particles, and the lanes' matches are placed by a prefix sum of their
-// counts, so the row holds the candidates in leaf order and, within a leaf,
-// in particle order -- the order of p's own walk.  The recorded leaves
-// include every leaf p's own test passes (the test of a leaf implies the
-// test of each ancestor, so the wave reached it through p's own path), and
-// only those pass here: the row is the one the walk would write.
-__device__ void neib_ovf_scan(KGeom kg, bool box, int p, int g, int nl,
-                              const int *__restrict__ nbl, const HNode *__restrict__ hn,
-                              const double4 *__restrict__ rec, const int *__restrict__ cid,
-                              const int2 *__restrict__ root_range, const int *__restrict__ pptot,
-                              const int *__restrict__ ovf_off, int *__restrict__ ovf_list) {
-    const int lane = (int)(threadIdx.x & (WAVE - 1));
-    const double4 a = rec[p];
-    const double rpx = a.x, rpy = a.y, rpz = a.z, hp = a.w;
-    const double hrangesqd_p = kg.rangesqd * hp * hp;
-    const double R = kg.range * hp;
-    const int2 rr = root_range[cid[p]];
-    int *row = ovf_list + ovf_off[p];
-    const int lim = pptot[p];
-    int base = 0;
-    for (int e0 = 0; e0 < nl; e0 += WAVE) {
-        const int e = e0 + lane;
-        unsigned hit = 0;   // bit i: particle i of the lane's leaf is a neighbour
-        int first = 0, cnt = 0;
-        if (e < nl) {
-            const int c = nbl[(size_t)g * NB_CAP + e];
-            const HNode nd = hn[c];
-            if (nd.leaf > 0 && neib_pass(nd, box, c >= rr.x && c < rr.y, R, rpx, rpy, rpz)) {
-                first = nd.first;
-                for (int i = 0; i < nd.leaf; i++) {
-                    const int j = first + i;
-                    if (j == p) continue;
-                    const double4 aj = rec[j];
-                    const double hrangesqd_pp = kg.rangesqd * aj.w * aj.w;
-                    const double qx = aj.x - rpx, qy = aj.y - rpy, qz = aj.z - rpz;
-                    const double dsq = qx * qx + qy * qy + qz * qz;
-                    if (dsq <= hrangesqd_p || dsq <= hrangesqd_pp) {
-                        hit |= 1u << i;
-                        cnt++;
-                    }
-                }
-            }
-        }
-        int incl = cnt;   // inclusive prefix sum over the lanes
-        for (int d = 1; d < WAVE; d <<= 1) {
-            const int u = __shfl_up(incl, d, WAVE);
-            if (lane >= d) incl += u;
-        }
-        int o = base + incl - cnt;
-        for (int i = 0; hit != 0; i++, hit >>= 1)
-            if (hit & 1u) {
-                if (o < lim) row[o] = first + i;
-                o++;
-            }
-        base += __shfl(incl, WAVE - 1, WAVE);
-    }
-}
-
-// get_neib.F90:46-118 with one walk per wave instead of one per particle.
-// Every particle j with r^2 <= KERNRANGESQD h_p^2 or r^2 <= KERNRANGESQD
-// h_j^2 lies in a leaf that the reference's BHhydro_walk opens for p: every
-// ancestor's bounding sphere holds j, so |r_p - r_c| <= |r_p - r_j| + rmax_c,
-// and hrangemax_c >= KERNRANGE h_j.  The reference keeps exactly those
-// particles, in DFS order.  Any walk that opens a superset of those leaves,
-// in DFS order, therefore yields the reference's lists once each candidate
-// passes the reference's pair test (formed as get_neib.F90:89-95 forms it).
-// This walk visits a cell's children when any lane's own test of
-// BHhydro_walk.F90:36-43 (and, with fresh boxes, the box test) passes the
-// cell, so every cell on any lane's own path is visited; a lane takes the
-// candidates of the leaves its own test passes.  Unlike group_walk it keeps
-// no per-lane resume state: the visit is one test per lane and a ballot.
-template <bool OVERFLOW_PASS>
-__global__ void __launch_bounds__(256) k_neib_group(KGeom kg, bool box, int n,
-                                                    const int *__restrict__ ovf_idx, int nc,
-                                                    const HNode *__restrict__ hn,
-                                                    const double4 *__restrict__ rec,
-                                                    const int *__restrict__ cid,
-                                                    const int2 *__restrict__ root_range,
-                                                    const uint8_t *__restrict__ active,
-                                                    int pp_limit, int *__restrict__ pptot,
-                                                    int *__restrict__ pplist,
-                                                    const int *__restrict__ ovf_off,
-                                                    int *__restrict__ ovf_list,
-                                                    int *__restrict__ ovf_count,
-                                                    unsigned long long *__restrict__ wstat,
-                                                    int *__restrict__ nbl,
-                                                    int *__restrict__ nbl_len, int nb_cap) {
-    const int t = xcd_block() * blockDim.x + threadIdx.x;
-    const int wv = t / WAVE;
-    if (OVERFLOW_PASS) {
-        // one overflow particle per wave: from the leaf list of its
-        // first-pass wave when that list is complete, else by its own walk
-        if (wv >= n) return;
-        const int po = uniform(ovf_idx[wv]);
-        const int g = po / WAVE;
-        const int nl = uniform(nbl_len[g]);
-        if (nl <= nb_cap) {
-            neib_ovf_scan(kg, box, po, g, nl, nbl, hn, rec, cid, root_range, pptot, ovf_off,
-                          ovf_list);
-            return;
-        }
-    }
-    const int ot = (t / WAVE) * OVF_PER_WAVE + (t % WAVE);
-    const bool ovf_lane = (t % WAVE) < OVF_PER_WAVE && ot < n;
-    const int p = OVERFLOW_PASS ? (ovf_lane ? ovf_idx[ot] : 0) : t;
-    const bool valid = OVERFLOW_PASS ? ovf_lane : (p < n && active[p]);
-    double rpx = 0, rpy = 0, rpz = 0, hp = 0;
-    if (valid) {
-        const double4 a = rec[p];
-        rpx = a.x; rpy = a.y; rpz = a.z;
-        hp = a.w;
-    }
-    if (ballot(valid) == 0) return;
-    const double hrangesqd_p = kg.rangesqd * hp * hp;
-    const double R = kg.range * hp;
-    int tot = 0;
-    int *row = nullptr;
-    int lim = pp_limit;   // entries this lane may store
-    if (valid) {
-        row = OVERFLOW_PASS ? ovf_list + ovf_off[p] : pplist + (size_t)p * pp_limit;
-        if (OVERFLOW_PASS) lim = pptot[p];
-    }
-    const int2 rr = valid ? root_range[cid[p]] : make_int2(nc, nc);
-    int c = uniform(wave_min_int(rr.x));
-    const int cend = uniform(wave_max_int(valid ? rr.y : 0));
-    unsigned vis = 0, lvis = 0;
-    int nl = 0;   // leaves opened (wave-uniform), recorded for the overflow pass
-    while (c < cend) {
-        const HNode nd = hn[c];
-        vis++;
-        const bool pass = neib_pass(nd, box, valid && c >= rr.x && c < rr.y, R, rpx, rpy, rpz);
-        lvis += lanes(pass);
-        if (ballot(pass) == 0) {
-            c = nd.next;
-            continue;
-        }
-        if (nd.leaf == 0) {
-            c = c + 1;
-            continue;
-        }
-        if (!OVERFLOW_PASS) {
-            if ((threadIdx.x & (WAVE - 1)) == 0 && nl < nb_cap) nbl[(size_t)wv * NB_CAP + nl] = c;
-            nl++;
-        }
-        const int k = nd.leaf, f0 = nd.first;
-        for (int i = 0; i < k; i++) {
-            const int j = f0 + i;
-            const double4 aj = rec[j];   // one scalar load per candidate
-            if (!pass || j == p) continue;
-            const double hrangesqd_pp = kg.rangesqd * aj.w * aj.w;
-            const double qx = aj.x - rpx, qy = aj.y - rpy, qz = aj.z - rpz;
-            const double dsq = qx * qx + qy * qy + qz * qz;
-            if (dsq <= hrangesqd_p || dsq <= hrangesqd_pp) {
-                if (tot < lim) row[tot] = j;
-                tot++;
-            }
-        }
-        c = nd.next;
-    }
-    if (valid && !OVERFLOW_PASS) {
-        pptot[p] = tot;
-        if (tot > pp_limit) atomicAdd(ovf_count, 1);
-    }
-    if (!OVERFLOW_PASS) {
-        if ((threadIdx.x & (WAVE - 1)) == 0) nbl_len[wv] = nl;
-        wave_stats(wstat, 8, vis, lvis);
-    }
-}
-
 // a lane's value in scalar registers
 __device__ __forceinline__ double lane_value(double v, int from) {
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), from),
                             __builtin_amdgcn_readlane(__double2loint(v), from));
 }
 
-// The rows of k_neib_group from searches by whole waves, with fresh boxes: a
-// wave takes NW_T consecutive particles (one: a row above pp_limit).  The
-// leaves that can hold a neighbour of any of them -- their boxes lie within
-// max(KERNRANGE h_p, hrangemax) of a particle, k_neib_group's test -- come from
-// a front of 64 nodes at a time (wave_leaves), in DFS order; then 64
-// candidates at a time are put to each particle's pair test, and the matches
-// are placed by their rank among the lanes.  Same candidates in the same
-// order, so the same rows.
+// get_neib.F90:46-118 from searches by whole waves: a wave takes NW_T
+// consecutive particles (one: a row above pp_limit).
+//
+// Every particle j with r^2 <= KERNRANGESQD h_p^2 or r^2 <= KERNRANGESQD
+// h_j^2 lies in a leaf that the reference's BHhydro_walk opens for p: every
+// ancestor's bounding sphere holds j, so |r_p - r_c| <= |r_p - r_j| + rmax_c,
+// and hrangemax_c >= KERNRANGE h_j.  The reference keeps exactly those
+// particles, in DFS order.  Any search that finds a superset of those leaves,
+// in DFS order, therefore yields the reference's lists once each candidate
+// passes the reference's pair test (formed as get_neib.F90:89-95 forms it).
+//
+// The leaves that a particle's own cell test passes come from a front of 64
+// nodes at a time (wave_leaves), in DFS order: with fresh boxes, those whose
+// box lies within max(KERNRANGE h_p, hrangemax) of it; with stale ones,
+// BHhydro_walk.F90:36-43, and a particle takes the candidates of the leaves
+// that its own test passes.  64 candidates at a time are put to each
+// particle's pair test, and the matches are placed by their rank among the
+// lanes.
 //
 // Why: a wave that walks node by node for 64 particles needs 0.3 us per cell
 // and 0.1 us per candidate, one after the other: 275 us at 2,048 particles and
@@ -1094,7 +922,7 @@ __device__ __forceinline__ double lane_value(double v, int from) {
 // of the tree from opening all that lies between (1M: 17.8 ms).
 constexpr int NW_T = 8;
 
-template <bool OVERFLOW_PASS>
+template <bool OVERFLOW_PASS, bool BOX>
 __global__ void __launch_bounds__(256) k_neib_wave(
     KGeom kg, int n, const int *__restrict__ ovf_idx, const BNode *__restrict__ bn,
     const double4 *__restrict__ rec, const int *__restrict__ cid,
@@ -1104,6 +932,9 @@ __global__ void __launch_bounds__(256) k_neib_wave(
     constexpr int T = OVERFLOW_PASS ? 1 : NW_T;
     __shared__ WaveSearch lds[256 / WAVE];
     WaveSearch &L = lds[threadIdx.x / WAVE];
+    // stale boxes: per leaf found, the particles whose test passes it
+    __shared__ uint8_t pass_all[256 / WAVE][BOX ? 1 : WS_CAP];
+    uint8_t *passes = pass_all[threadIdx.x / WAVE];
     const int lane = (int)(threadIdx.x & (WAVE - 1));
     const int t0 = (xcd_block() * (256 / WAVE) + (int)(threadIdx.x / WAVE)) * T;
     if (t0 >= n) return;
@@ -1139,19 +970,35 @@ __global__ void __launch_bounds__(256) k_neib_wave(
         }
         int resume = root;
         do {
-            const int m = wave_leaves(L, bn, root, resume, vis, [&](const BNode &nd) {
-                bool pass = false;
+            // the particles (bit t) whose cell test passes a node
+            auto test = [&](const BNode &nd) -> unsigned {
+                unsigned pass = 0;
 #pragma unroll
                 for (int t = 0; t < T; t++) {
-                    const double ex = fmax(fabs(nd.r[0] - tx[t]) - (double)nd.half[0], 0.0);
-                    const double ey = fmax(fabs(nd.r[1] - ty[t]) - (double)nd.half[1], 0.0);
-                    const double ez = fmax(fabs(nd.r[2] - tz[t]) - (double)nd.half[2], 0.0);
-                    const double Rb = fmax(tr[t], nd.hrangemax);
-                    pass = pass || ex * ex + ey * ey + ez * ez <= Rb * Rb * (1.0 + 1.0e-12);
+                    const double dx = nd.r[0] - tx[t], dy = nd.r[1] - ty[t], dz = nd.r[2] - tz[t];
+                    bool ok;
+                    if (BOX) {
+                        const double ex = fmax(fabs(dx) - (double)nd.half[0], 0.0);
+                        const double ey = fmax(fabs(dy) - (double)nd.half[1], 0.0);
+                        const double ez = fmax(fabs(dz) - (double)nd.half[2], 0.0);
+                        const double Rb = fmax(tr[t], nd.hrangemax);
+                        ok = ex * ex + ey * ey + ez * ez <= Rb * Rb * (1.0 + 1.0e-12);
+                    } else {
+                        const double dsq = dx * dx + dy * dy + dz * dz;
+                        ok = dsq <= (tr[t] + nd.rmax) * (tr[t] + nd.rmax) ||
+                             dsq <= (nd.hrangemax + nd.rmax) * (nd.hrangemax + nd.rmax);
+                    }
+                    pass |= ok ? 1u << t : 0u;
                 }
                 return pass;
-            });
-            wave_candidates(L, m, rec, 0, [&](int j, const double4 &aj, bool ok) {
+            };
+            const int m = wave_leaves(
+                L, bn, root, resume, vis, [&](const BNode &nd) { return test(nd) != 0; },
+                [&](int e, const BNode &nd) {
+                    if (!BOX) passes[e] = (uint8_t)test(nd);
+                });
+            wave_candidates(L, m, rec, 0, [&](int j, const double4 &aj, bool ok, int e) {
+                const unsigned own = BOX || !ok ? ~0u : passes[e];
                 const double hrangesqd_pp = kg.rangesqd * aj.w * aj.w;
 #pragma unroll
                 for (int t = 0; t < T; t++) {
@@ -1159,7 +1006,8 @@ __global__ void __launch_bounds__(256) k_neib_wave(
                     const int p = OVERFLOW_PASS ? mine : t0 + t;
                     const double qx = aj.x - tx[t], qy = aj.y - ty[t], qz = aj.z - tz[t];
                     const double dsq = qx * qx + qy * qy + qz * qz;
-                    const bool hit = ok && j != p && (dsq <= th[t] || dsq <= hrangesqd_pp);
+                    const bool hit = ok && ((own >> t) & 1u) && j != p &&
+                                     (dsq <= th[t] || dsq <= hrangesqd_pp);
                     const unsigned long long hm = ballot(hit);
                     if (hm == 0) continue;
                     const int o = tot[t] + __popcll(hm & ((1ull << lane) - 1ull));
@@ -2018,28 +1866,23 @@ int sph_density(Ctx &c) {
 // pp_limit ids, every particle's count, and the number of particles above
 // pp_limit copied to pinned slot 9 (read by sph_neib_finish once the stream
 // has got there).
-// Neighbour rows by searches of whole waves (k_neib_wave), which need the boxes
-// of the current positions; with stale ones each lane's own sphere test of a
-// leaf decides what it takes, which k_neib_group has at hand.
-static bool neib_by_waves(const Ctx &c) { return c.neib_group && c.box_ok; }
-
 int sph_neib_rows(Ctx &c) {
     hipStream_t s = c.stream;
     double4 *rec = reinterpret_cast<double4 *>(c.hrec);
     // [0] x y z h with the solved h
     hipLaunchKernelGGL(k_pack_xyzh, dim3(nblk(std::max(c.n, c.nc))), dim3(TB), 0, s, c.n, c.x, c.y,
-                       c.z, c.h, rec, c.nc, c.bfs2dfs, c.hn, neib_by_waves(c) ? c.bn : nullptr);
+                       c.z, c.h, rec, c.nc, c.bfs2dfs, c.hn, c.neib_group ? c.bn : nullptr);
     SX_TRY(zero_words(c.ovf_count, 1, s));
-    if (neib_by_waves(c)) {
-        hipLaunchKernelGGL(k_neib_wave<false>, dim3(nblk((c.n + NW_T - 1) / NW_T, 256 / WAVE)),
+    if (c.neib_group) {
+        auto k = c.box_ok ? k_neib_wave<false, true> : k_neib_wave<false, false>;
+        hipLaunchKernelGGL(k, dim3(nblk((c.n + NW_T - 1) / NW_T, 256 / WAVE)),
                            dim3(256), 0, s, c.kg, c.n, c.ovf_idx, c.bn, rec, c.cid, c.active,
                            c.pp_limit, c.pptot, c.pplist, c.ovf_off, c.ovf_list, c.ovf_count,
                            c.wstat);
     } else {
-        hipLaunchKernelGGL(c.neib_group ? k_neib_group<false> : k_neib<false>, dim3(nblk(c.n)),
-                           dim3(TB), 0, s, c.kg, c.box_ok, c.n, c.ovf_idx, c.nc, c.hn, rec, c.cid,
-                           c.root_range, c.active, c.pp_limit, c.pptot, c.pplist, c.ovf_off,
-                           c.ovf_list, c.ovf_count, c.wstat, c.nbl, c.nbl_len, c.nb_cap);
+        hipLaunchKernelGGL(k_neib<false>, dim3(nblk(c.n)), dim3(TB), 0, s, c.kg, c.box_ok, c.n,
+                           c.ovf_idx, c.nc, c.hn, rec, c.cid, c.root_range, c.active, c.pp_limit,
+                           c.pptot, c.pplist, c.ovf_off, c.ovf_list, c.ovf_count, c.wstat);
     }
     SX_HIP(hipGetLastError());
     SX_HIP(hipMemcpyAsync(c.hostpin + 9, c.ovf_count, sizeof(int), hipMemcpyDeviceToHost, s));
@@ -2087,18 +1930,18 @@ int sph_neib_finish(Ctx &c) {
                 return set_error(SERENX_ENOMEM, "hipMalloc failed for overflow neighbour lists");
         }
         const int nov = c.hostpin[9];   // overflow particles, counted by k_neib<false>
-        const long ovf_threads = (long)((nov + OVF_PER_WAVE - 1) / OVF_PER_WAVE) * WAVE;
-        if (neib_by_waves(c)) {
-            hipLaunchKernelGGL(k_neib_wave<true>, dim3(nblk(nov, 256 / WAVE)), dim3(256), 0, s,
-                               c.kg, nov, c.ovf_idx, c.bn, rec, c.cid, c.active, c.pp_limit,
-                               c.pptot, c.pplist, c.ovf_off, c.ovf_list, c.ovf_count, c.wstat);
-            SX_HIP(hipGetLastError());
-            return SERENX_OK;
+        if (c.neib_group) {
+            auto k = c.box_ok ? k_neib_wave<true, true> : k_neib_wave<true, false>;
+            hipLaunchKernelGGL(k, dim3(nblk(nov, 256 / WAVE)), dim3(256), 0, s, c.kg, nov,
+                               c.ovf_idx, c.bn, rec, c.cid, c.active, c.pp_limit, c.pptot,
+                               c.pplist, c.ovf_off, c.ovf_list, c.ovf_count, c.wstat);
+        } else {
+            const long threads = (long)((nov + OVF_PER_WAVE - 1) / OVF_PER_WAVE) * WAVE;
+            hipLaunchKernelGGL(k_neib<true>, dim3(nblk(threads)), dim3(TB), 0, s, c.kg, c.box_ok,
+                               nov, c.ovf_idx, c.nc, c.hn, rec, c.cid, c.root_range, c.active,
+                               c.pp_limit, c.pptot, c.pplist, c.ovf_off, c.ovf_list, c.ovf_count,
+                               c.wstat);
         }
-        hipLaunchKernelGGL(c.neib_group ? k_neib_group<true> : k_neib<true>, dim3(nblk(ovf_threads)), dim3(TB), 0, s, c.kg, c.box_ok, nov, c.ovf_idx, c.nc,
-                           c.hn, rec, c.cid, c.root_range, c.active, c.pp_limit,
-                           c.pptot, c.pplist, c.ovf_off, c.ovf_list, c.ovf_count, c.wstat,
-                           c.nbl, c.nbl_len, c.nb_cap);
         SX_HIP(hipGetLastError());
     }
     return SERENX_OK;

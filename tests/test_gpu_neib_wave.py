@@ -33,3 +33,26 @@ def test_rows_equal_the_walks(sizes, profile):
             eng.close()
     for key in got[0]:
         assert np.array_equal(got[0][key], got[1][key]), key
+
+
+@pytest.mark.parametrize("n,profile", [(58, "uniform"), (71, "r2"), (2053, "plummer")])
+def test_rows_equal_the_walks_on_a_tree_stocked_before(n, profile):
+    """The drop-in drivers cannot know whether the host moved its particles since
+    the tree was stocked: there each particle's own sphere test decides."""
+    from seren_amd import engine as sx
+    pos, vel, mass, h = cloud(n, profile, 80)
+    got = []
+    for group in (1, 0):
+        print(f"case {n} {profile} group {group}", flush=True)
+        eng = sx.ForceEngine(multipole="quadrupole", mac="geometric", sound_speed=CS)
+        try:
+            eng.set_tuning(sx.TUNE_NEIB_GROUP, group)
+            st = sx.SerenState(pos, vel, mass, np.full(n, 0.2) if h is None else h, eng.pp_limit)
+            sx.tree_update(eng, st)
+            st.parray[:, :3] += 1e-3 * np.random.default_rng(1).standard_normal((n, 3))
+            sx.sph_update(eng, st)
+            got.append((st.parray.copy(), st.pptot.copy(), st.pplist.copy(), st.rho.copy()))
+        finally:
+            eng.close()
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
