@@ -2009,14 +2009,15 @@ int pair_cap(const Ctx &c) {
 
 // Blocks of a walk launch that has `groups` groups per block at a time: as many
 // as the device holds at once and at most cap per CU, where the knob counts
-// blocks of TB threads.
+// blocks of TB threads (rounded up to whole blocks: at 3 of them the pair phase
+// of a 1M step keeps 16 waves a CU, with 8 it held the step back by 0.4 ms).
 template <class K>
 int walk_blocks(Ctx &c, K kernel, int cap, int tb, int groups = 1) {
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, tb, 0) != hipSuccess ||
         per_cu <= 0)
         per_cu = 1;
-    if (c.walk_queue != 0) per_cu = std::min(per_cu, std::max(1, cap * TB / tb));
+    if (c.walk_queue != 0) per_cu = std::min(per_cu, (cap * TB + tb - 1) / tb);
     return std::max(1, std::min((c.gq.ngroups + groups - 1) / groups, per_cu * c.ncu));
 }
 

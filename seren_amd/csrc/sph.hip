@@ -1063,6 +1063,80 @@ __global__ void __launch_bounds__(256) k_neib_wave(
     }
 }
 
+// The same rows by one walk per wave of 64 particles, for large clouds with
+// fresh boxes: it visits a cell's children when the box test at any lane's
+// larger radius passes the cell, and a lane takes the candidates of the
+// leaves its own test passes.  Slower alone in small clouds (275 against 40 us at
+// 2,048 particles) and equal at 300,007, but 5.7e8 instead of 7.2e8 VALU
+// instructions at 1M, where the walk's pair phase beside it wants the same
+// units: 3.9 against 4.8 ms there, so clouds above NEIB_WAVE_MAX particles take it.
+constexpr int NEIB_WAVE_MAX = 1 << 18;
+
+__global__ void __launch_bounds__(256) k_neib_group(KGeom kg, int n, int nc,
+                                                    const HNode *__restrict__ hn,
+                                                    const double4 *__restrict__ rec,
+                                                    const int *__restrict__ cid,
+                                                    const int2 *__restrict__ root_range,
+                                                    const uint8_t *__restrict__ active,
+                                                    int pp_limit, int *__restrict__ pptot,
+                                                    int *__restrict__ pplist,
+                                                    int *__restrict__ ovf_count,
+                                                    unsigned long long *__restrict__ wstat) {
+    const int p = xcd_block() * blockDim.x + threadIdx.x;
+    const bool valid = p < n && active[p];
+    if (ballot(valid) == 0) return;
+    double rpx = 0, rpy = 0, rpz = 0, hp = 0;
+    if (valid) {
+        const double4 a = rec[p];
+        rpx = a.x; rpy = a.y; rpz = a.z;
+        hp = a.w;
+    }
+    const double hrangesqd_p = kg.rangesqd * hp * hp;
+    const double R = kg.range * hp;
+    int tot = 0;
+    int *row = pplist + (size_t)(valid ? p : 0) * pp_limit;
+    const int2 rr = valid ? root_range[cid[p]] : make_int2(nc, nc);
+    int c = uniform(wave_min_int(rr.x));
+    const int cend = uniform(wave_max_int(valid ? rr.y : 0));
+    unsigned vis = 0, lvis = 0;
+    while (c < cend) {
+        const HNode nd = hn[c];
+        vis++;
+        const double Rb = fmax(R, nd.hrangemax);
+        const bool pass = valid && c >= rr.x && c < rr.y &&
+                          box_dist2(nd, nd.r[0] - rpx, nd.r[1] - rpy, nd.r[2] - rpz) <=
+                              Rb * Rb * (1.0 + 1.0e-12);
+        lvis += lanes(pass);
+        if (ballot(pass) == 0) {
+            c = nd.next;
+            continue;
+        }
+        if (nd.leaf == 0) {
+            c = c + 1;
+            continue;
+        }
+        const int k = nd.leaf, f0 = nd.first;
+        for (int i = 0; i < k; i++) {
+            const int j = f0 + i;
+            const double4 aj = rec[j];   // one scalar load per candidate
+            if (!pass || j == p) continue;
+            const double hrangesqd_pp = kg.rangesqd * aj.w * aj.w;
+            const double qx = aj.x - rpx, qy = aj.y - rpy, qz = aj.z - rpz;
+            const double dsq = qx * qx + qy * qy + qz * qz;
+            if (dsq <= hrangesqd_p || dsq <= hrangesqd_pp) {
+                if (tot < pp_limit) row[tot] = j;
+                tot++;
+            }
+        }
+        c = nd.next;
+    }
+    if (valid) {
+        pptot[p] = tot;
+        if (tot > pp_limit) atomicAdd(ovf_count, 1);
+    }
+    wave_stats(wstat, 8, vis, lvis);
+}
+
 __global__ void k_ovf_sizes(int n, int pp_limit, const int *__restrict__ pptot,
                             const uint8_t *__restrict__ active, int *__restrict__ sz,
                             int *__restrict__ is_ovf) {
@@ -1900,7 +1974,11 @@ int sph_neib_rows(Ctx &c) {
     hipLaunchKernelGGL(k_pack_xyzh, dim3(nblk(std::max(c.n, c.nc))), dim3(TB), 0, s, c.n, c.x, c.y,
                        c.z, c.h, rec, c.nc, c.bfs2dfs, c.hn, c.neib_group ? c.bn : nullptr);
     SX_TRY(zero_words(c.ovf_count, 1, s));
-    if (c.neib_group) {
+    if (c.neib_group && c.box_ok && c.n > NEIB_WAVE_MAX) {
+        hipLaunchKernelGGL(k_neib_group, dim3(nblk(c.n)), dim3(TB), 0, s, c.kg, c.n, c.nc, c.hn, rec,
+                           c.cid, c.root_range, c.active, c.pp_limit, c.pptot, c.pplist,
+                           c.ovf_count, c.wstat);
+    } else if (c.neib_group) {
         auto k = c.box_ok ? k_neib_wave<false, true> : k_neib_wave<false, false>;
         hipLaunchKernelGGL(k, dim3(nblk((c.n + NW_T - 1) / NW_T, 256 / WAVE)),
                            dim3(256), 0, s, c.kg, c.n, c.ovf_idx, c.bn, rec, c.cid, c.active,
