@@ -425,15 +425,24 @@ __device__ __forceinline__ int wave_prefix(int v, int lane) {
 // WS_CAP is cut: resume then names the first node left out (another call
 // continues there), else it is -1.  Every call moves resume on or ends the
 // search: the node it starts at is expanded until it is a leaf or fails.
-// keep(e, node) is called for entry e of the list by the lane that writes it.
-template <class Test, class Keep>
-__device__ __forceinline__ int wave_leaves(WaveSearch &L, const BNode *__restrict__ bn, int root,
-                                           int &resume, unsigned &visits, Test &&test,
-                                           Keep &&keep) {
+//
+// MASKED: a search for several particles, whose tests of a node are the bits
+// of test().  masks holds, beside the two fronts, the particles that passed
+// every ancestor of an entry: a leaf's test does not imply its ancestors'
+// (its sphere need not lie within theirs), so the particles that open it are
+// those of its entry's mask and its own test.  They are left in
+// masks[0 .. number of leaves).  all: the particles searched for.
+template <bool MASKED, class Test>
+__device__ __forceinline__ int wave_leaves(WaveSearch &L, uint8_t *masks, unsigned all,
+                                           const BNode *__restrict__ bn, int root, int &resume,
+                                           unsigned &visits, Test &&test) {
     const int lane = (int)(threadIdx.x & (WAVE - 1));
     int len = 0, cur = 0;
     if (resume == root) {
-        if (lane == 0) L.front[0][0] = root;
+        if (lane == 0) {
+            L.front[0][0] = root;
+            if (MASKED) masks[0] = (uint8_t)all;
+        }
         len = 1;
     } else {
         // the rest of the tree in DFS order: resume and its later siblings,
@@ -447,6 +456,17 @@ __device__ __forceinline__ int wave_leaves(WaveSearch &L, const BNode *__restric
             c = p + 1;
             p = bn[p].parent;
         }
+        if (MASKED) {   // their ancestors' tests again, one entry per lane
+            wave_lds_fence();
+            for (int e = lane; e < len; e += WAVE) {
+                unsigned mk = all;
+                for (int a = bn[L.front[0][e]].parent;; a = bn[a].parent) {
+                    mk &= test(bn[a]);
+                    if (a == root) break;
+                }
+                masks[e] = (uint8_t)mk;
+            }
+        }
     }
     resume = -1;
     bool branches = true;
@@ -459,15 +479,18 @@ __device__ __forceinline__ int wave_leaves(WaveSearch &L, const BNode *__restric
         for (int base = 0; base < len; base += WAVE) {
             const int e = base + lane;
             int v = 0, nout = 0, first = 0;   // a leaf that passed is kept as ~id
+            unsigned mk = 0;
             bool branch = false;
             if (e < len) {
                 v = in[e];
+                if (MASKED) mk = masks[cur * WS_CAP + e];
                 if (v < 0) {
                     nout = 1;
                     first = v;
                 } else {
                     const BNode nd = bn[v];
-                    if (test(nd)) {
+                    mk = MASKED ? mk & test(nd) : (unsigned)test(nd);
+                    if (mk) {
                         branch = nd.k < 0;
                         nout = branch ? -nd.k : 1;
                         first = branch ? nd.fc : ~v;
@@ -480,10 +503,10 @@ __device__ __forceinline__ int wave_leaves(WaveSearch &L, const BNode *__restric
             const int cutlane = over ? __ffsll((long long)over) - 1 : WAVE;
             if (lane < cutlane) {
                 const int o = out + incl - nout;
-                if (branch)
-                    for (int i = 0; i < nout; i++) dst[o + i] = first + i;
-                else if (nout)
-                    dst[o] = first;
+                for (int i = 0; i < nout; i++) {
+                    dst[o + i] = first + i;
+                    if (MASKED) masks[(cur ^ 1) * WS_CAP + o + i] = (uint8_t)mk;
+                }
             }
             branches = branches || ballot(branch && lane < cutlane) != 0;
             if (over) {
@@ -502,7 +525,7 @@ __device__ __forceinline__ int wave_leaves(WaveSearch &L, const BNode *__restric
     for (int e = lane; e < len; e += WAVE) {
         const BNode &nd = bn[~L.front[cur][e]];
         L.leaf[e] = (nd.fc << 4) | nd.k;
-        keep(e, nd);
+        if (MASKED) masks[e] = masks[cur * WS_CAP + e];
     }
     wave_lds_fence();
     return len;
@@ -511,7 +534,7 @@ __device__ __forceinline__ int wave_leaves(WaveSearch &L, const BNode *__restric
 template <class Test>
 __device__ __forceinline__ int wave_leaves(WaveSearch &L, const BNode *__restrict__ bn, int root,
                                            int &resume, unsigned &visits, Test &&test) {
-    return wave_leaves(L, bn, root, resume, visits, test, [](int, const BNode &) {});
+    return wave_leaves<false>(L, nullptr, 0u, bn, root, resume, visits, test);
 }
 
 // Calls use(j, record, ok) for the particles of the leaves found, 64 slots
@@ -932,13 +955,16 @@ __device__ __forceinline__ double lane_value(double v, int from) {
 // in DFS order, therefore yields the reference's lists once each candidate
 // passes the reference's pair test (formed as get_neib.F90:89-95 forms it).
 //
-// The leaves that a particle's own cell test passes come from a front of 64
-// nodes at a time (wave_leaves), in DFS order: with fresh boxes, those whose
-// box lies within max(KERNRANGE h_p, hrangemax) of it; with stale ones,
-// BHhydro_walk.F90:36-43, and a particle takes the candidates of the leaves
-// that its own test passes.  64 candidates at a time are put to each
-// particle's pair test, and the matches are placed by their rank among the
-// lanes.
+// The leaves come from a front of 64 nodes at a time (wave_leaves), in DFS
+// order.  With fresh boxes, those whose box lies within max(KERNRANGE h_p,
+// hrangemax) of any of the particles: that box holds every neighbour in it.
+// With stale ones (particles moved since the tree was stocked) a neighbour
+// can lie outside its leaf's and its leaf's ancestors' spheres, and the
+// reference's list is what its walk opens: each particle's path is followed
+// by itself (BHhydro_walk.F90:36-43 on the leaf and on all its ancestors), so
+// that the rows, and the counts of both passes, are those of its own walk.
+// 64 candidates at a time are put to each particle's pair test, and the
+// matches are placed by their rank among the lanes.
 //
 // Why: a wave that walks node by node for 64 particles needs 0.3 us per cell
 // and 0.1 us per candidate, one after the other: 275 us at 2,048 particles and
@@ -959,9 +985,11 @@ __global__ void __launch_bounds__(256) k_neib_wave(
     constexpr int T = OVERFLOW_PASS ? 1 : NW_T;
     __shared__ WaveSearch lds[256 / WAVE];
     WaveSearch &L = lds[threadIdx.x / WAVE];
-    // stale boxes: per leaf found, the particles whose test passes it
-    __shared__ uint8_t pass_all[256 / WAVE][BOX ? 1 : WS_CAP];
-    uint8_t *passes = pass_all[threadIdx.x / WAVE];
+    // the particles whose own walk opens a node, for several on stale boxes
+    constexpr bool MASKED = !BOX && T > 1;
+    static_assert(NW_T <= 8, "a mask is a byte");
+    __shared__ uint8_t masks_all[256 / WAVE][MASKED ? 2 * WS_CAP : 1];
+    uint8_t *masks = masks_all[threadIdx.x / WAVE];
     const int lane = (int)(threadIdx.x & (WAVE - 1));
     const int t0 = (xcd_block() * (256 / WAVE) + (int)(threadIdx.x / WAVE)) * T;
     if (t0 >= n) return;
@@ -1019,13 +1047,10 @@ __global__ void __launch_bounds__(256) k_neib_wave(
                 }
                 return pass;
             };
-            const int m = wave_leaves(
-                L, bn, root, resume, vis, [&](const BNode &nd) { return test(nd) != 0; },
-                [&](int e, const BNode &nd) {
-                    if (!BOX) passes[e] = (uint8_t)test(nd);
-                });
+            const int m =
+                wave_leaves<MASKED>(L, masks, (unsigned)im, bn, root, resume, vis, test);
             wave_candidates(L, m, rec, 0, [&](int j, const double4 &aj, bool ok, int e) {
-                const unsigned own = BOX || !ok ? ~0u : passes[e];
+                const unsigned own = MASKED && ok ? masks[e] : ~0u;
                 const double hrangesqd_pp = kg.rangesqd * aj.w * aj.w;
 #pragma unroll
                 for (int t = 0; t < T; t++) {
@@ -1060,6 +1085,8 @@ __global__ void __launch_bounds__(256) k_neib_wave(
             if (mytot > pp_limit) atomicAdd(ovf_count, 1);
         }
         wave_stats(wstat, 8, (vis + WAVE - 1) / WAVE, vis);
+    } else if (valid && mytot < pptot[mine]) {
+        pptot[mine] = mytot;   // a row's readers go as far as it was written
     }
 }
 
