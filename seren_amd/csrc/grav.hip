@@ -1718,6 +1718,7 @@ __device__ __forceinline__ void pairs_group_mixed(
             pair_f32(kg, t4, tp, valid && j != p, mact, a.x + ox, a.y + oy, a.z + oz, a.w, b.x,
                      b.y, b.z, b.w, bx, by, bz, bp, nin_p, nin_j);
         }
+        wave_lds_fence();   // the last leaf's sums take the stage's place
         out[0 * WAVE] = bx;
         out[1 * WAVE] = by;
         out[2 * WAVE] = bz;
@@ -1752,14 +1753,16 @@ __device__ __forceinline__ void pairs_group_mixed(
     const bool ordered = cloud_off[root + 1] - cloud_off[root] <= LW_ORDERED;
     if (ordered && len != NEAR_DROPPED) {
         // PM_LEAVES leaves per wave and round; their sums go to the four waves
-        // that add them in list order, one component each (px)
+        // that add them in list order, one component each (px).  The sums fill
+        // the waves' LDS; the leaves are staged where the last one's sums go
+        float4 *last = stage + (PM_LEAVES - 1) * WAVE;
         for (int r = 0; r < len; r += PM_WAVES * PM_LEAVES) {
             const int e0 = r + wave * PM_LEAVES, nb = max(0, min(PM_LEAVES, len - e0));
             int dl = 0;
             if (lane < nb) {
                 dl = near.leaf[near.slot(g, e0) + lane];   // in one page
                 const int f = dl >> 4, k = dl & 15;
-                float4 *dst = stage + 2 * LEAFMAX * lane;
+                float4 *dst = last + 2 * LEAFMAX * lane;
                 for (int i = 0; i < k; i++) {
                     dst[2 * i] = rec[2 * (size_t)(f + i)];
                     dst[2 * i + 1] = rec[2 * (size_t)(f + i) + 1];
@@ -1768,7 +1771,7 @@ __device__ __forceinline__ void pairs_group_mixed(
             wave_lds_fence();
             for (int e = 0; e < nb; e++) {
                 const int d = __builtin_amdgcn_readlane(dl, e);
-                leaf_sums(stage + 2 * LEAFMAX * e, d >> 4, d & 15,
+                leaf_sums(last + 2 * LEAFMAX * e, d >> 4, d & 15,
                           xsum + ((wave * PM_LEAVES + e) * 4) * WAVE + lane);
             }
             __syncthreads();
@@ -1881,10 +1884,12 @@ __global__ void __launch_bounds__(PM_TB) k_grav_pairs_mixed(
     // longest-first (by the previous walk's cost), as phase 1 takes them
     __builtin_amdgcn_s_setprio(2);
     // each wave's LDS stage: PL_STAGE leaves of LEAFMAX two-float4 records;
-    // in its place at the end, the waves' sums
+    // in its place the leaves' sums where they are added in list order, and the
+    // waves' sums at the end
     __shared__ float4 stage_all[PM_WAVES * PL_STAGE * LEAFMAX * 2];
     static_assert(sizeof(stage_all) >= sizeof(double) * 4 * PM_TB, "sums fit");
-    __shared__ float xsum[PM_WAVES * PM_LEAVES * 4 * WAVE];
+    static_assert(sizeof(stage_all) == sizeof(float) * PM_WAVES * PM_LEAVES * 4 * WAVE &&
+                      PM_LEAVES * LEAFMAX * 2 <= WAVE, "leaves' sums fit, their stage in one's");
     __shared__ int job;
     const int wave = uniform((int)(threadIdx.x / WAVE));
     float4 *stage = stage_all + wave * (PL_STAGE * LEAFMAX * 2);
@@ -1901,10 +1906,10 @@ __global__ void __launch_bounds__(PM_TB) k_grav_pairs_mixed(
         const int g = uniform(job);
         if (g < 0) break;
         pairs_group_mixed<MACT, QUINTIC>(g, wave, n, nc, gn, rec, stage,
-                                         reinterpret_cast<double *>(stage_all), xsum, cloud_off, x,
-                                         y, z, h, zeta,
-                                         cid, root_range, active, t4, ax, ay, az, cpot, gpot, agm,
-                                         near, icount, grp, ngrp, npp, nin_p, nin_j);
+                                         reinterpret_cast<double *>(stage_all),
+                                         reinterpret_cast<float *>(stage_all), cloud_off, x, y, z,
+                                         h, zeta, cid, root_range, active, t4, ax, ay, az, cpot,
+                                         gpot, agm, near, icount, grp, ngrp, npp, nin_p, nin_j);
     }
     if ((threadIdx.x & 63) == 0) {
         unsigned long long *ic = ctr_row(icount);
