@@ -1473,7 +1473,7 @@ __device__ __forceinline__ unsigned walk_budget(const LongWalks &lw, bool valid,
 
 template <int OCT, int MACT>
 __global__ void __launch_bounds__(256) k_grav_cells_fp64(
-    int n, int nc, const GNode *__restrict__ gn, const double *__restrict__ x,
+    int nc, const GNode *__restrict__ gn, const double *__restrict__ x,
     const double *__restrict__ y, const double *__restrict__ z, const int *__restrict__ cid,
     const int2 *__restrict__ root_range, const uint8_t *__restrict__ active,
     const double *__restrict__ gpot, const double *__restrict__ agm, double *__restrict__ cx,
@@ -1546,7 +1546,7 @@ __global__ void __launch_bounds__(256) k_grav_cells_fp64(
 
 template <int OCT, int MACT>
 __global__ void __launch_bounds__(256) k_grav_cells_mixed(
-    int n, int nc, const GNodeF *__restrict__ gn, const double *__restrict__ x,
+    int nc, const GNodeF *__restrict__ gn, const double *__restrict__ x,
     const double *__restrict__ y, const double *__restrict__ z, const int *__restrict__ cid,
     const int2 *__restrict__ root_range, const uint8_t *__restrict__ active,
     const double *__restrict__ gpot, const double *__restrict__ agm, double *__restrict__ ox,
@@ -1640,7 +1640,7 @@ constexpr int PM_TB = PM_WAVES * WAVE;
 
 template <int MACT, bool QUINTIC>
 __device__ __forceinline__ void pairs_group_mixed(
-    int g, int wave, int n, int nc, const GNodeF *__restrict__ gn, const float4 *__restrict__ rec,
+    int g, int wave, int nc, const GNodeF *__restrict__ gn, const float4 *__restrict__ rec,
     float4 *__restrict__ stage, double *__restrict__ sums, float *__restrict__ xsum,
     const int *__restrict__ cloud_off,
     const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
@@ -1649,9 +1649,8 @@ __device__ __forceinline__ void pairs_group_mixed(
     const uint8_t *__restrict__ active, const float4 *__restrict__ t4,
     double *__restrict__ ax, double *__restrict__ ay, double *__restrict__ az,
     const double *__restrict__ cpot, double *__restrict__ gpot, double *__restrict__ agm,
-    NearList near, unsigned long long *__restrict__ icount, const int2 *__restrict__ grp,
-    int ngrp,
-    unsigned &npp_out, unsigned &nin_p_out, unsigned &nin_j_out) {
+    NearList near, const int2 *__restrict__ grp, unsigned &npp_out, unsigned &nin_p_out,
+    unsigned &nin_j_out) {
     constexpr KGeom kg64 = walk_geom<QUINTIC>();
     constexpr KGeomF kg{(float)kg64.half, (float)kg64.range, (float)kg64.invrange};
     const int lane = (int)(threadIdx.x & (WAVE - 1));
@@ -1870,7 +1869,7 @@ __device__ __forceinline__ void pairs_group_mixed(
 
 template <int MACT, bool QUINTIC>
 __global__ void __launch_bounds__(PM_TB) k_grav_pairs_mixed(
-    int n, int nc, const GNodeF *__restrict__ gn, const float4 *__restrict__ rec,
+    int nc, const GNodeF *__restrict__ gn, const float4 *__restrict__ rec,
     const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
     const double *__restrict__ h, const double *__restrict__ zeta,
     const int *__restrict__ cid, const int2 *__restrict__ root_range,
@@ -1878,7 +1877,6 @@ __global__ void __launch_bounds__(PM_TB) k_grav_pairs_mixed(
     double *__restrict__ ax, double *__restrict__ ay, double *__restrict__ az,
     const double *__restrict__ cpot, double *__restrict__ gpot, double *__restrict__ agm,
     NearList near, unsigned long long *__restrict__ icount, const int2 *__restrict__ grp,
-    int ngrp,
     const int *__restrict__ cloud_off, GroupQueue queue) {
     // persistent over the walk's queue: the groups of each XCD range
     // longest-first (by the previous walk's cost), as phase 1 takes them
@@ -1905,11 +1903,10 @@ __global__ void __launch_bounds__(PM_TB) k_grav_pairs_mixed(
         __syncthreads();
         const int g = uniform(job);
         if (g < 0) break;
-        pairs_group_mixed<MACT, QUINTIC>(g, wave, n, nc, gn, rec, stage,
-                                         reinterpret_cast<double *>(stage_all),
-                                         reinterpret_cast<float *>(stage_all), cloud_off, x, y, z,
-                                         h, zeta, cid, root_range, active, t4, ax, ay, az, cpot,
-                                         gpot, agm, near, icount, grp, ngrp, npp, nin_p, nin_j);
+        pairs_group_mixed<MACT, QUINTIC>(
+            g, wave, nc, gn, rec, stage, reinterpret_cast<double *>(stage_all),
+            reinterpret_cast<float *>(stage_all), cloud_off, x, y, z, h, zeta, cid, root_range,
+            active, t4, ax, ay, az, cpot, gpot, agm, near, grp, npp, nin_p, nin_j);
     }
     if ((threadIdx.x & 63) == 0) {
         unsigned long long *ic = ctr_row(icount);
@@ -2056,13 +2053,13 @@ void launch_cells(Ctx &c, hipStream_t s, int cap) {
     const LongWalks lw{waves ? c.lw_group : nullptr, c.lw_at, cont, cont + 1, LW_BUDGET, LW_ALONE};
     if (waves && mixed) {
         auto kw = k_grav_cells_mixed<OCT, MACT>;
-        hipLaunchKernelGGL(kw, dim3(walk_blocks(c, kw, cap, TB, TB / WAVE)), dim3(TB), 0, s, c.n, c.nc, c.gnf,
+        hipLaunchKernelGGL(kw, dim3(walk_blocks(c, kw, cap, TB, TB / WAVE)), dim3(TB), 0, s, c.nc, c.gnf,
                            c.x, c.y, c.z, c.cid, c.root_range, c.active, c.gpot, c.agm, c.gax,
                            c.gay, c.gaz, c.gpc, near_list(c), c.icount, c.wstat, q, c.gq.cost,
                            c.grp, c.cloud_off, lw);
     } else if (waves) {
         auto kw = k_grav_cells_fp64<OCT, MACT>;
-        hipLaunchKernelGGL(kw, dim3(walk_blocks(c, kw, cap, TB, TB / WAVE)), dim3(TB), 0, s, c.n, c.nc, c.gn,
+        hipLaunchKernelGGL(kw, dim3(walk_blocks(c, kw, cap, TB, TB / WAVE)), dim3(TB), 0, s, c.nc, c.gn,
                            c.x, c.y, c.z, c.cid, c.root_range, c.active, c.gpot, c.agm, c.gax,
                            c.gay, c.gaz, c.gpc, near_list(c), c.icount, c.wstat, q, c.gq.cost,
                            c.grp, c.cloud_off, lw);
@@ -2096,11 +2093,11 @@ void launch_pairs(Ctx &c, const double4 *rec, hipStream_t s, int cap) {
     GroupQueue q{c.gq.ctr + NXCD, c.gq.order, c.gq.ngroups};
     if (c.opt.precision == SERENX_MIXED) {
         auto k = k_grav_pairs_mixed<MACT, QUINTIC>;
-        hipLaunchKernelGGL(k, dim3(walk_blocks(c, k, cap, PM_TB)), dim3(PM_TB), 0, s, c.n, c.nc,
-                           c.gnf, reinterpret_cast<const float4 *>(rec), c.x, c.y, c.z, c.h,
+        hipLaunchKernelGGL(k, dim3(walk_blocks(c, k, cap, PM_TB)), dim3(PM_TB), 0, s, c.nc, c.gnf,
+                           reinterpret_cast<const float4 *>(rec), c.x, c.y, c.z, c.h,
                            c.zeta, c.cid, c.root_range, c.active,
                            reinterpret_cast<const float4 *>(c.ktab + KT_G4F_OFF), c.gax, c.gay,
-                           c.gaz, c.gpc, c.gpot, c.agm, near_list(c), c.icount, c.grp, c.ngrp,
+                           c.gaz, c.gpc, c.gpot, c.agm, near_list(c), c.icount, c.grp,
                            c.cloud_off, q);
     } else {
         int least, most;

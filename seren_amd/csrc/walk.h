@@ -222,30 +222,19 @@ struct GroupQueue {
 
 __device__ __forceinline__ int queue_lo(int q, int ngroups) { return (q * ngroups + NXCD - 1) / NXCD; }
 
-// the next part of a group for the calling wave (wave-uniform): the queue
-// hands out PARTS parts of every group in turn.  Returns the group and its
-// part, -1 when none is left; q counts the ranges this wave has exhausted
-template <int PARTS>
-__device__ __forceinline__ int next_part(const GroupQueue &Q, int home, int &q, int &part) {
+// the next group of the calling wave (wave-uniform), -1 when none is left;
+// q counts the ranges this wave has exhausted
+__device__ __forceinline__ int next_group(const GroupQueue &Q, int home, int &q) {
     while (q < NXCD) {
         const int r = (home + q) % NXCD;
         const int lo = queue_lo(r, Q.ngroups), hi = queue_lo(r + 1, Q.ngroups);
         int t = 0;
         if ((threadIdx.x & 63) == 0) t = atomicAdd(Q.ctr + r, 1);
         t = uniform(__shfl(t, 0, 64));
-        if (lo + t / PARTS < hi) {
-            part = t % PARTS;
-            return Q.order[lo + t / PARTS];
-        }
+        if (lo + t < hi) return Q.order[lo + t];
         q++;
     }
     return -1;
-}
-
-// the next group of the calling wave (wave-uniform), -1 when none is left
-__device__ __forceinline__ int next_group(const GroupQueue &Q, int home, int &q) {
-    int part;
-    return next_part<1>(Q, home, q, part);
 }
 
 // Adds per-wave walk statistics into stats[k0], stats[k0 + 1] from lane 0:
