@@ -1636,9 +1636,8 @@ __global__ void __launch_bounds__(256) k_grav_cells_mixed(
 constexpr int PL_STAGE = 16;
 constexpr int PM_WAVES = 8;
 constexpr int PM_LEAVES = 4;   // leaves per wave and round of ordered sums
-constexpr int PM_TB = PM_WAVES * WAVE;
 
-template <int MACT, bool QUINTIC>
+template <int MACT, bool QUINTIC, int NW>
 __device__ __forceinline__ void pairs_group_mixed(
     int g, int wave, int nc, const GNodeF *__restrict__ gn, const float4 *__restrict__ rec,
     float4 *__restrict__ stage, double *__restrict__ sums, float *__restrict__ xsum,
@@ -1651,6 +1650,8 @@ __device__ __forceinline__ void pairs_group_mixed(
     const double *__restrict__ cpot, double *__restrict__ gpot, double *__restrict__ agm,
     NearList near, const int2 *__restrict__ grp, unsigned &npp_out, unsigned &nin_p_out,
     unsigned &nin_j_out) {
+    constexpr int SHARES = PM_WAVES / NW;   // a wave's, taken one after the other
+    static_assert(SHARES <= 2, "one share's sums held");
     constexpr KGeom kg64 = walk_geom<QUINTIC>();
     constexpr KGeomF kg{(float)kg64.half, (float)kg64.range, (float)kg64.invrange};
     const int lane = (int)(threadIdx.x & (WAVE - 1));
@@ -1671,6 +1672,7 @@ __device__ __forceinline__ void pairs_group_mixed(
         if (MACT != SERENX_MAC_GEOMETRIC) afactor = mac_afactor<MACT>(agm[p], gpot[p]);
     }
     CSum px, py, pz, pq;   // pair terms, one compensated addition per leaf
+    double held[4] = {0.0, 0.0, 0.0, 0.0};   // the first share's sums
     unsigned npp = 0, nin_p = 0, nin_j = 0;
     auto leaf_pairs = [&](int first, int count, bool mine) {
         // r_f - r_p in FP64, once per leaf (r_f: the leaf's first particle)
@@ -1750,12 +1752,63 @@ __device__ __forceinline__ void pairs_group_mixed(
     const int root =
         __builtin_amdgcn_readlane(valid ? cid[p] : 0, __ffsll((long long)ballot(valid)) - 1);
     const bool ordered = cloud_off[root + 1] - cloud_off[root] <= LW_ORDERED;
+    auto stored_pairs = [&](int share) {
+        // the near list in batches of PL_STAGE leaves: lane l copies the
+        // records of the batch's leaf l into the wave's LDS stage (all the
+        // batch's loads in flight at once), then the wave forms the pairs
+        // leaf by leaf in list order from LDS
+        for (int e0 = share * PL_STAGE; e0 < len; e0 += PM_WAVES * PL_STAGE) {
+            const int nb = min(PL_STAGE, len - e0);
+            const size_t at = near.slot(g, e0);   // a batch lies in one page
+            int dl = 0;
+            if (lane < nb) {
+                dl = near.leaf[at + lane];
+                const int f = dl >> 4, k = dl & 15;
+                float4 *dst = stage + 2 * LEAFMAX * lane;
+                for (int i = 0; i < k; i++) {
+                    dst[2 * i] = rec[2 * (size_t)(f + i)];
+                    dst[2 * i + 1] = rec[2 * (size_t)(f + i) + 1];
+                }
+            }
+            wave_lds_fence();   // lanes read other lanes' slots
+            for (int e = 0; e < nb; e++) {
+                const int d = __builtin_amdgcn_readlane(dl, e);
+                const unsigned long long m = near.mask[at + e];
+                leaf_pairs_staged(stage + 2 * LEAFMAX * e, d >> 4, d & 15,
+                                  valid && ((m >> lane) & 1ull));
+            }
+            wave_lds_fence();   // every read before the next batch's writes
+        }
+    };
+    auto walked_pairs = [&](int share) {
+        // the list was not stored: the same wave-uniform walk again, pairs of
+        // the share's batches only
+        int e = 0;
+        const int2 rr = valid ? root_range[cid[p]] : make_int2(nc, nc);
+        int c = uniform(wave_min_int(valid ? rr.x : nc));
+        const int cend = uniform(wave_max_int(valid ? rr.y : 0));
+        const unsigned long long vmask = ballot(valid);
+        while (c < cend) {
+            const GNodeF nd = gn[c];
+            double d0, d1, d2;
+            if (group_accepts<MACT>(nd, vmask, rpx, rpy, rpz, afactor, d0, d1, d2)) {
+                c = nd.next;
+            } else if (nd.leaf > 0) {
+                if ((ordered ? 0 : e / PL_STAGE % PM_WAVES) == share)
+                    leaf_pairs(nd.first, nd.leaf, valid);
+                e++;
+                c = nd.next;
+            } else {
+                c = c + 1;
+            }
+        }
+    };
     if (ordered && len != NEAR_DROPPED) {
         // PM_LEAVES leaves per wave and round; their sums go to the four waves
         // that add them in list order, one component each (px).  The sums fill
         // the waves' LDS; the leaves are staged where the last one's sums go
         float4 *last = stage + (PM_LEAVES - 1) * WAVE;
-        for (int r = 0; r < len; r += PM_WAVES * PM_LEAVES) {
+        for (int r = 0; r < len; r += NW * PM_LEAVES) {
             const int e0 = r + wave * PM_LEAVES, nb = max(0, min(PM_LEAVES, len - e0));
             int dl = 0;
             if (lane < nb) {
@@ -1775,81 +1828,44 @@ __device__ __forceinline__ void pairs_group_mixed(
             }
             __syncthreads();
             if (wave < 4)
-                for (int e = 0; e < min(PM_WAVES * PM_LEAVES, len - r); e++)
+                for (int e = 0; e < min(NW * PM_LEAVES, len - r); e++)
                     px.add(xsum[(e * 4 + wave) * WAVE + lane]);
             __syncthreads();
         }
-    } else if (len != NEAR_DROPPED) {
-        // the near list in batches of PL_STAGE leaves: lane l copies the
-        // records of the batch's leaf l into the wave's LDS stage (all the
-        // batch's loads in flight at once), then the wave forms the pairs
-        // leaf by leaf in list order from LDS
-        for (int e0 = wave * PL_STAGE; e0 < len; e0 += PM_WAVES * PL_STAGE) {
-            const int nb = min(PL_STAGE, len - e0);
-            const size_t at = near.slot(g, e0);   // a batch lies in one page
-            int dl = 0;
-            if (lane < nb) {
-                dl = near.leaf[at + lane];
-                const int f = dl >> 4, k = dl & 15;
-                float4 *dst = stage + 2 * LEAFMAX * lane;
-                for (int i = 0; i < k; i++) {
-                    dst[2 * i] = rec[2 * (size_t)(f + i)];
-                    dst[2 * i + 1] = rec[2 * (size_t)(f + i) + 1];
-                }
-            }
-            // the wave's LDS writes before its reads (lanes read other
-            // lanes' slots)
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            for (int e = 0; e < nb; e++) {
-                const int d = __builtin_amdgcn_readlane(dl, e);
-                const unsigned long long m = near.mask[at + e];
-                leaf_pairs_staged(stage + 2 * LEAFMAX * e, d >> 4, d & 15,
-                                  valid && ((m >> lane) & 1ull));
-            }
-            // every read of this batch before the next batch's writes
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
     } else {
-        // the list was not stored: the same wave-uniform walk again, pairs of
-        // the wave's batches only
-        int e = 0;
-        const int2 rr = valid ? root_range[cid[p]] : make_int2(nc, nc);
-        int c = uniform(wave_min_int(valid ? rr.x : nc));
-        const int cend = uniform(wave_max_int(valid ? rr.y : 0));
-        const unsigned long long vmask = ballot(valid);
-        while (c < cend) {
-            const GNodeF nd = gn[c];
-            double d0, d1, d2;
-            if (group_accepts<MACT>(nd, vmask, rpx, rpy, rpz, afactor, d0, d1, d2)) {
-                c = nd.next;
-            } else if (nd.leaf > 0) {
-                if ((ordered ? 0 : e / PL_STAGE % PM_WAVES) == wave)
-                    leaf_pairs(nd.first, nd.leaf, valid);
-                e++;
-                c = nd.next;
-            } else {
-                c = c + 1;
+        // the wave's shares of the list: the batches of PL_STAGE leaves go to
+        // PM_WAVES shares in turn
+        for (int share = wave; share < PM_WAVES; share += NW) {
+            if (share != wave) {
+                held[0] = px.value();
+                held[1] = py.value();
+                held[2] = pz.value();
+                held[3] = pq.value();
+                px = py = pz = pq = CSum{};
             }
+            if (len != NEAR_DROPPED)
+                stored_pairs(share);
+            else
+                walked_pairs(share);
         }
     }
     // every wave is done with its stage and with the previous |a|
     __syncthreads();
-    sums[(wave * 4 + 0) * WAVE + lane] = px.value();
-    sums[(wave * 4 + 1) * WAVE + lane] = py.value();
-    sums[(wave * 4 + 2) * WAVE + lane] = pz.value();
-    sums[(wave * 4 + 3) * WAVE + lane] = pq.value();
+    const int at = wave + PM_WAVES - NW;   // the last share (ordered: the wave's sum)
+    sums[(at * 4 + 0) * WAVE + lane] = px.value();
+    sums[(at * 4 + 1) * WAVE + lane] = py.value();
+    sums[(at * 4 + 2) * WAVE + lane] = pz.value();
+    sums[(at * 4 + 3) * WAVE + lane] = pq.value();
+    if (SHARES > 1)
+        for (int k = 0; k < 4; k++) sums[(wave * 4 + k) * WAVE + lane] = held[k];
     __syncthreads();
     if (wave == 0 && valid) {
         double gx = ax[p], gy = ay[p], gz = az[p], gp = cpot[p];
         if (ordered && len != NEAR_DROPPED) {   // component w is wave w's px
-            gx += sums[(0 * 4 + 0) * WAVE + lane];
-            gy += sums[(1 * 4 + 0) * WAVE + lane];
-            gz += sums[(2 * 4 + 0) * WAVE + lane];
-            gp += sums[(3 * 4 + 0) * WAVE + lane];
+            gx += sums[((at + 0) * 4 + 0) * WAVE + lane];
+            gy += sums[((at + 1) * 4 + 0) * WAVE + lane];
+            gz += sums[((at + 2) * 4 + 0) * WAVE + lane];
+            gp += sums[((at + 3) * 4 + 0) * WAVE + lane];
         } else for (int w = 0; w < (ordered ? 1 : PM_WAVES); w++) {
             gx += sums[(w * 4 + 0) * WAVE + lane];
             gy += sums[(w * 4 + 1) * WAVE + lane];
@@ -1867,8 +1883,8 @@ __device__ __forceinline__ void pairs_group_mixed(
     nin_j_out += nin_j;
 }
 
-template <int MACT, bool QUINTIC>
-__global__ void __launch_bounds__(PM_TB) k_grav_pairs_mixed(
+template <int MACT, bool QUINTIC, int NW>
+__global__ void __launch_bounds__(NW * WAVE) k_grav_pairs_mixed(
     int nc, const GNodeF *__restrict__ gn, const float4 *__restrict__ rec,
     const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
     const double *__restrict__ h, const double *__restrict__ zeta,
@@ -1884,9 +1900,9 @@ __global__ void __launch_bounds__(PM_TB) k_grav_pairs_mixed(
     // each wave's LDS stage: PL_STAGE leaves of LEAFMAX two-float4 records;
     // in its place the leaves' sums where they are added in list order, and the
     // waves' sums at the end
-    __shared__ float4 stage_all[PM_WAVES * PL_STAGE * LEAFMAX * 2];
-    static_assert(sizeof(stage_all) >= sizeof(double) * 4 * PM_TB, "sums fit");
-    static_assert(sizeof(stage_all) == sizeof(float) * PM_WAVES * PM_LEAVES * 4 * WAVE &&
+    __shared__ float4 stage_all[NW * PL_STAGE * LEAFMAX * 2];
+    static_assert(sizeof(stage_all) >= sizeof(double) * 4 * PM_WAVES * WAVE, "sums fit");
+    static_assert(sizeof(stage_all) == sizeof(float) * NW * PM_LEAVES * 4 * WAVE &&
                       PM_LEAVES * LEAFMAX * 2 <= WAVE, "leaves' sums fit, their stage in one's");
     __shared__ int job;
     const int wave = uniform((int)(threadIdx.x / WAVE));
@@ -1903,7 +1919,7 @@ __global__ void __launch_bounds__(PM_TB) k_grav_pairs_mixed(
         __syncthreads();
         const int g = uniform(job);
         if (g < 0) break;
-        pairs_group_mixed<MACT, QUINTIC>(
+        pairs_group_mixed<MACT, QUINTIC, NW>(
             g, wave, nc, gn, rec, stage, reinterpret_cast<double *>(stage_all),
             reinterpret_cast<float *>(stage_all), cloud_off, x, y, z, h, zeta, cid, root_range,
             active, t4, ax, ay, az, cpot, gpot, agm, near, grp, npp, nin_p, nin_j);
@@ -2086,19 +2102,40 @@ void launch_cells(Ctx &c, hipStream_t s, int cap) {
     }
 }
 
+// Whether the mixed pair phase takes blocks of half its waves (each wave two of
+// the eight shares of a list, so the sums are the same).  The knob counts blocks
+// of four waves; of blocks of eight two fit a CU, so 3 is the odd number above
+// one that they round up.  At 3 the pair phase of a 1M r^-2 step at the tuned
+// tolerance kept 16 waves a CU where 12 were asked for, and the neighbour rows
+// beside it, on the way to the hydro forces, took 3.6 instead of 2.9 ms (step
+// 15.4 -> 14.8 ms).  In smaller clouds the longest lists bound the phase, and
+// four waves take longer over them (uniform 131,071: 4.8 against 4.1 ms), so
+// only clouds whose walks single waves begin are halved.
+bool pairs_halved(const Ctx &c, int cap) {
+    int least, most;
+    cloud_sizes(c, least, most);
+    return c.walk_queue != 0 && cap == 3 && most > LW_ALONE;
+}
+
 // phase 2 (pair terms), persistent over the same queue order (its second
 // set of counters), on stream s with at most cap blocks per CU
 template <int MACT, bool QUINTIC>
 void launch_pairs(Ctx &c, const double4 *rec, hipStream_t s, int cap) {
     GroupQueue q{c.gq.ctr + NXCD, c.gq.order, c.gq.ngroups};
     if (c.opt.precision == SERENX_MIXED) {
-        auto k = k_grav_pairs_mixed<MACT, QUINTIC>;
-        hipLaunchKernelGGL(k, dim3(walk_blocks(c, k, cap, PM_TB)), dim3(PM_TB), 0, s, c.nc, c.gnf,
-                           reinterpret_cast<const float4 *>(rec), c.x, c.y, c.z, c.h,
-                           c.zeta, c.cid, c.root_range, c.active,
-                           reinterpret_cast<const float4 *>(c.ktab + KT_G4F_OFF), c.gax, c.gay,
-                           c.gaz, c.gpc, c.gpot, c.agm, near_list(c), c.icount, c.grp,
-                           c.cloud_off, q);
+        auto launch = [&](auto k, int tb) {
+            hipLaunchKernelGGL(k, dim3(walk_blocks(c, k, cap, tb)), dim3(tb), 0, s, c.nc, c.gnf,
+                               reinterpret_cast<const float4 *>(rec), c.x, c.y, c.z, c.h, c.zeta,
+                               c.cid, c.root_range, c.active,
+                               reinterpret_cast<const float4 *>(c.ktab + KT_G4F_OFF), c.gax, c.gay,
+                               c.gaz, c.gpc, c.gpot, c.agm, near_list(c), c.icount, c.grp,
+                               c.cloud_off, q);
+        };
+        constexpr int NW = PM_WAVES, HALF = PM_WAVES / 2;
+        if (pairs_halved(c, cap))
+            launch(k_grav_pairs_mixed<MACT, QUINTIC, HALF>, HALF * WAVE);
+        else
+            launch(k_grav_pairs_mixed<MACT, QUINTIC, NW>, NW * WAVE);
     } else {
         int least, most;
         cloud_sizes(c, least, most);
