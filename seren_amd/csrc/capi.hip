@@ -642,15 +642,15 @@ __global__ void k_unpack_in(int n, int m, const double *__restrict__ rec, Unpack
         if (a.dst[k]) a.dst[k][i] = rec[(size_t)m * i + k];
 }
 
-// Neighbour rows as the caller has them: 1-based, zero past the end and in
-// rows above pp_limit
-__global__ void k_rows_out(size_t m, int pp_limit, size_t row0, const int *__restrict__ pptot,
+// m entries from entry at0 on of the neighbour rows, as the caller has them:
+// 1-based, zero past a row's end and in rows above pp_limit
+__global__ void k_rows_out(size_t m, int pp_limit, size_t at0, const int *__restrict__ pptot,
                            const int *__restrict__ pplist, int *__restrict__ out) {
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= m) return;
-    const size_t p = row0 + t / pp_limit;
-    const int i = (int)(t % pp_limit), k = pptot[p];
-    out[t] = k <= pp_limit && i < k ? pplist[p * pp_limit + i] + 1 : 0;
+    const size_t at = at0 + t, p = at / pp_limit;
+    const int i = (int)(at % pp_limit), k = pptot[p];
+    out[t] = k <= pp_limit && i < k ? pplist[at] + 1 : 0;
 }
 
 // records of the host (m doubles a particle) to the device arrays; the
@@ -1374,16 +1374,14 @@ int serenx_fetch(serenx_ctx *ctx, int32_t *porig, double *pos, double *vel, doub
     SX_TRY(out.flush());
     if (pplist) {
         // through the near lists' masks, which a walk writes before it reads
-        const size_t lim = (size_t)c.pp_limit, room = near_list_entries(c.cap) * 2;
-        const size_t rows = std::max<size_t>(1, room / lim);
-        if (lim > room) return set_error(SERENX_EINVAL, "neighbour rows too long to fetch");
-        for (size_t r0 = 0; r0 < (size_t)c.n; r0 += rows) {
-            const size_t m = std::min(rows, (size_t)c.n - r0) * lim;
-            int *tmp = reinterpret_cast<int *>(c.pl_mask);
+        const size_t all = (size_t)c.n * c.pp_limit, room = near_list_entries(c.cap) * 2;
+        int *tmp = reinterpret_cast<int *>(c.pl_mask);
+        for (size_t at = 0; at < all; at += room) {
+            const size_t m = std::min(room, all - at);
             hipLaunchKernelGGL(k_rows_out, dim3(nblk((long)m)), dim3(TB), 0, c.stream, m,
-                               c.pp_limit, r0, c.pptot, c.pplist, tmp);
+                               c.pp_limit, at, c.pptot, c.pplist, tmp);
             SX_HIP(hipGetLastError());
-            SX_TRY(down_parts(c, {{pplist + r0 * lim, tmp, sizeof(int) * m}}));
+            SX_TRY(down_parts(c, {{pplist + at, tmp, sizeof(int) * m}}));
         }
     }
     return SERENX_OK;
