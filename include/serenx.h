@@ -297,38 +297,42 @@ int serenx_serve_info(serenx_ctx *ctx, int32_t ncloud, double *dt, double *time)
  * how the kernels run, and the autotuner in seren_amd/autotune.py sets them).
  *  SERENX_TUNE_HSOLVE_SLOTS: potential-neighbour leaves recorded per particle
  *    in the grad-h solve and h_gather lists, 1..96 (default 96).  A particle
- *    whose list does not fit is summed over the tree walk at the same radius
- *    (the same leaves in the same order): results do not change, only speed;
- *    tests lower it to drive that path.
+ *    whose list does not fit is searched for by a whole wave in the grad-h
+ *    solve, and summed over the tree walk in h_gather (the same leaves in the
+ *    same order): results do not change, only speed; tests lower it to drive
+ *    those paths.
  *  SERENX_TUNE_MIXED_ABSERROR: multipole-MAC tolerance of the mixed-precision
  *    gravity walk (GADGET, GADGET2, EIGEN MACs; 0 = the options' abserror).
  *    The FP64 walk always uses abserror (the reference's interaction sets);
  *    the mixed walk may trade part of its accuracy margin for speed.  Takes
  *    effect at the next tree stock.
- *  SERENX_TUNE_WALK_QUEUE: v >= 1 runs the gravity walk as a persistent
- *    kernel of at most v blocks per CU (default 64: as many as fit) whose
- *    waves take groups of 64 particles from per-XCD work queues, each ordered
- *    by the cost of the group's previous walk (longest first).  Fewer blocks
+ *  SERENX_TUNE_WALK_QUEUE: the gravity walk's kernels are persistent; their
+ *    blocks take groups of 64 particles from per-XCD work queues, ordered by
+ *    the cost of the group's previous walk (longest first).  v >= 1 keeps at
+ *    most v blocks of four waves per CU of each (default 64: as many as fit;
+ *    kernels with blocks of 8 or 16 waves round up to whole blocks).  Fewer
  *    leave wave slots to the SPH kernels that run beside the walk in force
  *    evaluations and steps; the best value depends on the workload (the
  *    autotuner in seren_amd/autotune.py times a few).  A walk with nothing
- *    beside it (serenx_grav_forces) takes all that fit.  0 launches one wave
- *    per group in tree order.  Results do not change.
+ *    beside it (serenx_grav_forces) takes all that fit.  0: as many as fit,
+ *    the groups in tree order.  Results do not change.
  *  SERENX_TUNE_NEIB_GROUP: 1 (default) builds the neighbour lists with searches
- *    by whole waves, eight particles each; 0 with the particles' own walks
- *    (BHhydro_walk.F90's test per particle).
- *    The lists are the same.
+ *    by whole waves, of eight particles each (above 262,144 particles on a tree
+ *    stocked at their positions one walk per wave of 64); 0 with the particles'
+ *    own walks (BHhydro_walk.F90's test per particle).  The lists are the same.
  *  SERENX_TUNE_HSOLVE_WAVES: waves per SIMD of the grad-h iteration kernel:
  *    8 (registers capped at 64, a few spills), 0 (the compiler's budget,
  *    5 waves), -1 (default: 8 in mixed precision, where the SPH kernels are
  *    the critical path, 0 in FP64, where the h solve runs beside the
  *    issue-bound FP64 walk).  Results do not change.
  *  SERENX_TUNE_NEAR_CAP: near-field leaves the gravity walk's cell phase
- *    records per group of 64 particles for the pair phase, 1..4096 (default
- *    4096).  A group whose list does not fit walks the tree again in the
- *    pair phase with the same MAC decisions (the same leaves in the same
- *    order): results do not change, only speed; tests lower it to drive
- *    that path.
+ *    records per group of 64 particles for the pair phase: 1..4095, or 4096
+ *    (default) for as many as the context's pool holds, which the groups share
+ *    (4,096 leaves a group on average, 32,768 at most for one).  A group whose
+ *    list does not fit, or that finds the pool empty, walks the tree again in
+ *    the pair phase with the same MAC decisions (the same leaves in the same
+ *    order): results do not change, only speed; tests lower it to drive that
+ *    path.
  *  SERENX_TUNE_NEIB_LEAVES: 0..512 (default 512).  Kept for programs that set
  *    it: rows above pp_limit are searched by whole waves, which keep no list
  *    of leaves, so the value has no effect.
