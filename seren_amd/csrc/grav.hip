@@ -2,11 +2,12 @@
 // terms and the grad-h kernel-softened near field, plus the FP64
 // kernel-softened direct sum, on gfx950.
 //
-// A wave walks the gravity tree for 64 consecutive (tree-ordered) particles
-// with group_walk.  At each cell every active lane applies its own MAC
-// (BHgrav_accel.F90:154-158): accepted cells add a multipole term, opened
-// leaves add kernel-softened pair terms (gravity_gradh.F90), opened branches
-// descend.  Each lane therefore sees exactly the reference particle's
+// The tree is walked for groups of 64 consecutive (tree-ordered) particles, by a
+// block that opens it level by level (k_grav_list) or, in large clouds, begun by
+// a wave cell by cell (k_grav_cells_*).  In FP64 every particle applies its own
+// MAC (BHgrav_accel.F90:154-158): cells it accepts add a multipole term, leaves
+// it opens add kernel-softened pair terms (gravity_gradh.F90), branches it opens
+// descend.  Each particle therefore sees exactly the reference particle's
 // interaction set; MAC tests use the reference's arithmetic (no contraction)
 // so that accept/open decisions are identical.  The reference sums all cell
 // terms first and the near-field pairs at the end (BHgrav_accel.F90:272-290);

@@ -81,13 +81,20 @@ constexpr int LW_BITS = 131072;
 // clouds of more particles are walked by one wave per group, which leaves a
 // walk to the list walk after LW_BUDGET visits (grav.hip has the reasons)
 constexpr int LW_ALONE = 393216;
-// clouds of at most this many particles have their terms added in walk order
-// (grav.hip; twice the time of a walk there, and nothing to gain by it where a
-// cloud is not followed through a collapse)
+// Clouds of at most this many particles have their terms added in walk order.
+// A choice for compatibility, not for speed: their results are those of a walk
+// by one wave bit for bit, by which runs of small collapsing cores (where a last
+// bit grows to 1e-8 in 60 steps) can be compared; results of larger clouds
+// differ from such a walk's by rounding.  There is no size at which the order
+// is free (evaluations, ordered / in wave order, ms: FP64 uniform 1.37 / 0.85
+// and r^-2 1.35 / 1.18 at 4,096, 1.80 / 1.20 and 1.79 / 1.44 at 8,192, 3.23 /
+// 1.78 and 2.29 / 1.81 at 16,384; mixed uniform 0.84 / 0.73 and r^-2 1.19 / 1.15
+// at 4,096, 1.16 / 1.00 and 1.45 / 1.40 at 8,192); the line keeps its price
+// near half a millisecond.
 constexpr int LW_ORDERED = 6144;
 constexpr int LW_BUDGET = 8192;
 constexpr int LW_CAP = 8192;
-// largest value of SERENX_TUNE_NEIB_LEAVES
+// largest value of SERENX_TUNE_NEIB_LEAVES, which has no effect
 constexpr int NB_CAP = 512;
 
 // Counters that every wave of a launch updates (walk statistics, interaction

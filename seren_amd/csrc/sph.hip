@@ -394,7 +394,7 @@ __global__ void __launch_bounds__(256) k_hsolve_final(
 // nodes of a search front, and leaves of a list, held in LDS.  512 entries
 // hold a front of the largest chain of a resumed search (7 siblings on each
 // of LMAX levels) and the lists of all but a few particles; 8 KB per wave
-// leave 20 waves on a CU.
+// leave room for 20 waves on a CU.
 constexpr int WS_CAP = 512;
 static_assert(WS_CAP >= 8 * (LMAX + 1), "a resumed search's first front must fit");
 
@@ -580,15 +580,22 @@ __device__ __forceinline__ void wave_candidates(const WaveSearch &L, int nleaf,
 // in most of the cloud.
 //
 // Bound by the latency of the front's node loads and of the serial sums
-// (about a microsecond each per pass), hidden by the 20 waves on a CU.
+// (about a microsecond each per pass), hidden by the 12 waves on a CU.
 // Measured (steady evaluation, beside the gravity walk): 60 us at 2,048
 // particles, 232 us at 16,384 and 4.4 ms at 131,072, against 680, 980 and
 // 3,560 us of the lane kernels, which keep 64 particles' worth of work per
-// wave: clouds up to HSOLVE_WAVE_MAX particles take this kernel, larger ones
-// the lane kernels (first evaluation of a 2,053-particle Plummer sphere,
-// whose outskirts go through the bisection: 21 -> 3.2 ms).  Held to 4 or 5
-// waves per SIMD instead of the compiler's 153 registers it was slower (242
-// and 289 us at 16,384).
+// wave (first evaluation of a 2,053-particle Plummer sphere, whose outskirts
+// go through the bisection: 21 -> 3.2 ms).  Contexts of up to HSOLVE_WAVE_MAX
+// particles take this kernel, larger ones the lane kernels.  The profiles
+// cross at different sizes, and the line lies between them.  Steady
+// evaluations, waves / lanes (ms), FP64: uniform 2.6 / 2.7 at 32,768, 3.3 / 3.0
+// at 49,152, 3.8 / 3.2 at 65,536, 5.5 / 4.3 at 98,304; r^-2 2.2 / 3.8, 3.4 /
+// 3.8, 4.0 / 4.4, 5.2 / 5.7 (6.6 / 6.4 at 131,071); Plummer 2.6 / 2.9, 3.4 /
+// 3.2, 4.1 / 3.8, 5.8 / 4.7.  Mixed: uniform 2.1 / 2.5, 2.5 / 2.5, 2.8 / 2.4,
+// 4.0 / 3.2; r^-2 2.0 / 3.5, 3.0 / 3.4, 3.6 / 3.9, 4.5 / 5.1; Plummer 2.2 /
+// 2.6, 2.7 / 2.8, 3.1 / 3.2, 4.3 / 3.6.  Held to 4 or 5 waves per SIMD instead
+// of the compiler's 149 registers (three) it was slower (242 and 289 us at
+// 16,384).
 constexpr int HSOLVE_WAVE_MAX = 1 << 16;
 
 __global__ void __launch_bounds__(256) k_hsolve_wave(
