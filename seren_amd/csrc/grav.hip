@@ -1020,9 +1020,21 @@ __device__ __forceinline__ void lw_targets(ListWalk<NW> &L, const ListScratch &s
 }
 
 // (four waves per SIMD: two blocks of a CU hide each other's barriers)
-template <bool MIXED, bool ORDERED, int OCT, int MACT>
+//
+// LEAN: registers for 6 (FP64) or 8 (mixed) waves per SIMD, where LDS admits
+// four, and no raised priority.  The others are the h solve's: with 114 to 128
+// registers the walk's two blocks filled a CU's register files, and where there
+// are groups for every CU the h solve had to wait until the walk was done.  Some
+// values are spilled (56 in FP64, 53 mixed).  Forests of 4,096 to 262,144
+// particles a cloud, an evaluation: mixed 14.4M particles 194 -> 171 ms (walk
+// and h solve beside each other 134 -> 107), FP64 6.1M 235 -> 219; one cloud,
+// mixed uniform 131,071 4.1 -> 3.6, r^-2 390,000 10.4 -> 8.9, FP64 Plummer
+// 200,000 10.5 -> 8.0, r^-2 16,384 1.80 -> 1.78.  FP64 walks of fewer groups than
+// CUs, which leave the h solve room anyway, keep their registers (uniform 8,192:
+// 1.19, 1.22 lean); mixed ones gain there too (1.03 -> 0.98).
+template <bool MIXED, bool ORDERED, bool LEAN, int OCT, int MACT>
 __global__ void __launch_bounds__(ORDERED ? OW_TB : LW_TB)
-__attribute__((amdgpu_waves_per_eu(4))) k_grav_list(
+__attribute__((amdgpu_waves_per_eu(!LEAN ? 4 : MIXED ? 8 : 6))) k_grav_list(
     int nc, const GMac *__restrict__ gmac, double macscale, const GNode *__restrict__ gn,
     const GNodeF *__restrict__ gnf, const double *__restrict__ x,
     const double *__restrict__ y, const double *__restrict__ z, const int *__restrict__ cid,
@@ -1033,12 +1045,15 @@ __attribute__((amdgpu_waves_per_eu(4))) k_grav_list(
     unsigned long long *__restrict__ wstat, GroupQueue queue, int *__restrict__ cost,
     const int2 *__restrict__ grp, const int *__restrict__ cloud_off, LongWalks lw) {
     constexpr int NW = ORDERED ? OW_WAVES : LW_WAVES, NT = NW * WAVE;
-    __shared__ ListWalk<NW> L;
+    // (given at the launch: the compiler would keep the registers of no more waves
+    // than its LDS admits)
+    extern __shared__ double list_walk_lds[];
+    ListWalk<NW> &L = *reinterpret_cast<ListWalk<NW> *>(list_walk_lds);
     // a round's factors [wave][dx, Q, H, ir5, ir7, crad, phi][lane]
     __shared__ double xc[ORDERED ? NW : 1][13][ORDERED ? WAVE : 1];
-    // the walk is the critical path while the SPH kernels run beside it: its
-    // waves take issue priority over theirs on shared SIMDs
-    __builtin_amdgcn_s_setprio(2);
+    // a walk of few groups is the critical path while the SPH kernels run beside
+    // it: its waves take issue priority over theirs on shared SIMDs
+    if (!LEAN) __builtin_amdgcn_s_setprio(2);
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = uniform(tid / WAVE);
     ListScratch sc = all;
     sc.ids += (size_t)blockIdx.x * all.cap;
@@ -2032,9 +2047,9 @@ int pair_cap(const Ctx &c) {
 // of a mixed 1M step keeps 16 waves a CU: 14.8 ms, 16.1 with the 8 of rounding
 // down, each one run).
 template <class K>
-int walk_blocks(Ctx &c, K kernel, int cap, int tb, int groups = 1) {
+int walk_blocks(Ctx &c, K kernel, int cap, int tb, int groups = 1, size_t lds = 0) {
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, tb, 0) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, tb, lds) != hipSuccess ||
         per_cu <= 0)
         per_cu = 1;
     if (c.walk_queue != 0) per_cu = std::min(per_cu, (cap * TB + tb - 1) / tb);
@@ -2083,22 +2098,27 @@ void launch_cells(Ctx &c, hipStream_t s, int cap) {
     }
     const ListScratch sc{c.lw_ids, c.lw_in, c.lw_open, c.lw_list, c.lw_mask, c.lw_cap};
     auto launch = [&](auto k, int tb, const GroupQueue &gq, const LongWalks &walks) {
-        const int nb = std::min(walk_blocks(c, k, cap, tb), c.lw_blocks);
-        hipLaunchKernelGGL(k, dim3(nb), dim3(tb), 0, s, c.nc, c.gmac,
+        const size_t lds =
+            tb == OW_TB ? sizeof(ListWalk<OW_WAVES>) : sizeof(ListWalk<LW_WAVES>);
+        const int nb = std::min(walk_blocks(c, k, cap, tb, 1, lds), c.lw_blocks);
+        hipLaunchKernelGGL(k, dim3(nb), dim3(tb), lds, s, c.nc, c.gmac,
                            mixed ? mixed_mac_scale(c) : 1.0, c.gn, c.gnf, c.x, c.y, c.z, c.cid,
                            c.root_range, c.active, c.gpot, c.agm, c.gax, c.gay, c.gaz, c.gpc,
                            near_list(c), sc, c.icount, c.wstat, gq, c.gq.cost, c.grp,
                            c.cloud_off, walks);
     };
     if (mixed) {
-        launch(k_grav_list<true, false, OCT, MACT>, LW_TB, q, lw);
+        launch(k_grav_list<true, false, true, OCT, MACT>, LW_TB, q, lw);
         return;
     }
-    if (most > LW_ORDERED) launch(k_grav_list<false, false, OCT, MACT>, LW_TB, q, lw);
+    if (most > LW_ORDERED && q.ngroups >= c.ncu)
+        launch(k_grav_list<false, false, true, OCT, MACT>, LW_TB, q, lw);
+    else if (most > LW_ORDERED)
+        launch(k_grav_list<false, false, false, OCT, MACT>, LW_TB, q, lw);
     if (least <= LW_ORDERED) {
         LongWalks lo = lw;
         lo.taken = cont + 2;
-        launch(k_grav_list<false, true, OCT, MACT>, OW_TB, GroupQueue{cont + 3, q.order, q.ngroups},
+        launch(k_grav_list<false, true, false, OCT, MACT>, OW_TB, GroupQueue{cont + 3, q.order, q.ngroups},
                lo);
     }
 }
