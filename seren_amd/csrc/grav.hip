@@ -778,9 +778,9 @@ __device__ __forceinline__ bool group_accepts(const GNodeF &nd, unsigned long lo
 // vote and term one after the other), so a launch took as long as its largest
 // walk: 16.6 ms on a uniform sphere of 131,071 particles whose central groups,
 // where |a| -> 0, visit 15,000 cells.  Here 64 tests run at once and the cells
-// to come are known before their terms are formed: 3.8 ms there; 300 -> 62 us
-// on 2,048 particles (FP64, quadrupole), 1,454 -> 385 us on an r^-2 sphere of
-// 16,384 and 5.3 -> 1.1 ms on a uniform one of 65,536 (mixed).  Bound by the
+// to come are known before their terms are formed: 3.5 ms there; 300 -> 62 us
+// on 2,048 particles (FP64, quadrupole), 1,454 -> 332 us on an r^-2 sphere of
+// 16,384 and 5.3 -> 0.7 ms on a uniform one of 65,536 (mixed).  Bound by the
 // vector ALU: on the 1M r^-2 sphere 89 instructions per accepted cell and
 // wave, and 1.1e9 of 8.1e9 in steps 1 and 2 (2.2e9 with every cell tested
 // against every target, without the sphere).
@@ -1440,13 +1440,16 @@ __attribute__((amdgpu_waves_per_eu(!LEAN ? 4 : MIXED ? 8 : 6))) k_grav_list(
 // In a cloud of more than LW_ALONE particles a wave walks for its group alone,
 // up to LW_BUDGET visits; the list walk takes what is left, from the cell where
 // the wave stopped.  With that many groups the waves hide each other's
-// latency, and the walk by one wave issues slightly fewer instructions and
-// leaves the SPH kernels beside it more room: an evaluation of r^-2 spheres
-// takes (waves / list walk, ms) 22.8 / 28.3 at 1M, 12.7 / 13.8 at 524k, 9.7 /
-// 10.9 at 400k (mixed), 10.6 / 11.5 at 300k and 8.4 / 8.6 at 200k (FP64).  Where
-// a few groups walk far, the list walk wins up to 400k and beyond: uniform
-// 18.1 / 14.8 at 524k, 14.8 / 11.2 at 400k (mixed), Plummer 18.7 / 12.7 at 300k
-// (FP64).  The line lies where the two gains balance; the budget keeps the
+// latency, and the walk by one wave issues slightly fewer instructions: an
+// evaluation of an r^-2 sphere of 1M takes (waves / list walk, ms) 22.0 / 22.8
+// mixed, 31.6 / 32.9 in FP64.  Elsewhere the list walk, with the registers it
+// has now, is ahead: r^-2 12.4 / 11.5 at 524k, 10.0 / 9.3 at 400k (mixed), 17.4 /
+// 17.0 and 13.9 / 13.3 (FP64); uniform 28.9 / 26.6 at 1M, 17.8 / 12.7 at 524k, 13.3
+// / 10.4 at 400k (mixed); Plummer 39.4 / 37.1, 25.8 / 18.8, 20.1 / 15.0 (FP64).
+// The line was drawn where the gains balanced when two blocks of the list walk
+// filled a CU's registers (r^-2 12.7 / 13.8 at 524k, 9.7 / 10.9 at 400k, uniform
+// 14.8 / 11.2 at 400k), and stays below the 1M steps that the knobs are tuned
+// for, which have been measured by waves only.  The budget keeps the
 // long walks of a large uniform cloud from their waves (1M: 75 -> 30 ms;
 // budgets of 3,000, 8,192 and 16,384 differ by 2 % there, and 3,000 costs the
 // r^-2 sphere 10 %).
