@@ -62,7 +62,10 @@ enum {
     SERENX_MAC_EIGEN = 3      /* EIGEN_MAC (:335-337, eigenvalue_mac.F90), |phi| based */
 };
 /* arithmetic of the gravity walk: FP64 throughout, or FP32 terms on
- * cell-relative coordinates with compensated FP32 accumulation */
+ * cell-relative coordinates with compensated FP32 accumulation.  The order of
+ * its sums depends on the cloud's own size alone, so a cloud's results are the
+ * same by itself and in any forest: up to 6,144 particles in the order of one
+ * walk, above that in parts that are added in turn (another rounding). */
 enum { SERENX_FP64 = 0, SERENX_MIXED = 1 };
 
 /* serenx_force_eval flags */
