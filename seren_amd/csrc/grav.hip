@@ -2177,11 +2177,30 @@ void launch_pairs(Ctx &c, const double4 *rec, hipStream_t s, int cap) {
     }
 }
 
+// Whether a launch takes its groups in tree order: forests with many groups for
+// every block of the device have no long last walk to fear, and groups that are
+// neighbours share the cells in L2.  The forests' evaluations with a build,
+// longest first / in tree order (ms): FP64 33.6 / 34.2 at 19,000 groups, 50.8 /
+// 48.6 at 28,000, 98 / 91 at 43,000, 153 / 137 at 67,000, 535 / 461 at 224,000
+// (519 when single waves took the walks longest first); mixed 10.4 / 11.7 at 9,000,
+// 22.5 / 22.0 at 19,000, 55.4 / 52.4 at 67,000, 186 / 168 at 224,000.  A cloud
+// that single waves walk keeps longest first (uniform 2M FP64 82.7 / 88.3, r^-2
+// 64.1 / 63.4).
+bool tree_order(const Ctx &c) {
+    int least, most;
+    cloud_sizes(c, least, most);
+    return c.gq.ngroups >= 100 * c.ncu && most <= LW_ALONE;
+}
+
 // sorts the queue order from the costs of the last walk, on the gravity
 // stream
 int sort_queue(Ctx &c) {
     Ctx::WalkQueue &q = c.gq;
     const int ng = q.ngroups;
+    if (tree_order(c)) {
+        hipLaunchKernelGGL(k_queue_identity, dim3(nblk(ng)), dim3(TB), 0, c.gstream, ng, q.order);
+        return SERENX_OK;
+    }
     hipLaunchKernelGGL(k_queue_keys, dim3(nblk(ng)), dim3(TB), 0, c.gstream, ng, q.cost,
                        (int)(q.have_cost && c.walk_queue != 0), q.keys, q.vals);
     size_t tb = q.tmp_bytes;
