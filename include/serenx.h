@@ -311,7 +311,8 @@ int serenx_serve_info(serenx_ctx *ctx, int32_t ncloud, double *dt, double *time)
  *    effect at the next tree stock.
  *  SERENX_TUNE_WALK_QUEUE: the gravity walk's kernels are persistent; their
  *    blocks take groups of 64 particles from per-XCD work queues, ordered by
- *    the cost of the group's previous walk (longest first).  v >= 1 keeps at
+ *    the cost of the group's previous walk (longest first; large forests in
+ *    tree order).  v >= 1 keeps at
  *    most v blocks of four waves per CU of each (default 64: as many as fit;
  *    kernels with blocks of 8 or 16 waves round up to whole blocks).  Fewer
  *    leave wave slots to the SPH kernels that run beside the walk in force
